@@ -484,7 +484,7 @@ constexpr int kPlanScratch = kPsMisc + 4;
 template <int NT>
 __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, long long T, int R, int gcap,
                           const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-                          int* __restrict__ rec_start, int* __restrict__ lists, int* ps, int& total_recs,
+                          int* __restrict__ rec_start, int* __restrict__ lists, int* ps, int& total_recs, bool wide,
                           long long t0_first = 0, long long t1_first = -1) {
   constexpr int kW = NT / 64;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -610,7 +610,9 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       // tokens: 16, 4 x 16384: 64, all measured faster than the earlier
       // estimate's 20, 28 and 96).
       constexpr float kWarmItem = 1.5f, kTailShare = 0.25f, kSegmented = 0.75f;
-      constexpr float kMachines = static_cast<float>(kConsumerGroups / 16);
+      // the split consumer takes a run's 16 items on 256 groups, the wide one
+      // its 8 on 256 CUs (two groups of a CU share its throughput)
+      const float kMachines = static_cast<float>(kConsumerGroups / (wide ? 8 : 16));
       const float T = 0.5f * (runs + nl);                      // runs = sum of 2 nseg - 1
       const float work = sl + static_cast<float>(w_est) * (T - nl);
       const float longest = ml > Lc ? static_cast<float>(Lc + w_est) : static_cast<float>(ml);
@@ -620,7 +622,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     } else {
       // M-run scheme: W(L) counts the M-runs of later segments.  The scan
       // adds about half a step per segment and segmenting at all 1.5 steps.
-      const float per_wg = (16.f * (2.f * sl - a) + kItemOverhead * 16.f * runs) / kConsumerGroups;
+      const float per_wg = (2.f * sl - a + kItemOverhead * runs) * (wide ? 8.f : 16.f) / kConsumerGroups;
       const float crit = static_cast<float>(min(Lc, ml)) + kItemOverhead;
       est = fmaxf(crit, per_wg) + (nseg_max > 1 ? 0.5f * static_cast<float>(nseg_max - 1) + 1.5f : 0.f);
     }
@@ -775,7 +777,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     const void* __restrict__ cu, int is64, int num_seqs, long long T, int R, int gcap,
     const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-    int* __restrict__ rec_start, int4* __restrict__ recs, int* __restrict__ lists) {
+    int* __restrict__ rec_start, int4* __restrict__ recs, int* __restrict__ lists, int wide) {
   __shared__ int ps[kPlanScratch];
   const int tid = threadIdx.x;
   const int per = (num_seqs + kPlanThreads - 1) / kPlanThreads;
@@ -783,7 +785,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   const int s_end = min(num_seqs, s_begin + per);
   int total_recs;
   int base = plan_batch<kPlanThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, ps,
-                                      total_recs);
+                                      total_recs, wide != 0);
   for (int s = s_begin; s < s_end; ++s) {
     long long t0, t1;
     seq_bounds(cu, is64, s, T, t0, t1);
@@ -1250,14 +1252,14 @@ __global__ __launch_bounds__(kPrepassThreads, kGroups) void prepass_kernel(
     const float* __restrict__ dt_bias, const uint16_t* __restrict__ b,
     const int4* __restrict__ recs, const void* __restrict__ cu, int is64, int num_seqs, long long T, int R,
     int gcap, int fused_plan, int* __restrict__ rec_start, int* __restrict__ lists,
-    uint16_t* __restrict__ ws_frag, float* __restrict__ ws_gam) {
+    uint16_t* __restrict__ ws_frag, float* __restrict__ ws_gam, int wide) {
   __shared__ PrepassSmem sm;
   if (fused_plan && blockIdx.x == 0) {
     // work-group 0 plans the batch (lists for the consumer) while the others
     // run the records
     int total_recs;
     plan_batch<kPrepassThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, sm.u.plan,
-                                total_recs);
+                                total_recs, wide != 0);
     return;
   }
   const int lane = threadIdx.x & 63;
@@ -2792,6 +2794,710 @@ void consumer_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict_
 }
 
 // ============================================================================
+// wide consumer: one work-group per (run or short sequence, v-head)
+// ============================================================================
+// For batches with work for every CU.  A group of four waves carries a whole
+// head, wave w the value rows 32 w .. 32 w + 31 as two 16-row tiles (row i of
+// tile e is value row 32 w + wide_row(e, i): a lane then holds eight
+// consecutive value columns of an output token over the two tiles), and runs
+// everything a chunk needs (X, Y^T, Aqk tiles, R, Delta, O^T, S') itself: no
+// state or Delta leaves the wave's registers, and every K / Q / Tb / Aqk
+// fragment read from LDS feeds both tiles.  Two groups share a CU (78 KB of
+// LDS, 256 VGPRs per wave, two waves per SIMD) and are independent of each
+// other, so one group's barriers, copies, item starts and state traffic run
+// under the other's products.
+//
+// LDS: K rows and the gate block are double-buffered (K is read to the end of
+// the chunk by the state update); Q, V, Tb and Aqk have one buffer each.  Two
+// barriers per chunk: W1 after Delta (every wave's Aqk tiles are in LDS, and
+// Q, V and Tb are dead: their copies for the next chunk are issued then) and
+// W2 at the end (the next chunk's operands have landed).
+constexpr int kWideThreads = 256;
+constexpr int kWideWaves = kWideThreads / 64;
+constexpr int kWideGroups = 512;           // two per CU
+constexpr int kWideStores = 4;             // output stores of a wave per chunk (one per 16-token block)
+
+__host__ __device__ constexpr int wide_row(int e, int i) { return 8 * (i >> 2) + 4 * e + (i & 3); }
+
+// The lane index through an opaque move: keeps the compiler from computing the
+// lane-dependent addresses of every phase once, outside the chunk and item
+// loops, and spilling them.
+__device__ __forceinline__ int opaque_lane(int lane) {
+  int l;
+  asm volatile("v_and_b32 %0, 63, %1" : "=v"(l) : "v"(lane));
+  return l;
+}
+
+struct __align__(16) WideSmem {
+  uint16_t ks[2][kChunk][kDim];
+  uint16_t qs[kChunk][kDim];
+  uint16_t vs[kChunk][kDim];
+  uint16_t tb[kMatElems];
+  uint16_t aqk[kMatElems];
+  float gt[2][4 * kChunk];
+  int next_item;
+};
+static_assert(2 * sizeof(WideSmem) <= 160 * 1024, "two groups per CU");
+
+// Resources over an item's rows and records, formed once per item: a chunk's
+// copies and stores then differ only in a 32-bit offset.  Row i 64 + t of an
+// item is token t of its chunk i; rows past the item's last token fall outside
+// and arrive as zeros.
+struct WideItem {
+  u32x4 k, q, v, fr, g;
+  __amdgpu_buffer_rsrc_t out;
+};
+constexpr uint32_t kKqRow = kQKHeads * kDim * 2, kVRow = kVHeads * kDim * 2;          // bytes per token
+constexpr uint32_t kFragRec = kVHeads * kMatElems * 2, kGamRec = kVHeads * kGamStride * 4;   // bytes per record
+// an item's rows of V, the widest stream, must fit the 32-bit offsets
+constexpr long long kWideMaxTokens = 1 << 20;
+static_assert((kWideMaxTokens + 2 * kChunk) * kVRow < (1ll << 32), "32-bit offsets");
+
+__device__ __forceinline__ u32x4 rsrc_words(const void* base, uint32_t bytes) {
+  const uint64_t b = reinterpret_cast<uint64_t>(base);
+  return u32x4{static_cast<uint32_t>(b), static_cast<uint32_t>(b >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
+}
+
+// The copies are issued in assembly blocks, which hold no output register:
+// through the builtin the compiler makes every transposed LDS read wait for
+// every copy in flight (it cannot tell their LDS ranges apart), which ends the
+// overlap.  The waits are the barriers' own (W2).  Unknown operations in
+// flight only make the compiler's own vmcnt waits stricter.  The leading nops
+// cover a resource word written by a VALU instruction just before.
+//
+// One 1 KB piece: lane i's 16 bytes at voff go to lds + 16 i.
+__device__ __forceinline__ void wide_dma1(const u32x4& rs, uint32_t voff, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\ts_nop 4\n\t"
+      "buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
+      : "memory", "m0");
+}
+
+// Four pieces: rows voff + j step, j < 4, to lds + 4096 j.
+template <bool kNt>
+__device__ __forceinline__ void wide_dma4(const u32x4& rs, uint32_t voff, uint32_t step, uint32_t lds) {
+  const uint32_t v1 = voff + step, v2 = voff + 2 * step, v3 = voff + 3 * step;
+  if constexpr (kNt)
+    asm volatile(
+        "s_mov_b32 m0, %5\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %4, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen nt lds" ::"v"(voff),
+        "v"(v1), "v"(v2), "v"(v3), "s"(rs), "s"(lds)
+        : "memory", "m0", "scc");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %5\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen lds" ::"v"(voff),
+        "v"(v1), "v"(v2), "v"(v3), "s"(rs), "s"(lds)
+        : "memory", "m0", "scc");
+}
+
+// Copies of chunk i's operands: wave w copies rows 4 w + lane / 16 + 16 j of K,
+// Q and V (1 KB per instruction).
+//
+// K rows and the gate block into buffer P.
+__device__ __forceinline__ void wide_dma_k(WideSmem& sm, int P, const WideItem& it, int i, int lane, int w) {
+  lane = opaque_lane(lane);
+  const int row = 4 * w + (lane >> 4);
+  const uint32_t off = static_cast<uint32_t>(i * kChunk + row) * kKqRow +
+                       16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(row));
+  wide_dma4<false>(it.k, off, 16 * kKqRow, lds_addr(&sm.ks[0][0][0]) + 16384u * P + 1024u * w);
+  if (w == kWideWaves - 1)
+    wide_dma1(it.g, 16u * static_cast<uint32_t>(lane) + i * kGamRec, lds_addr(&sm.gt[0][0]) + 1024u * P);
+}
+
+// Q and V rows and the Tb fragments.
+__device__ __forceinline__ void wide_dma_qvt(WideSmem& sm, const WideItem& it, int i, int lane, int w) {
+  lane = opaque_lane(lane);
+  const int row = 4 * w + (lane >> 4);
+  const uint32_t r = static_cast<uint32_t>(i * kChunk + row);
+  // V first: the only stream the prepass has not touched
+  wide_dma4<true>(it.v, r * kVRow + 16u * static_cast<uint32_t>((lane & 15) ^ v_swz(row)), 16 * kVRow,
+                  lds_addr(&sm.vs[0][0]) + 1024u * w);
+  wide_dma4<false>(it.q, r * kKqRow + 16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(row)), 16 * kKqRow,
+                   lds_addr(&sm.qs[0][0]) + 1024u * w);
+  const uint32_t foff = static_cast<uint32_t>(64 * w + lane) * 16u + i * kFragRec;
+  wide_dma1(it.fr, foff, lds_addr(sm.tb) + 1024u * w);
+  if (w + kWideWaves < kMatFrags) wide_dma1(it.fr, foff + 4096u, lds_addr(sm.tb) + 4096u + 1024u * w);
+}
+
+// A 32 x 128 fp32 state tile (two 16-row tiles of a wave) between memory and
+// the C layout in kappa order.  Memory is accessed 4 rows x 256 contiguous
+// bytes per instruction; the lanes then trade pieces through 4 KB of LDS, 16
+// rows (of one tile) x 64 columns at a time, 16-byte piece p of row r at p ^ r.
+// Reading the C layout straight from memory (16 rows per instruction, adjacent
+// lanes in different rows) costs one cache-line lookup per lane: a copy of
+// 4,096 head states in that pattern ran at 3.6 TB/s (two groups per CU, no
+// compute) against 5.8 TB/s with contiguous rows.
+__device__ __forceinline__ void load_state_rows(const float* __restrict__ src, f32x4 (&r)[16], int lane) {
+  const float* p = src + (lane >> 4) * kDim + 4 * (lane & 15);
+#pragma unroll
+  for (int j = 0; j < 16; ++j)   // j = 8 e + 4 half + i: rows wide_row(e, 4 i ..), columns 64 half
+    r[j] = __builtin_nontemporal_load(
+        reinterpret_cast<const f32x4*>(p + (4 * (j >> 3) + 8 * (j & 3)) * kDim + 64 * ((j >> 2) & 1)));
+}
+
+__device__ __forceinline__ void state_rows_to_tiles(const f32x4 (&r)[16], f32x4 (&st)[2][8], f32x4* sc, int lane) {
+  const int l16 = lane & 15, lg = lane >> 4;
+#pragma unroll
+  for (int th = 0; th < 4; ++th) {   // 2 e + half
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 4 * i + lg;
+      sc[row * 16 + (l16 ^ row)] = r[4 * th + i];
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int pc = 8 * (j >> 1) + 2 * lg + (j & 1);
+      st[th >> 1][4 * (th & 1) + j] = sc[l16 * 16 + (pc ^ l16)];
+    }
+    wave_lds_sync();
+  }
+}
+
+// The reverse, stored to dst: non-temporally for new_state (kNt), cached for a
+// segment slot that the finish reads.
+template <bool kNt>
+__device__ __forceinline__ void store_state_tiles(float* __restrict__ dst, const f32x4 (&st)[2][8], f32x4* sc,
+                                                  int lane) {
+  const int l16 = lane & 15, lg = lane >> 4;
+  float* p = dst + lg * kDim + 4 * l16;
+#pragma unroll
+  for (int th = 0; th < 4; ++th) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int pc = 8 * (j >> 1) + 2 * lg + (j & 1);
+      sc[l16 * 16 + (pc ^ l16)] = st[th >> 1][4 * (th & 1) + j];
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 4 * i + lg;
+      const f32x4 x = sc[row * 16 + (l16 ^ row)];
+      auto* d = reinterpret_cast<f32x4*>(p + (4 * (th >> 1) + 8 * i) * kDim + 64 * (th & 1));
+      if constexpr (kNt)
+        __builtin_nontemporal_store(x, d);
+      else
+        *d = x;
+    }
+    wave_lds_sync();
+  }
+}
+
+// bf16 S fragment of depth chunk d (slots st[2d + s/4][s%4]) and its rounding residue.
+__device__ __forceinline__ bf16x8 state_frag(const f32x4 (&st)[8], int d) {
+  float x[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) x[s] = st[2 * d + (s >> 2)][s & 3];
+  return round_frag(x);
+}
+
+// Operands of R = V - gam X, read while the last products of X run.
+struct WideR {
+  f32x4 gam[4];
+  u32x2 vw[2][4];   // [tile][token block]: V of the lane's column, four tokens
+};
+
+// A chunk's first phase: X = K S^T and, when the chunk has outputs (kEmit),
+// Y^T = S Q^T of both tiles and wave W's Aqk tiles (aqk_owner).  Depth
+// chunk by depth chunk: the K fragments of the next one are read while this
+// one's Y^T products run, and the Aqk tiles take their operands from the same
+// registers.
+template <int W, bool kEmit>
+__device__ __forceinline__ void wide_front(WideSmem& sm, int P, const f32x4 (&st)[2][8], int w, int lane,
+                                           f32x4 (&X)[2][4], f32x4 (&YT)[2][4], WideR& ro) {
+  lane = opaque_lane(lane);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int rsw = kq_swz(l16);
+  const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+  bf16x8 ka[2][4], qa[4];
+  auto read_k = [&](int d, int b) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      ka[b][m] = *reinterpret_cast<const bf16x8*>(&sm.ks[P][16 * m + l16][8 * ((4 * d + lg) ^ rsw)]);
+  };
+  f32x4 acc[4][4];   // the wave's tiles only
+  read_k(0, 0);
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int b = d & 1;
+    if constexpr (kEmit) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        qa[m] = *reinterpret_cast<const bf16x8*>(&sm.qs[16 * m + l16][8 * ((4 * d + lg) ^ rsw)]);
+    } else if (d < 3) {
+      read_k(d + 1, b ^ 1);
+    }
+    const bf16x8 s0 = state_frag(st[0], d), s1 = state_frag(st[1], d);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      X[0][m] = mfma16(ka[b][m], s0, d == 0 ? z : X[0][m]);
+      X[1][m] = mfma16(ka[b][m], s1, d == 0 ? z : X[1][m]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (kEmit && d < 3) read_k(d + 1, b ^ 1);
+    if (d == 3) {
+      // V columns by transposed reads: lane (lg, l16) addresses row
+      // 16 m + 4 lg + l16 / 4, value columns 32 w + 8 (l16 & 3) + 4 e .. + 3
+      const int vrow = 4 * lg + (l16 >> 2);
+      const int vat = 8 * ((4 * w + (l16 & 3)) ^ v_swz(vrow));
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        ro.gam[m] = *reinterpret_cast<const f32x4*>(&sm.gt[P][16 * m + 4 * lg]);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) ro.vw[e][m] = lds_tr16(&sm.vs[16 * m + vrow][vat + 4 * e]);
+      }
+    }
+    if constexpr (kEmit) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        YT[0][m] = mfma16(s0, qa[m], d == 0 ? z : YT[0][m]);
+        YT[1][m] = mfma16(s1, qa[m], d == 0 ? z : YT[1][m]);
+      }
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int m = a; m < 4; ++m)
+          if (aqk_owner(a, m) == W) acc[a][m] = mfma16(ka[b][a], qa[m], d == 0 ? z : acc[a][m]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if constexpr (kEmit) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int m = a; m < 4; ++m)
+        if (aqk_owner(a, m) == W) {
+          const f32x4 gi = *reinterpret_cast<const f32x4*>(&sm.gt[P][kLgamAt + 16 * a + 4 * lg]);
+          put_aqk_tile(sm.aqk, a, m, lane, acc[a][m], sm.gt[P][kLgamAt + 16 * m + l16], gi);
+        }
+  }
+}
+
+// One chunk of a wave's two tiles (see chain_chunk for the numerics, which are
+// the same).  emit: the chunk has outputs (a warm-up chunk has none).  copy_k /
+// copy_qvt issue the next chunk's copies.
+template <typename CopyK, typename CopyQvt>
+__device__ __forceinline__ void wide_chunk(WideSmem& sm, int P, int c, f32x4 (&st)[2][8], int w, int lane, float scale,
+                                           bool emit, __amdgpu_buffer_rsrc_t orc, uint32_t obase,
+                                           CopyK&& copy_k, CopyQvt&& copy_qvt) {
+  lane = opaque_lane(lane);
+  const int l16 = lane & 15, lg = lane >> 4;
+  copy_k();
+  const float cbound = sm.gt[P][kBoundAt];
+  const float tbi = sm.gt[P][kTbScaleAt];
+  f32x4 X[2][4], YT[2][4];
+  WideR ro;
+  if (emit) {
+    switch (w) {   // uniform
+      case 0: wide_front<0, true>(sm, P, st, w, lane, X, YT, ro); break;
+      case 1: wide_front<1, true>(sm, P, st, w, lane, X, YT, ro); break;
+      case 2: wide_front<2, true>(sm, P, st, w, lane, X, YT, ro); break;
+      default: wide_front<3, true>(sm, P, st, w, lane, X, YT, ro); break;
+    }
+  } else {
+    wide_front<0, false>(sm, P, st, w, lane, X, YT, ro);
+  }
+  if (cbound > kHiLoBoundLog2) {   // uniform: slow decay, the state's rounding residue enters X too
+    const int rsw = kq_swz(l16);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      bf16x8 lo[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        float x[8];
+        bf16x8 hi;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) x[s] = st[e][2 * d + (s >> 2)][s & 3];
+        split_frag(x, hi, lo[e]);
+      }
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const bf16x8 ka = *reinterpret_cast<const bf16x8*>(&sm.ks[P][16 * m + l16][8 * ((4 * d + lg) ^ rsw)]);
+        X[0][m] = mfma16(ka, lo[0], X[0][m]);
+        X[1][m] = mfma16(ka, lo[1], X[1][m]);
+      }
+    }
+  }
+  // ---- R = V - gam X, Delta = Tb R (fp16); Tb lands while R forms ----
+  f16x8 tb[kMatFrags];
+#pragma unroll
+  for (int f = 0; f < kMatFrags; ++f) tb[f] = *reinterpret_cast<const f16x8*>(&sm.tb[(f * 64 + lane) * 8]);
+  __builtin_amdgcn_sched_barrier(0);
+  f16x8 rf[2][2];
+  float rsc[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const u32x2 vw = ro.vw[e][m];
+      const float vv[4] = {bf_lo(vw.x), bf_hi(vw.x), bf_lo(vw.y), bf_hi(vw.y)};
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) X[e][m][rr] = vv[rr] - ro.gam[m][rr] * X[e][m][rr];
+    }
+    rsc[e] = r_scale(X[e]);
+    if (rsc[e] != 1.0f) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) X[e][m] = X[e][m] * rsc[e];
+    }
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      float x[8];
+      gather_slots(X[e], d, x);
+      rf[e][d] = half_frag(x);
+    }
+  }
+  f32x4 D[2][4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    D[0][m] = D[1][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+      if (!frag_zero(m, d)) {
+        D[0][m] = mfma16h(tb[frag_slot(m, d)], rf[0][d], D[0][m]);
+        D[1][m] = mfma16h(tb[frag_slot(m, d)], rf[1][d], D[1][m]);
+      }
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    if (rsc[e] != 1.0f || tbi != 1.0f) {
+      const float inv = tbi / rsc[e];   // exact: powers of two
+#pragma unroll
+      for (int m = 0; m < 4; ++m) D[e][m] = D[e][m] * inv;
+    }
+  lds_barrier();   // W1: every wave's Aqk tiles are in LDS; Q, V and Tb are dead
+  copy_qvt();
+
+  // ---- O^T = scale (Y^T diag(gam) + Delta^T Aqk^T): lane (lg, l16) holds
+  //      token 16 m + l16, value columns 32 w + 8 lg .. + 7 ----
+  if (emit) {
+    bf16x8 dob[2][2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        float x[8];
+        gather_slots(D[e], d, x);
+        dob[e][d] = round_frag(x);
+      }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int t = 16 * m + l16;
+      const float sg = scale * sm.gt[P][t];
+      f32x4 OT[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+        if (!frag_zero(m, d)) {
+          const bf16x8 fa = *reinterpret_cast<const bf16x8*>(&sm.aqk[(frag_slot(m, d) * 64 + lane) * 8]);
+          OT[0] = mfma16(dob[0][d], fa, OT[0]);
+          OT[1] = mfma16(dob[1][d], fa, OT[1]);
+        }
+      u32x4 pk;
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          pk[2 * e + j] = pack_bf2(sg * YT[e][m][2 * j] + scale * OT[e][2 * j],
+                                   sg * YT[e][m][2 * j + 1] + scale * OT[e][2 * j + 1]);
+      __builtin_amdgcn_raw_buffer_store_b128(pk, orc,
+                                             obase + static_cast<uint32_t>(t) * kVRow + 2 * (32 * w + 8 * lg),
+                                             0, 0);
+    }
+  }
+
+  // ---- Delta' = tail Delta (hi + lo); S^T <- gam_c S^T + K^T Delta' ----
+  bf16x8 dh[2][2], dlo[2][2];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const f32x4 tl = *reinterpret_cast<const f32x4*>(&sm.gt[P][kChunk + 16 * m + 4 * lg]);
+    D[0][m] = D[0][m] * tl;
+    D[1][m] = D[1][m] * tl;
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      float x[8];
+      gather_slots(D[e], d, x);
+      split_frag(x, dh[e][d], dlo[e][d]);
+    }
+  const float gam_c = sm.gt[P][c - 1];
+  const int tsw = kq_swz(4 * lg + (l16 >> 2));
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt) {
+    const int at = 8 * ((4 * (kt >> 1) + (l16 & 3)) ^ tsw) + 4 * (kt & 1);
+    f32x4 a0 = st[0][kt] * gam_c, a1 = st[1][kt] * gam_c;
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const int ta = perm_depth(d, lg, l16 >> 2);
+      const bf16x8 kta = join_frag(lds_tr16(&sm.ks[P][ta][at]), lds_tr16(&sm.ks[P][ta + 16][at]));
+      a0 = mfma16(kta, dh[0][d], a0);
+      a1 = mfma16(kta, dh[1][d], a1);
+      a0 = mfma16(kta, dlo[0][d], a0);
+      a1 = mfma16(kta, dlo[1][d], a1);
+    }
+    st[0][kt] = a0;
+    st[1][kt] = a1;
+  }
+}
+
+// Which batches run on the wide consumer: those whose (sequence, v-head) items
+// fill the chip by themselves.  More items than CUs (N > 32) of at most four
+// chunks on average, or two rounds of items (N >= 64) of any length.  Below
+// that the split consumer's shorter chunk step (1.9 us for a half head on a CU
+// of its own against 3.6 us for a whole head here) wins.  Measured per call,
+// split -> wide (fast gates, mean length x sequences): 30 x 48 30.2 -> 26.6 us,
+// 120 x 48 51.2 -> 41.3, 60 x 64 49.8 -> 34.2, 60 x 128 77.3 -> 55.1, 400 x 96
+// 143 -> 112, 34 x 512 169 -> 139; but 60 x 16 24.0 -> 29.2, 400 x 24 46 -> 48,
+// 400 x 48 77 -> 83.
+inline bool wide_batch(int num_seqs, long long tokens) {
+  return tokens <= kWideMaxTokens &&
+         (num_seqs >= kWideGroups / kVHeads ||
+          (num_seqs > kConsumerGroups / kVHeads && tokens <= 4ll * kChunk * num_seqs));
+}
+
+// Barrier W2: every wave's copies have landed (at most kPending vector-memory
+// operations, the chunk's output stores, are younger) and its LDS reads are done.
+template <int kPending>
+__device__ __forceinline__ void wide_barrier() {
+  static_assert(kPending >= 0 && kPending < 16, "vmcnt field");
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070 | kPending);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Work items: (run, v-head) of the run list in list order (longest first),
+// then (short sequence, v-head).  Group g starts with item g; later items are
+// claimed from the queue counter, the claim issued during the item's last
+// chunk.  See split_items for what a run is and where its results go.
+__global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const float* __restrict__ state, int R, int gcap, float scale, int* __restrict__ lists, int num_seqs,
+    const uint16_t* __restrict__ ws_frag, const float* __restrict__ ws_gam, uint16_t* __restrict__ out,
+    float* __restrict__ new_state, uint16_t* __restrict__ oi, float* __restrict__ slotb,
+    uint16_t* __restrict__ slotm, int* __restrict__ mval, int4* __restrict__ fix) {
+  __shared__ WideSmem sm;
+  const ListView lv = list_view(lists, num_seqs, gcap);
+  const int fix_cap = R * kVHeads;
+  // written by earlier launches, constant here: scalar loads
+  const auto* runs_c = (const __attribute__((address_space(4))) u32x4*)lv.runs;
+  const auto* shorts_c = (const __attribute__((address_space(4))) u32x4*)lv.shorts;
+  const auto* hdr_c = (const __attribute__((address_space(4))) int*)lv.hdr;
+  const auto* gam_c = (const __attribute__((address_space(4))) float*)ws_gam;
+  const int nruns = hdr_c[0], nshort = hdr_c[1], seg_len = hdr_c[2];
+  const int nitems = (nruns + nshort) * kVHeads;
+  const int nwg = static_cast<int>(gridDim.x);
+  int* queue = lv.hdr + 8;
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane0 = tid & 63;
+  const int vrow0 = 32 * w;                      // first value row of the wave
+  int zero_v;   // see split_items
+  asm volatile("v_mov_b32 %0, 0" : "=v"(zero_v));
+
+  for (int item = static_cast<int>(blockIdx.x); item < nitems;) {
+    int claimed = 0;
+    bool has_claim = false;
+    auto claim = [&] {
+      if (tid == 0 && !has_claim) {
+        claimed = atomicAdd(queue + zero_v, 1);
+        has_claim = true;
+      }
+    };
+    const int lane = opaque_lane(lane0);
+    const int l16 = lane & 15, lg = lane >> 4;
+    auto kappa = [&](int kt, int rr) { return 32 * (kt >> 1) + 8 * lg + 4 * (kt & 1) + rr; };
+    const int h = item & 7, li = item >> 3;
+    int s, slot, rfirst, last_tok, jseg, nvalid, nrun;
+    bool mrun, from_state, warm;
+    long long c0r;
+    if (li < nruns) {
+      const u32x4 ua = runs_c[2 * li], ub = runs_c[2 * li + 1];
+      s = static_cast<int>(ua.x);
+      slot = static_cast<int>(ua.z);
+      rfirst = static_cast<int>(ua.w);
+      mrun = (ua.y & kRunM) != 0;
+      from_state = (ua.y & kRunFromState) != 0;
+      warm = (ua.y & kRunWarm) != 0;
+      last_tok = min(static_cast<int>(ua.y >> 8) & 0xff, kChunk);
+      jseg = static_cast<int>(ua.y) >> 16;
+      c0r = static_cast<long long>(ub.x) | (static_cast<long long>(static_cast<int>(ub.y)) << 32);
+      nvalid = static_cast<int>(ub.z);
+      nrun = static_cast<int>(ub.w);
+    } else {
+      // a short sequence: one chunk (none when it is empty, or when malformed
+      // cu_seqlens left it without a record: the state then passes through)
+      const u32x4 e = shorts_c[li - nruns];
+      s = static_cast<int>(e.x);
+      slot = -1;
+      rfirst = static_cast<int>(e.y);
+      const int zw = static_cast<int>(e.w);
+      last_tok = min(zw >> 16, kChunk);
+      c0r = static_cast<long long>(e.z) | (static_cast<long long>(zw & 0xffff) << 32);
+      mrun = warm = false;
+      from_state = last_tok > 0;
+      jseg = 0;
+      nrun = 1;
+      nvalid = rfirst >= 0 && last_tok > 0 ? 1 : 0;
+    }
+    // warm-up chunks of a warm-up run (see split_items)
+    int warmup = 0;
+    if (warm && nvalid > 0) {
+      const int before = jseg * seg_len;
+      float acc = 0.0f;
+      while (warmup < before && acc >= kNegligibleLog2) {
+        float b4[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int back = min(warmup + j + 1, before);
+          b4[j] = gam_c[(static_cast<size_t>(rfirst - back) * kVHeads + h) * kGamStride + kBoundAt];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (warmup < before && acc >= kNegligibleLog2) {
+            acc += b4[j];
+            ++warmup;
+          }
+        }
+      }
+      if (acc >= kNegligibleLog2) from_state = true;   // from the sequence's first chunk
+    }
+    const int n = nvalid + warmup;
+    // the item's rows: warm-up chunks first; every chunk but the run's last is full
+    const long long c_base = c0r - static_cast<long long>(warmup) * kChunk;
+    const uint32_t rows = n > 0 ? static_cast<uint32_t>((warmup + nrun - 1) * kChunk + last_tok) : 0u;
+    WideItem wi;
+    {
+      const size_t kq0 = (static_cast<size_t>(c_base) * kQKHeads + h / kGva) * kDim;
+      const size_t v0 = (static_cast<size_t>(c_base) * kVHeads + h) * kDim;
+      const size_t r0 = static_cast<size_t>(rfirst - warmup) * kVHeads + h;
+      wi.k = rsrc_words(k + kq0, rows * kKqRow);
+      wi.q = rsrc_words(q + kq0, rows * kKqRow);
+      wi.v = rsrc_words(v + v0, mrun ? 0u : rows * kVRow);   // an M-run reads V = 0: every copy a zero fill
+      wi.fr = rsrc_words(ws_frag + r0 * kMatElems, n * kFragRec);
+      wi.g = rsrc_words(ws_gam + r0 * kGamStride, n * kGamRec);
+      wi.out = buf_rsrc((mrun ? oi : out) + v0, rows * kVRow);
+    }
+    f32x4* sc = reinterpret_cast<f32x4*>(&sm.ks[1][0][0]) + 256 * w;   // 4 KB: buffer 1 is free at the item's start
+    if (n > 0) {
+      wide_dma_k(sm, 0, wi, 0, lane0, w);
+      wide_dma_qvt(sm, wi, 0, lane0, w);
+    }
+    f32x4 st[2][8];
+    if (from_state && !mrun && state != nullptr) {
+      f32x4 r[16];
+      load_state_rows(state + (static_cast<size_t>(s) * kVHeads + h) * kHeadState + vrow0 * kDim, r, lane);
+      state_rows_to_tiles(r, st, sc, lane);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int kt = 0; kt < 8; ++kt)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr)
+            st[e][kt][rr] = mrun && kappa(kt, rr) == vrow0 + wide_row(e, l16) ? 1.0f : 0.0f;
+    }
+    const int fix_max = n;
+    int fix_pos = 0;
+    float lbound = 0.0f;
+    int formed = n;
+    int pl = 0;   // K buffer of the last chunk run
+    if (n > 0) {
+      wide_barrier<0>();
+      if (mrun && tid == 64) fix_pos = atomicAdd(lv.hdr + 9 + zero_v, fix_max);
+      for (int i = 0;; ++i) {
+        const int P = i & 1;
+        const bool more = i + 1 < n;
+        if (!more) claim();
+        const int c = i - warmup == nrun - 1 ? last_tok : kChunk;
+        wide_chunk(
+            sm, P, c, st, w, lane0, scale, i >= warmup, wi.out, static_cast<uint32_t>(i) * kChunk * kVRow,
+            [&] {
+              if (more) wide_dma_k(sm, P ^ 1, wi, i + 1, lane0, w);
+            },
+            [&] {
+              if (more) wide_dma_qvt(sm, wi, i + 1, lane0, w);
+            });
+        lbound += sm.gt[P][kBoundAt];
+        // W2: a warm-up chunk has no output stores younger than its copies
+        if (i >= warmup)
+          wide_barrier<kWideStores>();
+        else
+          wide_barrier<0>();
+        pl = P;
+        if (mrun && lbound < kNegligibleLog2) {
+          formed = i + 1;
+          break;
+        }
+        if (!more) break;
+      }
+      // an M-run that stopped early has its next chunk's K copies in flight
+      // into the other buffer, which serves as scratch below: they landed at
+      // the chunk's closing barrier
+    } else {
+      lds_barrier();   // every wave has read this item's index before it is replaced
+    }
+    claim();
+    if (tid == 0) sm.next_item = nwg + claimed;
+    if (mrun && tid == 0) mval[static_cast<size_t>(slot) * kVHeads + h] = formed | (formed < n ? kMNegligible : 0);
+    if (mrun && tid == 64 && fix_max > 0) {
+      const int4 seg = make_int4(static_cast<int>(c0r & 0xffffffffLL), static_cast<int>(c0r >> 32),
+                                 ((nrun - 1) * kChunk + last_tok) | (jseg << 17), slot - 1);
+      const int bsz = formed > kFinBlockChunks && jseg >= kFinBlockSeg ? kFinBlockChunks : 1;
+      for (int b = 0; b < fix_max && fix_pos + b < fix_cap; ++b) {
+        fix[2 * (fix_pos + b)] = seg;
+        fix[2 * (fix_pos + b) + 1] = make_int4(h, b * bsz, min((b + 1) * bsz, formed), 0);
+      }
+    }
+    if (slot != kSlotNone && !(mrun && formed < n)) {
+      f32x4* so = reinterpret_cast<f32x4*>(&sm.ks[pl ^ 1][0][0]) + 256 * w;
+      const size_t row = static_cast<size_t>(vrow0) * kDim;
+      if (slot < 0) {
+        store_state_tiles<true>(new_state + (static_cast<size_t>(s) * kVHeads + h) * kHeadState + row, st, so, lane);
+      } else if (!mrun) {
+        store_state_tiles<false>(slotb + (static_cast<size_t>(slot) * kVHeads + h) * kHeadState + row, st, so, lane);
+      } else {
+        const int lane = opaque_lane(lane0);
+        const int l16 = lane & 15, lg = lane >> 4;
+        auto kappa = [&](int kt, int rr) { return 32 * (kt >> 1) + 8 * lg + 4 * (kt & 1) + rr; };
+        // M^T fragments (see split_items): this lane holds k' = 32 w +
+        // wide_row(e, l16), so d = w, lg' = 2 (l16 / 4 & 1) + e, s = 4 (l16 / 8) + l16 % 4
+        uint16_t* mb = slotm + (static_cast<size_t>(slot) * kVHeads + h) * kMSlotElems;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int kt = 0; kt < 8; ++kt)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+              const int kk = kappa(kt, rr);
+              const float x = st[e][kt][rr];
+              const uint16_t hi = f2bf(x);
+              const uint16_t lo = f2bf(x - bf2f(hi));
+              const size_t at = ((static_cast<size_t>((kk >> 4) * 4 + w) * 2 * 64) + 16 * (2 * ((l16 >> 2) & 1) + e) +
+                                 (kk & 15)) * 8 +
+                                4 * (l16 >> 3) + (l16 & 3);
+              mb[at] = hi;
+              mb[at + 512] = lo;
+            }
+      }
+    }
+    lds_barrier();   // publishes the next item; the item's stores stay in flight
+    item = __builtin_amdgcn_readfirstlane(sm.next_item);
+  }
+}
+
+// ============================================================================
 // finish: states before segments, output correction, final states
 // ============================================================================
 // S_{j+1} = S_j M_j + B_j and O_j = O0_j + OI_j S_j^T.  An M-run that stopped
@@ -3117,10 +3823,11 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
   // small batches: every prepass work-group finds its own record (one launch
   // fewer); large ones: a separate plan launch numbers the records once
   const int fused_plan = num_seqs <= kFusedPlanSeqs ? 1 : 0;
+  const int wide = wide_batch(num_seqs, total_tokens) ? 1 : 0;
   if (!fused_plan)
     plan_kernel<<<dim3(1), dim3(kPlanThreads), 0, st>>>(cu_seqlens, cu_seqlens_is_int64, num_seqs,
                                                         total_tokens, Ri, gc, A_log, dt_bias, rec_start, recs,
-                                                        lists);
+                                                        lists, wide);
   // one wave per (record, v-head) while every item fits in one round: two
   // waves per SIMD for up to 2048 items (a lone item's latency matters there),
   // three (a tighter register budget) for up to 3072.  Larger batches take one
@@ -3131,27 +3838,33 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
     const long long g_pre = (items_v + kPrepassWaves - 1) / kPrepassWaves;
     prepass_kernel<false, 2><<<dim3(static_cast<unsigned>(g_pre + fused_plan)), dim3(kPrepassThreads), 0, st>>>(
         kb, A_log, ab, dt_bias, bb, recs, cu_seqlens, cu_seqlens_is_int64, num_seqs, total_tokens,
-        Ri, gc, fused_plan, rec_start, lists, frag, gam);
+        Ri, gc, fused_plan, rec_start, lists, frag, gam, wide);
   } else if (items_v <= 3 * (kPrepassMaxGroups / 2) * kPrepassWaves) {
     const long long g_pre = (items_v + kPrepassWaves - 1) / kPrepassWaves;
     prepass_kernel<false, 3><<<dim3(static_cast<unsigned>(g_pre + fused_plan)), dim3(kPrepassThreads), 0, st>>>(
         kb, A_log, ab, dt_bias, bb, recs, cu_seqlens, cu_seqlens_is_int64, num_seqs, total_tokens,
-        Ri, gc, fused_plan, rec_start, lists, frag, gam);
+        Ri, gc, fused_plan, rec_start, lists, frag, gam, wide);
   } else {
     const long long g_pre =
         std::min<long long>((R * kQKHeads + kPrepassWaves - 1) / kPrepassWaves, kPrepassMaxGroups);
     prepass_kernel<true, 2><<<dim3(static_cast<unsigned>(g_pre + fused_plan)), dim3(kPrepassThreads), 0, st>>>(
         kb, A_log, ab, dt_bias, bb, recs, cu_seqlens, cu_seqlens_is_int64, num_seqs, total_tokens,
-        Ri, gc, fused_plan, rec_start, lists, frag, gam);
+        Ri, gc, fused_plan, rec_start, lists, frag, gam, wide);
   }
-  // persistent grids: one work-group per CU per consumer kind at most; a
-  // sequence needs 2 chunks (65 tokens) to be long
-  const long long g_long =
-      total_tokens > kChunk ? std::min<long long>(max_runs(num_seqs, gcap) * 2 * kVHeads, kConsumerGroups) : 0;
-  const long long g_short = std::min<long long>(static_cast<long long>(num_seqs) * kVHeads, kConsumerGroups);
-  consumer_kernel<<<dim3(static_cast<unsigned>(g_long + g_short)), dim3(kSplitThreads), 0, st>>>(
-      qb, kb, vb, state, Ri, gc, scale, lists, num_seqs, static_cast<int>(g_long), frag, gam, ob, new_state, oi,
-      slotb, slotm, mval, fix);
+  // persistent grids: two wide groups per CU, or one group per CU per kind of
+  // the split launch; a sequence needs 2 chunks (65 tokens) to be long
+  if (wide) {
+    const long long g_wide = std::min<long long>(max_runs(num_seqs, gcap) * kVHeads, kWideGroups);
+    wide_kernel<<<dim3(static_cast<unsigned>(g_wide)), dim3(kWideThreads), 0, st>>>(
+        qb, kb, vb, state, Ri, gc, scale, lists, num_seqs, frag, gam, ob, new_state, oi, slotb, slotm, mval, fix);
+  } else {
+    const long long g_long =
+        total_tokens > kChunk ? std::min<long long>(max_runs(num_seqs, gcap) * 2 * kVHeads, kConsumerGroups) : 0;
+    const long long g_short = std::min<long long>(static_cast<long long>(num_seqs) * kVHeads, kConsumerGroups);
+    consumer_kernel<<<dim3(static_cast<unsigned>(g_long + g_short)), dim3(kSplitThreads), 0, st>>>(
+        qb, kb, vb, state, Ri, gc, scale, lists, num_seqs, static_cast<int>(g_long), frag, gam, ob, new_state, oi,
+        slotb, slotm, mval, fix);
+  }
   // a second segment needs more than kMinSegChunks chunks in one sequence and a slot
   if (gcap > 0 && total_tokens > static_cast<long long>(kMinSegChunks) * kChunk) {
     const long long g_fin = std::min<long long>(R * kVHeads, kFinGroups);
