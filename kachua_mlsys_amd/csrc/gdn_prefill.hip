@@ -127,7 +127,7 @@ __host__ __device__ inline long long max_segments(long long tokens) {
 //   [3] multi-segment sequences, [4] segments >= 1 over all sequences,
 //   [5] 1 when the batch uses warm-up segments (no M-runs, no finish work),
 //   [8] split-consumer work queue (items claimed past each group's first),
-//   [9] correction blocks appended by the consumer's M-runs
+//   [9] correction blocks appended by the consumer's M-runs, [10] finish queue
 //   multi[e]   = (seq, first slot, segments, 0)
 //   segs[i]    = (first token lo, hi, tokens in the segment | j << 17, slot of
 //                 segment j - 1) for every segment j >= 1 (L <= 1024 chunks:
@@ -159,19 +159,27 @@ constexpr int kRunWarm = 4;
 constexpr int kWarmMaxChunks = 4;
 constexpr int kSlotNone = -2;
 
-// Finish work: a correction block is one or more chunks of one (segment,
-// v-head); wave w of a finish group corrects 16-token tile w of each chunk.
-// A block first forms the segment's starting state, which for segment j can
-// take up to j - 1 scan steps.  The M-run of a segment j >= kFinBlockSeg that
-// formed more than kFinBlockChunks chunks lists blocks of kFinBlockChunks
-// chunks, so that state is formed once per block rather than once per chunk;
-// otherwise it lists one block per chunk, and the blocks run in parallel.
-constexpr int kFinThreads = 256;
-constexpr int kFinGroups = 512;   // one round at two groups per CU (the launch bounds)
-static_assert(kFinGroups == 64 * 8, "finish item permutation: 64 items per XCD");
-constexpr int kFinBlockChunks = 4;
-constexpr int kFinBlockSeg = 3;
-static_assert(kFinThreads / 64 == kChunk / 16, "finish tiling: one wave per 16-token tile");
+// Finish work: a correction block is a few chunks of one (segment, v-head);
+// four waves of a finish group correct a chunk (16 tokens each), so a group
+// takes two at a time.  An M-run of n chunks reserves fin_blocks(n) blocks when
+// it starts: pairs of chunks in shorter segments (more groups at work), four
+// chunks in longer ones (the state's fragments are fetched once per block),
+// and spreads the chunks it formed over them at its end.
+__host__ __device__ constexpr int fin_blocks(int n) { return n <= 24 ? (n + 1) / 2 : (n + 3) / 4; }
+__host__ __device__ constexpr int fin_block_chunks(int n, int formed) {
+  const int nb = fin_blocks(n), even = nb > 0 ? (formed + nb - 1) / nb : 0;
+  return even > 2 ? even : 2;
+}
+// The count of waves that have published the state before segment j: in the
+// first slot's M area, which no M-run writes (segment 0 has none).  The
+// M-run of segment j clears it.
+__device__ __forceinline__ int* seg_ready(uint16_t* slotm, int g0, int j, int h) {
+  return reinterpret_cast<int*>(slotm + (static_cast<size_t>(g0) * kVHeads + h) * kMSlotElems) + j;
+}
+
+constexpr int kFinThreads = 512;
+constexpr int kFinGroups = 256;   // one group per CU
+static_assert(kFinThreads / 64 == 2 * kChunk / 16, "finish tiling: one wave per 16-token tile of two chunks");
 __host__ __device__ inline long long max_runs(int num_seqs, long long gcap) { return 2 * gcap + num_seqs; }
 
 struct ListView {
@@ -246,6 +254,9 @@ __host__ __device__ inline WsLayout ws_layout(int num_seqs, long long tokens, lo
 // segment map per v-head).  The planner's best segmentings of the benchmark
 // batches use at most a few dozen (16 sequences of 16384 tokens: 10).
 constexpr long long kDefaultSlots = 48;
+// A sequence's segments are counted ready in one slot's 64 KB (seg_ready).
+constexpr long long kMaxSlots = 16384;
+static_assert(kMaxSlots * sizeof(int) <= kMSlotElems * sizeof(uint16_t), "a count per segment");
 
 // The most slots (up to what the batch can use) whose layout fits `bytes`, or
 // -1 when not even the layout without slots fits.
@@ -569,9 +580,6 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
                          ? kChunk * kLog2e * log_decay(A_log[min(lane, kVHeads - 1)], 0.0f,
                                                        dt_bias[min(lane, kVHeads - 1)])
                          : -1.0e30f;
-    // fraction of v-heads that decay slowly (see below)
-    const bool slow_h = lane < kVHeads && 2.0f * hb > kNegligibleLog2;
-    const float slow_frac = static_cast<float>(__popcll(__builtin_amdgcn_ballot_w64(slow_h))) / kVHeads;
     // warm-up chunks each head needs (estimate), and the scheme
     const int wh = hb < kNegligibleLog2 ? 1 : (hb < 0.f ? static_cast<int>(ceilf(kNegligibleLog2 / hb)) : 1 << 20);
     const int w_est = wave_max0(min(wh, 1 << 20));
@@ -594,7 +602,6 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       slots += pj[kSegCands + ci];
       runs += static_cast<float>(pj[2 * kSegCands + ci]);
     }
-    constexpr float kItemOverhead = 1.0f;   // chunk steps per work item (metadata, state, first copies)
     const int Lc = seg_cand(ci);
     const int nseg_max = ml > 0 ? (ml - 1) / Lc + 1 : 0;
     float est;
@@ -620,26 +627,26 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       const float tail = T > kMachines ? kTailShare * (work / fmaxf(T, 1.f) + kWarmItem) : 0.f;
       est = fmaxf(longest + kWarmItem, balanced + tail) + (nseg_max > 1 ? kSegmented : 0.f);
     } else {
-      // M-run scheme: W(L) counts the M-runs of later segments.  The scan
-      // adds about half a step per segment and segmenting at all 1.5 steps.
-      const float per_wg = (2.f * sl - a + kItemOverhead * runs) * (wide ? 8.f : 16.f) / kConsumerGroups;
-      const float crit = static_cast<float>(min(Lc, ml)) + kItemOverhead;
-      est = fmaxf(crit, per_wg) + (nseg_max > 1 ? 0.5f * static_cast<float>(nseg_max - 1) + 1.5f : 0.f);
-    }
-    // Slowly decaying heads: their segment maps never become negligible, so
-    // every correction block of segment j >= 2 in the finish first takes j - 1
-    // scan steps.  The heads' chunk map bound is estimated from the per-head
-    // constants (a = 0): 64 log2 g = -64 log2(e) exp(A_log) softplus(dt_bias);
-    // a head is slow when two chunks do not reach the negligible bound.  Such
-    // batches pay about kScanStepCost chunk steps per chunk of the longest
-    // sequence's segments j >= 2, weighted by j - 1 (measured with forced
-    // segment lengths on configuration 3 with near-1 decay).
-    if (!warm && slow_frac > 0.f && nseg_max >= 3) {
-      constexpr float kScanStepCost = 0.45f;
-      const int last = ml - (nseg_max - 1) * Lc;
-      const float pj = static_cast<float>(Lc) * static_cast<float>((nseg_max - 3) * (nseg_max - 2) / 2) +
-                       static_cast<float>(last) * static_cast<float>(nseg_max - 2);
-      est += slow_frac * kScanStepCost * pj;
+      // M-run scheme: a later segment runs twice, its M-run per v-head only
+      // until the head's map is negligible (about wh chunks).  The same list
+      // schedule over all runs; the finish adds its scan (0.4 steps per segment
+      // of the longest sequence), the corrections (48 KB of traffic per
+      // corrected chunk and v-head) and 6 steps for having any.  Measured with
+      // forced lengths (mixed or near-1 gates, us per call at this estimate's
+      // choice / unsegmented): 1 x 1024 tokens 42 / 48, 1 x 8192 91 / 227,
+      // 1 x 32768 195 / 830; 32 x 256 50 unsegmented, 61 at L <= 10.
+      constexpr float kRunItem = 1.5f, kTailShare = 0.25f, kCorrShare = 0.04f, kScan = 0.4f, kFinish = 6.0f;
+      const float kMachines = static_cast<float>(kConsumerGroups / (wide ? 8 : 16));
+      float mfrac = 0.f;
+#pragma unroll
+      for (int hh = 0; hh < kVHeads; ++hh)
+        mfrac += static_cast<float>(min(__builtin_amdgcn_readlane(wh, hh), Lc)) / (kVHeads * static_cast<float>(Lc));
+      const float mwork = (sl - a) * mfrac;
+      const float longest = static_cast<float>(min(Lc, ml));
+      const float balanced = (sl + mwork + kRunItem * runs) / kMachines;
+      const float tail = runs > kMachines ? kTailShare * ((sl + mwork) / fmaxf(runs, 1.f) + kRunItem) : 0.f;
+      est = fmaxf(longest + kRunItem, balanced + tail) +
+            (nseg_max > 1 ? kScan * static_cast<float>(nseg_max - 1) + kFinish + kCorrShare * mwork : 0.f);
     }
     // key: estimate in 1/16 steps, then the longer candidate; invalid lanes hold
     // the maximum.  No slot is written in the warm-up scheme, but the slot
@@ -696,6 +703,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     if (lane == 0) {
       lv.hdr[8] = 0;   // work queue
       lv.hdr[9] = 0;   // correction blocks
+      lv.hdr[10] = 0;  // finish queue
     }
     if (lane == 63) {
       lv.hdr[0] = tot[4] + inc;
@@ -2638,14 +2646,12 @@ __device__ __forceinline__ void split_items(
   };
   const SplitDmaLane dl = split_dma_lane(wt, lane, hv);
   // Correction blocks of the segment: chunks [0, formed) get O0 + OI S_j^T in
-  // the finish.  Each M-run (once per v-head) reserves a block per chunk with
-  // records during its first chunk (the atomic returns before that chunk's
-  // closing barrier, with the next chunk's copies), and fills them at its end
-  // with blocks of one chunk, or of kFinBlockChunks chunks (see kFinBlockSeg);
-  // blocks past `formed` are left empty.  The finish then
-  // takes one block per group with a single descriptor load.  The entry
-  // repeats the later-segment table's.
-  const int fix_max = n;
+  // the finish.  Each M-run (once per v-head) reserves its blocks (fin_blocks)
+  // during its first chunk (the atomic returns before that chunk's closing
+  // barrier, with the next chunk's copies), and fills them at its end; blocks
+  // past `formed` are left empty.  The finish then takes a block with a single
+  // descriptor load.  The entry repeats the later-segment table's.
+  const int fix_max = fin_blocks(n);
   int fix_pos = 0;
 
   // An M-run stops once the bound of its map falls below kNegligibleLog2: its
@@ -2709,10 +2715,13 @@ __device__ __forceinline__ void split_items(
   // wave, and the stores would be among them.
   claim();
   if (threadIdx.x == 0) sm.next_item = nwg + claimed;
-  if (mrun && tid == 0) mval[static_cast<size_t>(slot) * kVHeads + h] = formed | (formed < n ? kMNegligible : 0);
+  if (mrun && tid == 0) {
+    mval[static_cast<size_t>(slot) * kVHeads + h] = formed | (formed < n ? kMNegligible : 0);
+    *seg_ready(slotm, slot - jseg, jseg, h) = 0;
+  }
   if (mrun && hv == 0 && tid == kFixLane && fix_max > 0) {
     const int4 seg = make_int4(rb.x, rb.y, ((nrun - 1) * kChunk + last_tok) | (jseg << 17), slot - 1);
-    const int bsz = formed > kFinBlockChunks && jseg >= kFinBlockSeg ? kFinBlockChunks : 1;
+    const int bsz = fin_block_chunks(n, formed);
     for (int b = 0; b < fix_max && fix_pos + b < fix_cap; ++b) {
       fix[2 * (fix_pos + b)] = seg;
       fix[2 * (fix_pos + b) + 1] = make_int4(h, b * bsz, min((b + 1) * bsz, formed), 0);
@@ -3408,7 +3417,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
           for (int rr = 0; rr < 4; ++rr)
             st[e][kt][rr] = mrun && kappa(kt, rr) == vrow0 + wide_row(e, l16) ? 1.0f : 0.0f;
     }
-    const int fix_max = n;
+    const int fix_max = fin_blocks(n);
     int fix_pos = 0;
     float lbound = 0.0f;
     int formed = n;
@@ -3450,11 +3459,14 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
     }
     claim();
     if (tid == 0) sm.next_item = nwg + claimed;
-    if (mrun && tid == 0) mval[static_cast<size_t>(slot) * kVHeads + h] = formed | (formed < n ? kMNegligible : 0);
+    if (mrun && tid == 0) {
+      mval[static_cast<size_t>(slot) * kVHeads + h] = formed | (formed < n ? kMNegligible : 0);
+      *seg_ready(slotm, slot - jseg, jseg, h) = 0;
+    }
     if (mrun && tid == 64 && fix_max > 0) {
       const int4 seg = make_int4(static_cast<int>(c0r & 0xffffffffLL), static_cast<int>(c0r >> 32),
                                  ((nrun - 1) * kChunk + last_tok) | (jseg << 17), slot - 1);
-      const int bsz = formed > kFinBlockChunks && jseg >= kFinBlockSeg ? kFinBlockChunks : 1;
+      const int bsz = fin_block_chunks(n, formed);
       for (int b = 0; b < fix_max && fix_pos + b < fix_cap; ++b) {
         fix[2 * (fix_pos + b)] = seg;
         fix[2 * (fix_pos + b) + 1] = make_int4(h, b * bsz, min((b + 1) * bsz, formed), 0);
@@ -3500,129 +3512,197 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
 // ============================================================================
 // finish: states before segments, output correction, final states
 // ============================================================================
-// S_{j+1} = S_j M_j + B_j and O_j = O0_j + OI_j S_j^T.  An M-run that stopped
-// early (kMNegligible) has a map below 2^-30, so the state after its segment is
-// B_j itself: the state before segment j is rebuilt from the latest such
-// segment before it (or from S_1), with scan steps only across segments whose
-// maps are not negligible.  Work items, one work-group each:
-//   a correction block (segment j >= 1, v-head, one or kFinBlockChunks chunks
-//        whose OI was formed), as the consumer's M-run appended it: S_j, then
-//        out = bf16(O0 + OI S_j^T) for the block's chunks (the other chunks
-//        keep O0), chunk by chunk, wave w taking 16-token tile w;
-//   (multi-segment sequence, v-head): new_state = S_nseg.
+// S_{j+1} = S_j M_j + B_j and O_j = O0_j + OI_j S_j^T.  Work items, claimed in
+// order from a queue counter:
+//   (multi-segment sequence, v-head, 32 value rows): the scan.  Rows of S are
+//        independent through the scan, so four groups share a head.  S_1 comes
+//        from the first slot; each step adds S_j M_j to B_j (or takes B_j
+//        alone after an M-run that stopped early, whose map is negligible) and
+//        publishes S_j as bf16 correction fragments; S_nseg goes to new_state.
+//   a correction block (segment j >= 1, v-head, a few chunks whose OI was
+//        formed), as the consumer's M-run appended it: waits
+//        until S_j is published, then out = bf16(O0 + OI S_j^T), wave w taking
+//        16-token tile w of each chunk (the other chunks keep O0).
+// Scan items precede every block in the queue and wait for nothing, so a block
+// only ever waits for items that running groups hold, whatever share of the
+// grid is resident.
+//
+// Forming S_j once per segment instead of once per block: a block of segment
+// j used to repeat up to j - 1 steps, which made long slowly decaying
+// sequences run in few segments.  One 32,768-token sequence with mixed gates
+// (some heads forget within a chunk, some hold for thousands of tokens):
+// 409 -> 187 us per call, one of 8,192 with near-1 decay 145 -> 95 us; 16 x 1024
+// tokens with near-1 decay (two or three segments) unchanged.  A step is bound
+// by the latency of its chain (LDS exchange, 24 MFMAs per wave, conversion:
+// about 1 us); its M and B operands are requested kScanAhead steps ahead.
+//
 // A scan step forms D = M^T S^T on MFMA with M^T as the M-run stored it (bf16
-// hi / lo) and S split into hi / lo from LDS (three products, fp32
-// accumulation from B_i).  The correction multiplies OI (bf16) by S as a single
-// bf16, as the chunk recurrence does in Q S^T.
-constexpr int kFinRow = kDim + 4;   // floats per LDS row of S
+// hi / lo) and S split into hi / lo (three products, fp32 accumulation from
+// B_j).  Wave w forms k tile w of both row tiles: as a B operand in permuted
+// order they are half of depth chunk w / 2 of the next step, so the waves trade
+// 8-byte halves of fragments through LDS.  The correction multiplies OI (bf16)
+// by S as a single bf16, as the chunk recurrence does in Q S^T.
+//
+// Published data crosses XCDs within the launch: it is stored and loaded past
+// the XCD's own L2 (sc0 sc1), and the count of finished waves is raised only
+// after the storing wave has waited for its stores (vector memory operations of
+// a wave complete in issue order).
+constexpr int kFinRows = 32;                      // value rows of a scan item
+constexpr int kFinParts = kDim / kFinRows;        // scan items per (sequence, v-head)
+constexpr int kFinReady = kFinParts * (kFinThreads / 64);   // waves that publish a segment's state
+constexpr int kScanAhead = 3;                     // steps between a step's loads and their use
+constexpr int kSc01 = 1 | 16;                     // cache policy bits sc0 and sc1
 
 union FinishLds {
-  float s[kDim][kFinRow];          // S (fp32, row-major, padded)
-  u32x4 frag[8][4][64];            // S as correction A fragments: [v-tile][d][lane], slot s = S[16 vt + l16][32 d + 8 lg + s]
+  u32x4 x[2][2][4][2][64];   // scan: [parity][row tile][depth chunk][hi / lo][lane]
+  // block: S as A fragments: [v-tile][d][lane], slot s of v-tile 2 p + e =
+  // S[32 p + wide_row(e, l16)][32 d + 8 lg + s]
+  u32x4 frag[8][4][64];
 };
 
-// One slot state (64 KB, row-major) into registers, thread tid taking the
-// 16-byte pieces tid + e * kFinThreads.
-constexpr int kFinPer = kDim * kDim / 4 / kFinThreads;
-__device__ __forceinline__ void load_slot(const float* __restrict__ src, f32x4 (&t)[kFinPer]) {
-  const int tid = threadIdx.x;
+// Operands of scan step i: M_i^T fragments of the wave's k tile and B_i (the
+// accumulators), rows r0 + 16 rt + l16, k = 16 w + 4 lg ..
+struct ScanOps {
+  bf16x8 m[4][2];   // [depth chunk][hi / lo]
+  f32x4 b[2];       // [row tile]
+};
+__device__ __forceinline__ void scan_load_b(const float* __restrict__ slot, int r0, int w, int lane, f32x4 (&b)[2]) {
 #pragma unroll
-  for (int e = 0; e < kFinPer; ++e) {
-    const int q4 = tid + e * kFinThreads;
-    t[e] = *reinterpret_cast<const f32x4*>(src + (q4 >> 5) * kDim + (q4 & 31) * 4);
-  }
+  for (int rt = 0; rt < 2; ++rt)
+    b[rt] = *reinterpret_cast<const f32x4*>(slot + (r0 + 16 * rt + (lane & 15)) * kDim + 16 * w + 4 * (lane >> 4));
 }
 
-// State before segment j of the sequence whose slots start at g0, v-head h,
-// into sm.s (fp32).  S_{i+1} is exactly slotb[g0 + i] for i = 0 (S_1) and after
-// a negligible map (B_i), so the rebuild starts from the latest such slot.  The
-// caller has loaded the usual one: `first` = slotb[g0 + j - 1], `prev` = the
-// M-run entry of segment j - 1 (any value with kMNegligible set when j = 1).
-__device__ void state_before(FinishLds& sm, int g0, int j, int h, const float* __restrict__ slotb,
-                             const uint16_t* __restrict__ slotm, const int* __restrict__ mval, int w, int lane,
-                             const f32x4 (&first)[kFinPer], int prev) {
-  const int tid = threadIdx.x;
+__device__ __forceinline__ void scan_item(FinishLds& sm, const int4& me, int h, int part, float* __restrict__ slotb,
+                                          uint16_t* __restrict__ slotm, const int* __restrict__ mval,
+                                          float* __restrict__ new_state, int w, int lane) {
   const int l16 = lane & 15, lg = lane >> 4;
-  int i0 = j - 1;
-  if ((prev & kMNegligible) == 0) {
-    // segment j-1's map is not negligible: step back to the latest slot that is a state
-    --i0;
-    while (i0 > 0 && (mval[static_cast<size_t>(g0 + i0) * kVHeads + h] & kMNegligible) == 0) --i0;
-    f32x4 t[kFinPer];
-    load_slot(slotb + (static_cast<size_t>(g0 + i0) * kVHeads + h) * kHeadState, t);
-    __builtin_amdgcn_sched_barrier(0);
+  const int g0 = me.y, nseg = me.z, r0 = kFinRows * part;
+  auto head = [&](int j) { return static_cast<size_t>(g0 + j) * kVHeads + h; };
+  f32x4 s[2];   // S_j in C layout: rows k = 16 w + 4 lg + rr, column (value row) r0 + 16 rt + l16
+  scan_load_b(slotb + head(0) * kHeadState, r0, w, lane, s);
+  // bit i of neg: the map of segment jb + i is negligible
+  unsigned long long neg = 0;
+  int jb = 1;
+  auto read_neg = [&] {
+    const int v = mval[head(min(jb + lane, nseg - 1))];
+    neg = __builtin_amdgcn_ballot_w64((v & kMNegligible) != 0);
+  };
+  // step j's operands, requested whether the map is used or not (a stopped
+  // M-run's slot may hold anything) and past the last segment too: every step
+  // issues the same number of loads, so a step waits for its own only
+  ScanOps op[kScanAhead];
+  auto load_ops = [&](int j, ScanOps& o) {
+    const size_t hd = head(min(j, nseg - 1));
+    const uint16_t* mp = slotm + hd * kMSlotElems + lane * 8;
 #pragma unroll
-    for (int e = 0; e < kFinPer; ++e) {
-      const int q4 = tid + e * kFinThreads;
-      *reinterpret_cast<f32x4*>(&sm.s[q4 >> 5][(q4 & 31) * 4]) = t[e];
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int hl = 0; hl < 2; ++hl)
+        o.m[d][hl] = *reinterpret_cast<const bf16x8*>(mp + ((w * 4 + d) * 2 + hl) * kFragTile);
+    scan_load_b(slotb + hd * kHeadState, r0, w, lane, o.b);
+  };
+#pragma unroll
+  for (int k = 0; k < kScanAhead; ++k) load_ops(1 + k, op[k]);
+  auto raise = [&](int j) {   // this wave's share of S_j is out
+    if (lane == 0)
+      __hip_atomic_fetch_add(seg_ready(slotm, g0, j, h), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  // kLong: of more than kScanAhead steps.  A short scan has every operand in
+  // flight from the start, so it waits for its publication at once
+  auto step = [&](int j, ScanOps& o, auto LC) {
+    constexpr bool kLong = decltype(LC)::value;
+    const int P = j & 1;
+    // S_j into LDS: half e = w & 1 of the fragments of depth chunk w / 2
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      const uint32_t h0 = pack_bf2(s[rt][0], s[rt][1]), h1 = pack_bf2(s[rt][2], s[rt][3]);
+      const u32x2 lo = {pack_bf2(s[rt][0] - bf_lo(h0), s[rt][1] - bf_hi(h0)),
+                        pack_bf2(s[rt][2] - bf_lo(h1), s[rt][3] - bf_hi(h1))};
+      *(reinterpret_cast<u32x2*>(&sm.x[P][rt][w >> 1][0][lane]) + (w & 1)) = u32x2{h0, h1};
+      *(reinterpret_cast<u32x2*>(&sm.x[P][rt][w >> 1][1][lane]) + (w & 1)) = lo;
     }
-  } else {
+    // this step's operands; the state published kScanAhead steps ago, issued
+    // before them, is out as well
+    asm volatile("" ::"v"(o.m[0][0]), "v"(o.m[0][1]), "v"(o.m[1][0]), "v"(o.m[1][1]), "v"(o.m[2][0]), "v"(o.m[2][1]),
+                 "v"(o.m[3][0]), "v"(o.m[3][1]), "v"(o.b[0]), "v"(o.b[1])
+                 : "memory");
+    if (kLong && j > kScanAhead) raise(j - kScanAhead);
+    lds_barrier();   // S_j in LDS; every wave holds its rows of B_{j-1}, whose place S_j takes
+    // publish S_j: natural-order A fragments, 8 bytes per row tile.  Value row
+    // 16 rt + l16 of the part goes to row i of v-tile e, 16 rt + l16 =
+    // wide_row(e, i), so that a block's lanes hold eight consecutive columns
+    auto* pub = reinterpret_cast<unsigned long long*>(slotb + head(j - 1) * kHeadState + r0 * kDim);
 #pragma unroll
-    for (int e = 0; e < kFinPer; ++e) {
-      const int q4 = tid + e * kFinThreads;
-      *reinterpret_cast<f32x4*>(&sm.s[q4 >> 5][(q4 & 31) * 4]) = first[e];
+    for (int rt = 0; rt < 2; ++rt) {
+      const u32x2 pk = {pack_bf2(s[rt][0], s[rt][1]), pack_bf2(s[rt][2], s[rt][3])};
+      const int e = (l16 >> 2) & 1, i = 4 * (2 * rt + (l16 >> 3)) + (l16 & 3);
+      __hip_atomic_store(pub + ((e * 4 + (w >> 1)) * 64 + 16 * (2 * (w & 1) + (lg >> 1)) + i) * 2 + (lg & 1),
+                         __builtin_bit_cast(unsigned long long, pk), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
-  }
-  __syncthreads();
-  for (int i = i0 + 1; i < j; ++i) {
-    // wave w forms output k-tiles 2w, 2w+1 for all 128 rows: D = M^T S^T; the
-    // step's operand loads are all issued before the first product
-    const size_t gh = static_cast<size_t>(g0 + i) * kVHeads + h;
-    const uint16_t* mp = slotm + gh * kMSlotElems + lane * 8;
-    const float* bp = slotb + gh * kHeadState;
-    bf16x8 am[2][4][2];
+    if constexpr (!kLong) {
+      __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+      asm volatile("" ::: "memory");
+      raise(j);
+    }
+    const bool map = ((neg >> (j - jb)) & 1) == 0;
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
+    for (int rt = 0; rt < 2; ++rt) s[rt] = o.b[rt];
+    if (map) {
 #pragma unroll
       for (int d = 0; d < 4; ++d)
 #pragma unroll
-        for (int hl = 0; hl < 2; ++hl)
-          am[e][d][hl] = *reinterpret_cast<const bf16x8*>(mp + (((2 * w + e) * 4 + d) * 2 + hl) * 512);
-    f32x4 acc[8][2];
-#pragma unroll
-    for (int vb = 0; vb < 8; ++vb)
-#pragma unroll
-      for (int e = 0; e < 2; ++e)
-        acc[vb][e] = *reinterpret_cast<const f32x4*>(bp + (16 * vb + l16) * kDim + 16 * (2 * w + e) + 4 * lg);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int vb = 0; vb < 8; ++vb) {
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        // B fragment: slot s of chunk d is S[16 vb + l16][perm_depth(d, lg, s)]
-        const f32x4 x0 = *reinterpret_cast<const f32x4*>(&sm.s[16 * vb + l16][32 * d + 4 * lg]);
-        const f32x4 x1 = *reinterpret_cast<const f32x4*>(&sm.s[16 * vb + l16][32 * d + 16 + 4 * lg]);
-        const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-        bf16x8 sh, sl;
-        split_frag(x, sh, sl);
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          acc[vb][e] = mfma16(am[e][d][0], sh, acc[vb][e]);
-          acc[vb][e] = mfma16(am[e][d][0], sl, acc[vb][e]);
-          acc[vb][e] = mfma16(am[e][d][1], sh, acc[vb][e]);
+        for (int rt = 0; rt < 2; ++rt) {
+          const bf16x8 sh = __builtin_bit_cast(bf16x8, sm.x[P][rt][d][0][lane]);
+          const bf16x8 sl = __builtin_bit_cast(bf16x8, sm.x[P][rt][d][1][lane]);
+          s[rt] = mfma16(o.m[d][0], sh, s[rt]);
+          s[rt] = mfma16(o.m[d][0], sl, s[rt]);
+          s[rt] = mfma16(o.m[d][1], sh, s[rt]);
         }
-      }
     }
-    __syncthreads();   // every wave has read S_i
-    // acc[vb][e][rr] = S_{i+1}[16 vb + l16][16 (2w + e) + 4 lg + rr]
+    if constexpr (kLong) load_ops(j + kScanAhead, o);
+  };
+  constexpr int kBlock = 64 / kScanAhead * kScanAhead;   // steps per read_neg
+  const bool lng = nseg > kScanAhead + 1;
+  if (!lng) {
+    read_neg();
 #pragma unroll
-    for (int vb = 0; vb < 8; ++vb)
+    for (int k = 0; k < kScanAhead; ++k)
+      if (1 + k < nseg) step(1 + k, op[k], std::false_type{});
+  } else {
+    for (; jb < nseg; jb += kBlock) {
+      read_neg();
+      const int je = min(jb + kBlock, nseg);
+      int j = jb;
+      for (; j + kScanAhead <= je; j += kScanAhead) {
 #pragma unroll
-      for (int e = 0; e < 2; ++e)
-        *reinterpret_cast<f32x4*>(&sm.s[16 * vb + l16][16 * (2 * w + e) + 4 * lg]) = acc[vb][e];
-    __syncthreads();
+        for (int k = 0; k < kScanAhead; ++k) step(j + k, op[k], std::true_type{});
+      }
+#pragma unroll
+      for (int k = 0; k < kScanAhead - 1; ++k)
+        if (j + k < je) step(j + k, op[k], std::true_type{});
+    }
+  }
+  float* dst = new_state + (static_cast<size_t>(me.x) * kVHeads + h) * kHeadState;
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt)
+    *reinterpret_cast<f32x4*>(dst + (r0 + 16 * rt + l16) * kDim + 16 * w + 4 * lg) = s[rt];
+  if (lng) {
+    __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0), lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    for (int j = nseg - kScanAhead; j < nseg; ++j) raise(j);
   }
 }
 
-__global__ __launch_bounds__(kFinThreads, 2) void finish_kernel(int* __restrict__ lists, int num_seqs, int gcap,
+__global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ lists, int num_seqs, int gcap,
                                                              const int4* __restrict__ fix, int fix_cap,
-                                                             const float* __restrict__ slotb,
-                                                             const uint16_t* __restrict__ slotm,
+                                                             float* __restrict__ slotb,
+                                                             uint16_t* __restrict__ slotm,
                                                              const int* __restrict__ mval,
                                                              const uint16_t* __restrict__ oi,
                                                              uint16_t* __restrict__ out,
                                                              float* __restrict__ new_state) {
   __shared__ FinishLds sm;
+  __shared__ int claimed;
   const ListView lv = list_view(lists, num_seqs, gcap);
   const int nmulti = lv.hdr[3];
   const int ncorr = min(lv.hdr[9], fix_cap);   // correction blocks
@@ -3632,44 +3712,30 @@ __global__ __launch_bounds__(kFinThreads, 2) void finish_kernel(int* __restrict_
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int l16 = lane & 15, lg = lane >> 4;
-  // The state items first: they may step through several segment maps.  The
-  // grid is one round of groups (two per CU); items past it go out in
-  // alternating order, pass k taking group g's item k G + g for even k and
-  // (k + 1) G - 1 - g for odd k, so second items land on the groups whose
-  // first item was a cheap one (the last correction blocks) rather than on
-  // the state items.
-  // With a full grid, the group's position in the item order is permuted so
-  // that runs of 64 consecutive items (the blocks of one segment and v-head,
-  // which load the same segment state and maps) share an XCD (group id % 8)
-  // and find those in one L2.
-  const int G = static_cast<int>(gridDim.x);
-  const int nitem = ncorr + nmulti * kVHeads;
-  const int gid = static_cast<int>(blockIdx.x);
-  const int slot_g = G == kFinGroups ? 64 * (gid & 7) + (gid >> 3) : gid;
-  for (int pass = 0;; ++pass) {
-    const int it = (pass & 1) ? (pass + 1) * G - 1 - slot_g : pass * G + slot_g;
+  const int nscan = nmulti * kVHeads * kFinParts;
+  const int nitem = ncorr + nscan;
+  if (nitem == 0) return;
+  // the next claim is requested while an item is worked on.  A group that waits
+  // in a block holds at most another block: claims only grow
+  int zero_v;   // as in split_items: a plain single-lane atomic, waited for at its use
+  asm volatile("v_mov_b32 %0, 0" : "=v"(zero_v));
+  int next = 0;
+  if (tid == 0) next = atomicAdd(lv.hdr + 10 + zero_v, 1);
+  for (;;) {
+    if (tid == 0) claimed = next;
+    __syncthreads();   // also: the previous item's readers of sm are done
+    const int it = __builtin_amdgcn_readfirstlane(claimed);
+    __syncthreads();   // every wave has the claim before the next one
     if (it >= nitem) break;
-    if (it < nmulti * kVHeads) {
-      const int h = it & 7;
-      // new_state = S_nseg
-      const int4 me = lv.multi[it >> 3];
-      // the usual starting slot and the entry that says whether it is the state
-      const int jl = me.z;
-      const int prev = jl >= 2 ? mval[static_cast<size_t>(me.y + jl - 1) * kVHeads + h] : kMNegligible;
-      f32x4 slot0[kFinPer];
-      load_slot(slotb + (static_cast<size_t>(me.y + jl - 1) * kVHeads + h) * kHeadState, slot0);
-      __syncthreads();   // the previous item's readers of sm are done
-      state_before(sm, me.y, jl, h, slotb, slotm, mval, w, lane, slot0, prev);
-      float* dst = new_state + (static_cast<size_t>(me.x) * kVHeads + h) * kHeadState;
-      for (int e = tid; e < kDim * kDim / 4; e += kFinThreads) {
-        const int row = e >> 5, col = (e & 31) * 4;
-        *reinterpret_cast<f32x4*>(dst + row * kDim + col) = *reinterpret_cast<const f32x4*>(&sm.s[row][col]);
-      }
+    if (tid == 0) next = atomicAdd(lv.hdr + 10 + zero_v, 1);
+    if (it < nscan) {
+      scan_item(sm, lv.multi[it / (kVHeads * kFinParts)], (it / kFinParts) % kVHeads, it % kFinParts, slotb, slotm,
+                mval, new_state, w, lane);
       continue;
     }
     // block: (first token lo, hi, tokens | j << 17, slot of segment j - 1) and
     // (v-head, first chunk, end chunk): chunks [first, last) need OI S_j^T
-    const int item = it - nmulti * kVHeads;
+    const int item = it - nscan;
     const u32x4 fa = fix_c[2 * item], fb = fix_c[2 * item + 1];
     const int4 sg = make_int4(static_cast<int>(fa.x), static_cast<int>(fa.y), static_cast<int>(fa.z),
                               static_cast<int>(fa.w));
@@ -3679,13 +3745,15 @@ __global__ __launch_bounds__(kFinThreads, 2) void finish_kernel(int* __restrict_
     const int first = static_cast<int>(fb.y);
     const int last = min(static_cast<int>(fb.z), (tok + kChunk - 1) / kChunk);
     if (first >= last) continue;
-    // wave w corrects token tile w of each chunk of the block (all 128 value
-    // rows); the first chunk's OI and O0 loads are issued before the state is
-    // formed, each later chunk's after the previous chunk's stores
+    // waves 0-3 take the block's even chunks, waves 4-7 the odd ones, one
+    // 16-token tile each (all 128 value rows); the first chunk's OI and O0
+    // loads are issued before the wait for the state, each later chunk's after
+    // the previous chunk's stores
+    const int wt = w & 3;
     const long long c0s = static_cast<long long>(static_cast<unsigned>(sg.x)) | (static_cast<long long>(sg.y) << 32);
-    const uint32_t trow = static_cast<uint32_t>(16 * w + l16) * (kVHeads * kDim * 2);
+    const uint32_t trow = static_cast<uint32_t>(16 * wt + l16) * (kVHeads * kDim * 2);
     bf16x8 b[4];   // [d]: OI rows as B fragments
-    u32x2 o0[8];   // [value tile]: O0, four value columns
+    u32x4 o0[4];   // [pair of value tiles]: O0, eight value columns
     __amdgpu_buffer_rsrc_t orc;
     auto load_chunk = [&](int ci) {
       const long long c0 = c0s + static_cast<long long>(ci) * kChunk;
@@ -3698,45 +3766,49 @@ __global__ __launch_bounds__(kFinThreads, 2) void finish_kernel(int* __restrict_
       for (int d = 0; d < 4; ++d)
         b[d] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(irc, trow + 2 * (32 * d + 8 * lg), 0, 0));
 #pragma unroll
-      for (int vt = 0; vt < 8; ++vt) o0[vt] = __builtin_amdgcn_raw_buffer_load_b64(orc, trow + 2 * (16 * vt + 4 * lg), 0, 0);
+      for (int p = 0; p < 4; ++p) o0[p] = __builtin_amdgcn_raw_buffer_load_b128(orc, trow + 2 * (32 * p + 8 * lg), 0, 0);
     };
-    // the usual starting slot of the state rebuild, loaded with the outputs
-    const int prev = j >= 2 ? mval[static_cast<size_t>(g0 + j - 1) * kVHeads + h] : kMNegligible;
-    f32x4 slot0[kFinPer];
-    load_slot(slotb + (static_cast<size_t>(g0 + j - 1) * kVHeads + h) * kHeadState, slot0);
-    load_chunk(first);
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();   // the previous item's readers of sm are done
-    state_before(sm, g0, j, h, slotb, slotm, mval, w, lane, slot0, prev);
-    // S -> bf16 correction fragments (in place: read, barrier, write)
-    u32x4 fr[2][4];
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const float* sp = &sm.s[16 * (2 * w + e) + l16][32 * d + 8 * lg];
-        const f32x4 x0 = *reinterpret_cast<const f32x4*>(sp);
-        const f32x4 x1 = *reinterpret_cast<const f32x4*>(sp + 4);
-        fr[e][d] = u32x4{pack_bf2(x0[0], x0[1]), pack_bf2(x0[2], x0[3]), pack_bf2(x1[0], x1[1]),
-                         pack_bf2(x1[2], x1[3])};
-      }
+    const int my = first + (w >> 2);
+    if (my < last) load_chunk(my);
+    if (tid == 0) {
+      int* rd = seg_ready(slotm, g0, j, h);
+      while (__hip_atomic_load(rd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kFinReady) __builtin_amdgcn_s_sleep(2);
+    }
     __syncthreads();
+    // S_j's fragments, published over the slot of segment j - 1: part p's 8 KB
+    // (v-tiles 2 p, 2 p + 1) at its rows' place
+    const __amdgpu_buffer_rsrc_t src =
+        buf_rsrc(slotb + (static_cast<size_t>(sg.w) * kVHeads + h) * kHeadState, kHeadState * 4);
+    u32x4 fr[4];
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
+    for (int e = 0; e < 4; ++e) {
+      const int vt = w, d = e;   // wave w brings v-tile w's fragments
+      fr[e] = __builtin_amdgcn_raw_buffer_load_b128(
+          src, (vt >> 1) * (kFinRows * kDim * 4) + (((vt & 1) * 4 + d) * 64 + lane) * 16, 0, kSc01);
+    }
 #pragma unroll
-      for (int d = 0; d < 4; ++d) sm.frag[2 * w + e][d][lane] = fr[e][d];
+    for (int e = 0; e < 4; ++e) sm.frag[w][e][lane] = fr[e];
     __syncthreads();
-    for (int ci = first; ci < last; ++ci) {
-      if (ci > first) load_chunk(ci);
+    for (int ci = my; ci < last; ci += 2) {
+      if (ci > my) load_chunk(ci);
 #pragma unroll
-      for (int vt = 0; vt < 8; ++vt) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int p = 0; p < 4; ++p) {
+        f32x4 acc[2];
 #pragma unroll
-        for (int d = 0; d < 4; ++d) acc = mfma16(__builtin_bit_cast(bf16x8, sm.frag[vt][d][lane]), b[d], acc);
-        const u32x2 o = o0[vt];
-        const u32x2 o1 = {pack_bf2(bf_lo(o.x) + acc[0], bf_hi(o.x) + acc[1]),
-                          pack_bf2(bf_lo(o.y) + acc[2], bf_hi(o.y) + acc[3])};
-        __builtin_amdgcn_raw_buffer_store_b64(o1, orc, trow + 2 * (16 * vt + 4 * lg), 0, 0);
+        for (int e = 0; e < 2; ++e) {
+          acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            acc[e] = mfma16(__builtin_bit_cast(bf16x8, sm.frag[2 * p + e][d][lane]), b[d], acc[e]);
+        }
+        const u32x4 o = o0[p];
+        u32x4 o1;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+            o1[2 * e + x] = pack_bf2(bf_lo(o[2 * e + x]) + acc[e][2 * x], bf_hi(o[2 * e + x]) + acc[e][2 * x + 1]);
+        __builtin_amdgcn_raw_buffer_store_b128(o1, orc, trow + 2 * (32 * p + 8 * lg), 0, 0);
       }
     }
   }
@@ -3786,7 +3858,7 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
       max_runs(num_seqs, max_segments(total_tokens)) * 2 * kVHeads > 0x7fffffffLL)
     return GDN_ERR_INVALID_ARGUMENT;
   // as many segment slots as the workspace holds (the planner adapts to them)
-  const long long gcap = slots_fitting(num_seqs, total_tokens, workspace_bytes);
+  const long long gcap = std::min(slots_fitting(num_seqs, total_tokens, workspace_bytes), kMaxSlots);
   if (gcap < 0) return GDN_ERR_WORKSPACE_TOO_SMALL;
   const WsLayout L = ws_layout(num_seqs, total_tokens, gcap);
   if (!(scale > 0.0f) && !(scale < 0.0f)) scale = 0.08838834764831845f;
