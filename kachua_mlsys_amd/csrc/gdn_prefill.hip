@@ -110,6 +110,11 @@ constexpr int kMatElems = kMatFrags * kFragTile;   // one packed 64x64 matrix
 //   S_{j+1} = S_j M_j + B_j,          O_j = O0_j + OI_j S_j^T,
 // which a short scan over segments and a parallel correction pass resolve.
 constexpr int kMinSegChunks = 4;   // shortest M-run segment (the warm-up scheme may take 2 or 3)
+// Sequences of at most this many chunks take no M-runs (the planner's estimate
+// never favours them there: the finish alone costs about six chunk steps), so
+// a call of at most as many tokens needs no finish launch.  An empty finish
+// launch cost 2 to 3 us of a call's 20.
+constexpr int kMaxWholeChunks = 11;
 constexpr int kMSlotElems = 8 * 4 * 2 * 64 * 8;   // M_j^T as bf16 hi / lo MFMA fragments, per head
 
 // Upper bound on the segments of all multi-segment sequences: a sequence of
@@ -495,7 +500,7 @@ constexpr int kPlanScratch = kPsMisc + 4;
 template <int NT>
 __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, long long T, int R, int gcap,
                           const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-                          int* __restrict__ rec_start, int* __restrict__ lists, int* ps, int& total_recs, bool wide,
+                          int* __restrict__ rec_start, int* __restrict__ lists, int* ps, int& total_recs, bool wide, int skip,
                           long long t0_first = 0, long long t1_first = -1) {
   constexpr int kW = NT / 64;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -519,10 +524,12 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       seq_bounds(cu, is64, s, T, t0, t1);
     }
   };
+  // sequences of at most `skip` chunks (none when skip < 0) run elsewhere: -1
   auto chunks = [&](int s) {
     long long t0, t1;
     bounds(s, t0, t1);
-    return static_cast<int>((t1 - t0 + kChunk - 1) / kChunk);
+    const int nch = static_cast<int>((t1 - t0 + kChunk - 1) / kChunk);
+    return nch <= skip ? -1 : nch;
   };
 
   // ---- pass 1: statistics per candidate segment length ----
@@ -656,7 +663,8 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     const int q = static_cast<int>(fminf(est * 16.f, 1.0e7f));
     // segments below kMinSegChunks only without M-runs (the workspace's slots
     // are sized for M-run segments of at least kMinSegChunks)
-    const bool allowed = lane < kSegCands && slots <= gcap && (warm || Lc >= kMinSegChunks);
+    const bool allowed = lane < kSegCands && slots <= gcap &&
+                         (warm || (Lc >= kMinSegChunks && (nseg_max <= 1 || ml > kMaxWholeChunks)));
     const int key = allowed ? q * 64 + (63 - lane) : 0x7fffffff;
     // minimum over the lanes: the maximum of the complements
     const int best = 0x7fffffff - wave_max0(0x7fffffff - key);
@@ -674,6 +682,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
   int v[5] = {0, 0, 0, 0, 0};
   for (int s = s_begin; s < s_end; ++s) {
     const int nch = chunks(s);
+    if (nch < 0) continue;
     const SeqPlan p = seq_plan(nch, L, warm);
     v[0] += nch;
     v[1] += p.is_long ? 0 : 1;
@@ -724,10 +733,11 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
   for (int s = s_begin; s < s_end; ++s) {
     long long t0, t1;
     bounds(s, t0, t1);
-    const int nch = static_cast<int>((t1 - t0 + kChunk - 1) / kChunk);
-    const SeqPlan p = seq_plan(nch, L, warm);
+    const int nch = chunks(s);
     const int rec0 = rb;
     rec_start[s] = rb;
+    if (nch < 0) continue;
+    const SeqPlan p = seq_plan(nch, L, warm);
     rb += nch;
     if (!p.is_long) {
       // chunks whose records exist (overlapping cu_seqlens can exhaust the capacity)
@@ -793,7 +803,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   const int s_end = min(num_seqs, s_begin + per);
   int total_recs;
   int base = plan_batch<kPlanThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, ps,
-                                      total_recs, wide != 0);
+                                      total_recs, wide != 0, -1);
   for (int s = s_begin; s < s_end; ++s) {
     long long t0, t1;
     seq_bounds(cu, is64, s, T, t0, t1);
@@ -853,6 +863,15 @@ __device__ __forceinline__ u32x2 lds_tr16(const uint16_t* p) {
   return __builtin_bit_cast(u32x2, v);
 }
 
+// The lane index through an opaque move: keeps the compiler from computing the
+// lane-dependent addresses of every phase once, outside the chunk and item
+// loops, and spilling them.
+__device__ __forceinline__ int opaque_lane(int lane) {
+  int l;
+  asm volatile("v_and_b32 %0, 63, %1" : "=v"(l) : "v"(lane));
+  return l;
+}
+
 // Work-group barrier that waits for this wave's LDS operations only; its
 // global-to-LDS copies stay in flight.
 __device__ __forceinline__ void lds_barrier() {
@@ -886,13 +905,15 @@ constexpr int kPrepassThreads = 256;              // four independent waves
 constexpr int kPrepassWaves = kPrepassThreads / 64;
 constexpr int kPrepassMaxGroups = 512;             // two per CU: eight waves, two per SIMD
 
+// Diagonal blocks N_aa of one v-head, column-major (nt[a][column][row]); the
+// forward substitution then overwrites each with its inverse T_aa (a wave reads
+// all of its N columns before its first T store).
+typedef float PrepassNt[4][16][16];
+
+template <int kHeads>
 struct __align__(16) PrepassWaveSmem {   // per v-head of the item
-  float lgam[kGva][kChunk];    // Gam_t / ln 2 (inclusive scan of log2 g)
-  float beta[kGva][kChunk];
-  // diagonal blocks N_aa, column-major (nt[a][column][row]); the forward
-  // substitution then overwrites each with its inverse T_aa (a wave reads all of
-  // its N columns before its first T store)
-  float nt[kGva][4][16][16];
+  float lgam[kHeads][kChunk];    // Gam_t / ln 2 (inclusive scan of log2 g)
+  float beta[kHeads][kChunk];
 };
 
 // Batches of at most kFusedPlanSeqs sequences number their records inside the
@@ -908,9 +929,13 @@ struct PrepassSeqSmem {
   long long s1[kFusedPlanSeqs];
 };
 
+template <int kWaves>
 struct PrepassSmem {
   union {
-    PrepassWaveSmem w[kPrepassWaves];
+    struct {
+      PrepassWaveSmem<kGva> g;
+      PrepassNt nt[kGva];
+    } w[kWaves];
     int plan[kPlanScratch];      // planner scratch (work-group 0 of a fused launch)
   } u;
   PrepassSeqSmem seq;
@@ -983,8 +1008,8 @@ __device__ __forceinline__ void store_frag(const u32x4& x, uint16_t* dst) {
 // to fp32 working precision, and a finite floor keeps Gam finite), beta_t;
 // gam / tail / Gam to the gate blocks, Gam and beta to ws rows 0 .. NH - 1,
 // Gam at the chunk's last token to last[].
-template <int NH, bool kToLds = false>
-__device__ __forceinline__ void prepass_gates(PrepassWaveSmem& ws, int c, const float (&a_t)[kGva],
+template <int NH, class Ws>
+__device__ __forceinline__ void prepass_gates(Ws& ws, int c, const float (&a_t)[kGva],
                                               const float (&b_t)[kGva], const float (&alog)[kGva],
                                               const float (&dtb)[kGva], float* __restrict__ gp0,
                                               float (&last)[NH]) {
@@ -1012,8 +1037,8 @@ __device__ __forceinline__ void prepass_gates(PrepassWaveSmem& ws, int c, const 
 
 // The rest of the terms of NH v-heads, whose gates prepass_gates left in ws
 // rows E0 .. E0 + NH - 1 (and last[]), from the chunk's raw gram.
-template <int NH, int E0 = 0, bool kToLds = false, int NB = 4>
-__device__ __forceinline__ void prepass_terms(PrepassWaveSmem& ws, const f32x4 (&kk)[4][4], int c,
+template <int NH, int E0 = 0, bool kToLds = false, int NB = 4, class Ws>
+__device__ __forceinline__ void prepass_terms(Ws& ws, PrepassNt* nts, const f32x4 (&kk)[4][4], int c,
                                               const float (&last)[NH], uint16_t* __restrict__ frag0,
                                               float* __restrict__ gp0) {
   const int lane = threadIdx.x & 63;
@@ -1056,7 +1081,7 @@ __device__ __forceinline__ void prepass_terms(PrepassWaveSmem& ws, const f32x4 (
 #pragma unroll
           for (int rr = 0; rr < 4; ++rr)
             if (m < NB && l16 == 4 * lg + rr) kb[e] += __log2f(fmaxf(1.0f, fabsf(1.0f - brow[e][m][rr] * kk[m][m][rr])));
-          *reinterpret_cast<f32x4*>(&ws.nt[E0 + e][m][l16][4 * lg]) = nv;
+          *reinterpret_cast<f32x4*>(&nts[E0 + e][m][l16][4 * lg]) = nv;
         } else {
           nlo[e][m][n] = nv;
         }
@@ -1084,7 +1109,7 @@ __device__ __forceinline__ void prepass_terms(PrepassWaveSmem& ws, const f32x4 (
     f32x4 ring[kAhead][4];
     auto read_col = [&](int i, f32x4 (&c)[4]) {
 #pragma unroll
-      for (int qv = (i + 1) >> 2; qv < 4; ++qv) c[qv] = *reinterpret_cast<const f32x4*>(&ws.nt[E0 + e][lg][i][4 * qv]);
+      for (int qv = (i + 1) >> 2; qv < 4; ++qv) c[qv] = *reinterpret_cast<const f32x4*>(&nts[E0 + e][lg][i][4 * qv]);
     };
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) read_col(i, ring[i]);
@@ -1099,7 +1124,7 @@ __device__ __forceinline__ void prepass_terms(PrepassWaveSmem& ws, const f32x4 (
     }
 #pragma unroll
     for (int qv = 0; qv < 4; ++qv)
-      *reinterpret_cast<f32x4*>(&ws.nt[E0 + e][lg][l16][4 * qv]) = f32x4{x[4 * qv], x[4 * qv + 1], x[4 * qv + 2], x[4 * qv + 3]};
+      *reinterpret_cast<f32x4*>(&nts[E0 + e][lg][l16][4 * qv]) = f32x4{x[4 * qv], x[4 * qv + 1], x[4 * qv + 2], x[4 * qv + 3]};
   }
   wave_lds_sync();
 
@@ -1112,9 +1137,9 @@ __device__ __forceinline__ void prepass_terms(PrepassWaveSmem& ws, const f32x4 (
     f32x4 tc[4], w[4][4];   // tc[a] = T_aa = (W_aa)^T in C layout; w[a][b] = W_ab, a <= b
 #pragma unroll
     for (int ab = 0; ab < 4; ++ab) {
-      tc[ab] = *reinterpret_cast<const f32x4*>(&ws.nt[E0 + e][ab][l16][4 * lg]);
+      tc[ab] = *reinterpret_cast<const f32x4*>(&nts[E0 + e][ab][l16][4 * lg]);
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) w[ab][ab][rr] = ws.nt[E0 + e][ab][4 * lg + rr][l16];
+      for (int rr = 0; rr < 4; ++rr) w[ab][ab][rr] = nts[E0 + e][ab][4 * lg + rr][l16];
     }
     const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
     // operands split once: tx[a] from T_aa, nx[m][a] from N_ma = U_am^T,
@@ -1225,7 +1250,7 @@ __device__ __forceinline__ void chunk_gram_loads(const uint16_t* __restrict__ k,
 // and the item count is a multiple of 8 (8 per record), so either all four
 // have an item or none has, and a wave that has ended no longer counts at a
 // barrier.
-static_assert(sizeof(PrepassWaveSmem::nt) >= 8 * 64 * sizeof(u32x4), "the exchange area holds eight fragments");
+static_assert(kGva * sizeof(PrepassNt) >= 8 * 64 * sizeof(u32x4), "the exchange area holds eight fragments");
 __device__ __forceinline__ void trade_gram_halves(u32x4* mine, const u32x4* partner, int lane,
                                                   bf16x8 (&kf)[4][4]) {
 #pragma unroll
@@ -1252,31 +1277,23 @@ __device__ __forceinline__ void chunk_gram_products(const bf16x8 (&kf)[4][4], f3
       for (int n = 0; n <= m; ++n) kk[m][n] = mfma16(kf[dd][m], kf[dd][n], kk[m][n]);
 }
 
-// kGroups: work-groups per CU the register budget is sized for (2, or 3 for
-// one-v-head items in batches of 2048-3072 of them).
-template <bool kPair, int kGroups>
-__global__ __launch_bounds__(kPrepassThreads, kGroups) void prepass_kernel(
+// The items of work-group `group` of `ngroups` (kWaves waves each).  Sequences of
+// at most `skip` chunks have no records (none is skipped when skip < 0).
+template <bool kPair, int kWaves>
+__device__ __forceinline__ void prepass_items(
+    PrepassSmem<kWaves>& sm, int group, int ngroups,
     const uint16_t* __restrict__ k, const float* __restrict__ A_log, const uint16_t* __restrict__ a,
-    const float* __restrict__ dt_bias, const uint16_t* __restrict__ b,
-    const int4* __restrict__ recs, const void* __restrict__ cu, int is64, int num_seqs, long long T, int R,
-    int gcap, int fused_plan, int* __restrict__ rec_start, int* __restrict__ lists,
-    uint16_t* __restrict__ ws_frag, float* __restrict__ ws_gam, int wide) {
-  __shared__ PrepassSmem sm;
-  if (fused_plan && blockIdx.x == 0) {
-    // work-group 0 plans the batch (lists for the consumer) while the others
-    // run the records
-    int total_recs;
-    plan_batch<kPrepassThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, sm.u.plan,
-                                total_recs, wide != 0);
-    return;
-  }
+    const float* __restrict__ dt_bias, const uint16_t* __restrict__ b, const int4* __restrict__ recs,
+    const void* __restrict__ cu, int is64, int num_seqs, long long T, int R, int fused_plan, int skip,
+    const int* __restrict__ rec_start, uint16_t* __restrict__ ws_frag, float* __restrict__ ws_gam) {
   const int lane = threadIdx.x & 63;
   // the per-head constants, requested first: lane l holds v-head l & 7's
   const float alog_l = A_log[lane & 7], dtb_l = dt_bias[lane & 7];
   const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  PrepassWaveSmem& ws = sm.u.w[wv];
-  const int gw = (static_cast<int>(blockIdx.x) - fused_plan) * kPrepassWaves + wv;
-  const int nw = (static_cast<int>(gridDim.x) - fused_plan) * kPrepassWaves;
+  PrepassWaveSmem<kGva>& ws = sm.u.w[wv].g;
+  PrepassNt* nts = sm.u.w[wv].nt;
+  const int gw = group * kWaves + wv;
+  const int nw = ngroups * kWaves;
 
   // records: small batches scan the chunk counts here (wave 0; lane l of block
   // j owns sequence 64 j + l), into LDS
@@ -1316,7 +1333,8 @@ __global__ __launch_bounds__(kPrepassThreads, kGroups) void prepass_kernel(
           if (s >= num_seqs) t0 = t1 = 0;
           b0[j] = t0;
           b1[j] = t1;
-          const int nch = static_cast<int>((b1[j] - b0[j] + kChunk - 1) / kChunk);
+          int nch = static_cast<int>((b1[j] - b0[j] + kChunk - 1) / kChunk);
+          nch = nch <= skip ? 0 : nch;   // run elsewhere
           const int inc = wave_incl_sum(nch) + carry;
           sm.seq.incl[s] = inc;
           sm.seq.s0[s] = b0[j];
@@ -1401,18 +1419,41 @@ __global__ __launch_bounds__(kPrepassThreads, kGroups) void prepass_kernel(
       // the v-heads of the pair one after the other (interleaving their
       // phases gains nothing: the phases are VALU-bound, not latency-bound)
       const float l0[1] = {last[0]}, l1[1] = {last[1]};
-      prepass_terms<1, 0>(ws, kk, c, l0, frag0, gp0);
-      prepass_terms<1, 1>(ws, kk, c, l1, frag0 + kMatElems, gp0 + kGamStride);
+      prepass_terms<1, 0>(ws, nts, kk, c, l0, frag0, gp0);
+      prepass_terms<1, 1>(ws, nts, kk, c, l1, frag0 + kMatElems, gp0 + kGamStride);
     } else {
       float last[1];
       prepass_gates<1>(ws, c, a_t, b_t, alog, dtb, gp0, last);
-      auto* mine = reinterpret_cast<u32x4*>(&ws.nt[0][0][0][0]);
-      const auto* partner = reinterpret_cast<const u32x4*>(&sm.u.w[wv ^ 1].nt[0][0][0][0]);
+      auto* mine = reinterpret_cast<u32x4*>(nts);
+      const auto* partner = reinterpret_cast<const u32x4*>(sm.u.w[wv ^ 1].nt);
       trade_gram_halves(mine, partner, lane, kf);
       chunk_gram_products(kf, kk);
-      prepass_terms<1, 0>(ws, kk, c, last, frag0, gp0);
+      prepass_terms<1, 0>(ws, nts, kk, c, last, frag0, gp0);
     }
   }
+}
+
+// kGroups: work-groups per CU the register budget is sized for (2, or 3 for
+// one-v-head items in batches of 2048-3072 of them).
+template <bool kPair, int kGroups>
+__global__ __launch_bounds__(kPrepassThreads, kGroups) void prepass_kernel(
+    const uint16_t* __restrict__ k, const float* __restrict__ A_log, const uint16_t* __restrict__ a,
+    const float* __restrict__ dt_bias, const uint16_t* __restrict__ b,
+    const int4* __restrict__ recs, const void* __restrict__ cu, int is64, int num_seqs, long long T, int R,
+    int gcap, int fused_plan, int* __restrict__ rec_start, int* __restrict__ lists,
+    uint16_t* __restrict__ ws_frag, float* __restrict__ ws_gam, int wide) {
+  __shared__ PrepassSmem<kPrepassWaves> sm;
+  if (fused_plan && blockIdx.x == 0) {
+    // work-group 0 plans the batch (lists for the consumer) while the others
+    // run the records
+    int total_recs;
+    plan_batch<kPrepassThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, sm.u.plan,
+                                total_recs, wide != 0, -1);
+    return;
+  }
+  prepass_items<kPair, kPrepassWaves>(sm, static_cast<int>(blockIdx.x) - fused_plan,
+                                      static_cast<int>(gridDim.x) - fused_plan, k, A_log, a, dt_bias, b, recs, cu,
+                                      is64, num_seqs, T, R, fused_plan, -1, rec_start, ws_frag, ws_gam);
 }
 
 // ============================================================================
@@ -1439,6 +1480,16 @@ struct __align__(16) ConsumerSmem {
   uint16_t vs[2][kChunk][kDim];
   uint16_t frag[2][kFrags][kMatElems];
   float gt[2][4 * kChunk];
+};
+
+// Where one chunk's operands sit in LDS (full-head consumer and direct path).
+struct ChunkLds {
+  const uint16_t (*ks)[kDim];
+  const uint16_t (*qs)[kDim];
+  const uint16_t (*vs)[kDim];
+  const uint16_t* tb;    // Tb fragments
+  uint16_t* aqk;         // Aqk fragments, formed by the waves
+  const float* gt;       // gate block
 };
 
 __device__ __forceinline__ int v_swz(int t) { return (t & 3) << 2; }
@@ -1583,8 +1634,8 @@ static_assert(fh_aqk_covers(), "full-head Aqk tiles");
 
 // Tiles of Q row blocks at or past the chunk length c feed only output rows
 // that are never stored: they are skipped (m1 > m0, so m0's test covers both).
-template <int W, int P>
-__device__ __forceinline__ void fh_aqk(ConsumerSmem& sm, int lane, int c) {
+template <int W>
+__device__ __forceinline__ void fh_aqk(const ChunkLds& sm, int lane, int c) {
   constexpr int a = fh_aqk_a(W), m0 = fh_aqk_m0(W), m1 = fh_aqk_m1(W);
   static_assert(m1 < 0 || m1 > m0, "tile order");
   if constexpr (a >= 0) {
@@ -1595,13 +1646,13 @@ __device__ __forceinline__ void fh_aqk(ConsumerSmem& sm, int lane, int c) {
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const int at = 8 * ((4 * d + lg) ^ rsw);
-      kb[d] = *reinterpret_cast<const bf16x8*>(&sm.ks[P][16 * a + l16][at]);
-      q0[d] = *reinterpret_cast<const bf16x8*>(&sm.qs[P][16 * m0 + l16][at]);
-      if constexpr (m1 >= 0) q1[d] = *reinterpret_cast<const bf16x8*>(&sm.qs[P][16 * m1 + l16][at]);
+      kb[d] = *reinterpret_cast<const bf16x8*>(&sm.ks[16 * a + l16][at]);
+      q0[d] = *reinterpret_cast<const bf16x8*>(&sm.qs[16 * m0 + l16][at]);
+      if constexpr (m1 >= 0) q1[d] = *reinterpret_cast<const bf16x8*>(&sm.qs[16 * m1 + l16][at]);
     }
-    const f32x4 gi = *reinterpret_cast<const f32x4*>(&sm.gt[P][kLgamAt + 16 * a + 4 * lg]);
-    const float g0 = sm.gt[P][kLgamAt + 16 * m0 + l16];
-    const float g1 = sm.gt[P][kLgamAt + 16 * (m1 >= 0 ? m1 : m0) + l16];
+    const f32x4 gi = *reinterpret_cast<const f32x4*>(&sm.gt[kLgamAt + 16 * a + 4 * lg]);
+    const float g0 = sm.gt[kLgamAt + 16 * m0 + l16];
+    const float g1 = sm.gt[kLgamAt + 16 * (m1 >= 0 ? m1 : m0) + l16];
     __builtin_amdgcn_sched_barrier(0);
     f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1609,9 +1660,9 @@ __device__ __forceinline__ void fh_aqk(ConsumerSmem& sm, int lane, int c) {
       acc0 = mfma16(kb[d], q0[d], acc0);
       if constexpr (m1 >= 0) acc1 = mfma16(kb[d], q1[d], acc1);
     }
-    put_aqk_tile(&sm.frag[P][1][0], a, m0, lane, acc0, g0, gi);
+    put_aqk_tile(sm.aqk, a, m0, lane, acc0, g0, gi);
     if constexpr (m1 >= 0)
-      if (16 * m1 < c) put_aqk_tile(&sm.frag[P][1][0], a, m1, lane, acc1, g1, gi);
+      if (16 * m1 < c) put_aqk_tile(sm.aqk, a, m1, lane, acc1, g1, gi);
   }
 }
 
@@ -1641,8 +1692,8 @@ __device__ __forceinline__ void chunk_by_tiles(int c, F&& f) {
 //         (zero columns of Tb, zero rows of Delta); their products are not
 //         formed (their R rows count as zero, also for R's range scale), and
 //         the state update skips the second 32-token depth half when NB <= 2.
-template <int P, int NB>
-__device__ __forceinline__ void consumer_chunk(ConsumerSmem& sm, int c, f32x4 (&st)[8], int w,
+template <int NB>
+__device__ __forceinline__ void consumer_chunk(const ChunkLds& sm, int c, f32x4 (&st)[8], int w,
                                                int lane, float scale, __amdgpu_buffer_rsrc_t orc,
                                                uint32_t ocol) {
   static_assert(NB >= 1 && NB <= 4, "token tiles");
@@ -1651,19 +1702,19 @@ __device__ __forceinline__ void consumer_chunk(ConsumerSmem& sm, int c, f32x4 (&
   // ---- this wave's Aqk tiles, first (fewest registers live); every wave
   // reads them after the barrier before O^T ----
   switch (w) {   // uniform
-    case 0: fh_aqk<0, P>(sm, lane, c); break;
-    case 1: fh_aqk<1, P>(sm, lane, c); break;
-    case 2: fh_aqk<2, P>(sm, lane, c); break;
-    case 3: fh_aqk<3, P>(sm, lane, c); break;
-    case 4: fh_aqk<4, P>(sm, lane, c); break;
-    case 5: fh_aqk<5, P>(sm, lane, c); break;
-    case 6: fh_aqk<6, P>(sm, lane, c); break;
+    case 0: fh_aqk<0>(sm, lane, c); break;
+    case 1: fh_aqk<1>(sm, lane, c); break;
+    case 2: fh_aqk<2>(sm, lane, c); break;
+    case 3: fh_aqk<3>(sm, lane, c); break;
+    case 4: fh_aqk<4>(sm, lane, c); break;
+    case 5: fh_aqk<5>(sm, lane, c); break;
+    case 6: fh_aqk<6>(sm, lane, c); break;
     default: break;
   }
   f32x4 gam[4];
 #pragma unroll
-  for (int m = 0; m < 4; ++m) gam[m] = *reinterpret_cast<const f32x4*>(&sm.gt[P][16 * m + 4 * lg]);
-  const float gam_c = sm.gt[P][c - 1];
+  for (int m = 0; m < 4; ++m) gam[m] = *reinterpret_cast<const f32x4*>(&sm.gt[16 * m + 4 * lg]);
+  const float gam_c = sm.gt[c - 1];
 
   // ---- X = K S^T (rows t), Y^T = S Q^T (rows v); S as single bf16 ----
   bf16x8 sb[4];
@@ -1684,10 +1735,24 @@ __device__ __forceinline__ void consumer_chunk(ConsumerSmem& sm, int c, f32x4 (&
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const int at = 8 * ((4 * d + lg) ^ rsw);
-      const bf16x8 ka = *reinterpret_cast<const bf16x8*>(&sm.ks[P][16 * m + l16][at]);
-      const bf16x8 qa = *reinterpret_cast<const bf16x8*>(&sm.qs[P][16 * m + l16][at]);
+      const bf16x8 ka = *reinterpret_cast<const bf16x8*>(&sm.ks[16 * m + l16][at]);
+      const bf16x8 qa = *reinterpret_cast<const bf16x8*>(&sm.qs[16 * m + l16][at]);
       X[m] = mfma16(ka, sb[d], X[m]);
       YT[m] = mfma16(sb[d], qa, YT[m]);
+    }
+  }
+
+  if (sm.gt[kBoundAt] > kHiLoBoundLog2) {   // uniform: slow decay (see chain_chunk)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      float x[8];
+      bf16x8 hi, lo;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) x[s] = st[2 * d + (s >> 2)][s & 3];
+      split_frag(x, hi, lo);
+#pragma unroll
+      for (int m = 0; m < NB; ++m)
+        X[m] = mfma16(*reinterpret_cast<const bf16x8*>(&sm.ks[16 * m + l16][8 * ((4 * d + lg) ^ rsw)]), lo, X[m]);
     }
   }
 
@@ -1700,7 +1765,7 @@ __device__ __forceinline__ void consumer_chunk(ConsumerSmem& sm, int c, f32x4 (&
   for (int m = 0; m < 4; ++m) {
     Rt[m] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (m >= NB) continue;
-    const u32x2 vw = lds_tr16(&sm.vs[P][16 * m + vrow][vat]);
+    const u32x2 vw = lds_tr16(&sm.vs[16 * m + vrow][vat]);
     const float vv[4] = {bf_lo(vw.x), bf_hi(vw.x), bf_lo(vw.y), bf_hi(vw.y)};
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) Rt[m][rr] = vv[rr] - gam[m][rr] * X[m][rr];
@@ -1725,9 +1790,9 @@ __device__ __forceinline__ void consumer_chunk(ConsumerSmem& sm, int c, f32x4 (&
 #pragma unroll
     for (int d = 0; d < ND; ++d)
       if (!frag_zero(m, d))
-        D[m] = mfma16h(*reinterpret_cast<const f16x8*>(&sm.frag[P][0][(frag_slot(m, d) * 64 + lane) * 8]), rf[d], D[m]);
+        D[m] = mfma16h(*reinterpret_cast<const f16x8*>(&sm.tb[(frag_slot(m, d) * 64 + lane) * 8]), rf[d], D[m]);
   }
-  const float tbi = sm.gt[P][kTbScaleAt];   // 1 / Tb's fp16 range scale (1 in the usual range)
+  const float tbi = sm.gt[kTbScaleAt];   // 1 / Tb's fp16 range scale (1 in the usual range)
   if (rsc != 1.0f || tbi != 1.0f) {
     const float inv = tbi / rsc;   // exact: powers of two
 #pragma unroll
@@ -1740,7 +1805,7 @@ __device__ __forceinline__ void consumer_chunk(ConsumerSmem& sm, int c, f32x4 (&
     f32x4 Dt[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m)
-      Dt[m] = m < NB ? D[m] * *reinterpret_cast<const f32x4*>(&sm.gt[P][kChunk + 16 * m + 4 * lg]) : D[m];
+      Dt[m] = m < NB ? D[m] * *reinterpret_cast<const f32x4*>(&sm.gt[kChunk + 16 * m + 4 * lg]) : D[m];
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
       float x[8];
@@ -1760,9 +1825,9 @@ __device__ __forceinline__ void consumer_chunk(ConsumerSmem& sm, int c, f32x4 (&
 #pragma unroll
     for (int d = 0; d < ND; ++d)
       if (!frag_zero(m, d))
-        OT = mfma16(dob[d], *reinterpret_cast<const bf16x8*>(&sm.frag[P][1][(frag_slot(m, d) * 64 + lane) * 8]), OT);
+        OT = mfma16(dob[d], *reinterpret_cast<const bf16x8*>(&sm.aqk[(frag_slot(m, d) * 64 + lane) * 8]), OT);
     const int t = 16 * m + l16;
-    const float sg = scale * sm.gt[P][t];
+    const float sg = scale * sm.gt[t];
     const u32x2 pk = {pack_bf2(sg * YT[m][0] + scale * OT[0], sg * YT[m][1] + scale * OT[1]),
                       pack_bf2(sg * YT[m][2] + scale * OT[2], sg * YT[m][3] + scale * OT[3])};
     __builtin_amdgcn_raw_buffer_store_b64(pk, orc, static_cast<uint32_t>(t) * (kVHeads * kDim * 2) + ocol, 0, 0);
@@ -1781,8 +1846,8 @@ __device__ __forceinline__ void consumer_chunk(ConsumerSmem& sm, int c, f32x4 (&
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
       const int ta = perm_depth(d, lg, sl >> 2);
-      const u32x2 a0 = lds_tr16(&sm.ks[P][ta][at]);
-      const u32x2 a1 = lds_tr16(&sm.ks[P][ta + 16][at]);
+      const u32x2 a0 = lds_tr16(&sm.ks[ta][at]);
+      const u32x2 a1 = lds_tr16(&sm.ks[ta + 16][at]);
       const bf16x8 kta = join_frag(a0, a1);
       acc = mfma16(kta, dh[d], acc);
       acc = mfma16(kta, dl[d], acc);
@@ -1903,9 +1968,10 @@ __device__ __forceinline__ void full_head_items(
     if (cur.rec >= 0 && cur.c > 0) {
       const __amdgpu_buffer_rsrc_t orc = __builtin_amdgcn_make_buffer_rsrc(
           out + (static_cast<size_t>(cur.c0) * kVHeads + cur.h) * kDim, 0, cur.c * (kVHeads * kDim * 2), 0x00020000);
+      const ChunkLds lds = {sm.ks[P], sm.qs[P], sm.vs[P], sm.frag[P][0], sm.frag[P][1], sm.gt[P]};
       // all four tiles: batches of many short sequences are bound by their
       // state traffic, and one body keeps the loop's code small
-      consumer_chunk<P, 4>(sm, cur.c, st, w, lane, scale, orc, ocol);
+      consumer_chunk<4>(lds, cur.c, st, w, lane, scale, orc, ocol);
     }
     // an empty sequence leaves new_state zero (st is zero); a chunk without a
     // record (malformed cu_seqlens) passes the state through.  State bytes are
@@ -1925,23 +1991,231 @@ __device__ __forceinline__ void full_head_items(
   }
 }
 
-// ============================================================================
-// direct path: calls of at most two chunks in total (T <= 128)
-// ============================================================================
-// Every sequence then has at most two chunks and the call is latency-bound, so
-// it runs as one launch with no plan and no workspace: one work-group per
-// (sequence, v-head).  All waves issue their share of the chunks' K / Q / V
-// copies (chunk j into buffer j) and load their state tile; wave j then forms
-// chunk j's terms (the prepass of one item, written to LDS instead of the
-// workspace) while those land, and the eight waves run the chunks one after
-// the other as the full-head consumer does, the state staying in registers.
-constexpr int kDirectMaxSeqs = 64;
-constexpr int kDirectMaxChunks = 2;
+// Barrier of the split consumer: every wave's LDS writes are visible, and each
+// side wave has at most kPending vector memory operations outstanding.  The
+// chain waves issue no vector memory operation a later phase depends on: their
+// state loads are waited for where the state is first used, and their
+// final-state stores need not have completed for the next item to start.
+// At the chunk's end (B3), kPending = kSideStores: a side wave issues its
+// copies at the chunk's start and its kSideStores output stores at the end,
+// and vector memory operations complete in issue order, so every copy has
+// landed while the output stores stay in flight into the next chunk.
+template <int kPending>
+__device__ __forceinline__ void split_barrier(bool chain) {
+  static_assert(kPending >= 0 && kPending < 16, "vmcnt field");
+  asm volatile("" ::: "memory");
+  if (chain)
+    __builtin_amdgcn_s_waitcnt(0xc07f);             // lgkmcnt(0)
+  else
+    __builtin_amdgcn_s_waitcnt(0x0070 | kPending);  // vmcnt(kPending), lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 
-struct DirectSmem {
-  ConsumerSmem c;                         // chunk j's operands in buffer j
-  PrepassWaveSmem w[kDirectMaxChunks];    // scratch of the terms waves
+// ============================================================================
+// direct path: small calls
+// ============================================================================
+// Latency-bound calls run as one launch with no plan and no workspace: one
+// work-group per (sequence, v-head).  Wave j forms chunk j's terms (the prepass
+// of one item, written to LDS instead of the workspace) while chunk 0's K / Q /
+// V copies and the state land, up to kDirectTerms chunks at once; the eight
+// waves then run the chunks one after the other as the full-head consumer does,
+// the state staying in registers and the next chunk's copies landing in the
+// other buffer.  The state moves as 8 rows x 128 contiguous bytes per
+// instruction and changes to the C layout through 2 KB of LDS per wave (see
+// load_state_rows for what the direct access pattern costs); its loads need
+// only the sequence index and are requested before the sequence's bounds.
+constexpr int kDirectTerms = 7;
+constexpr int kDirectMaxSeqs = 64;
+constexpr int kDirectMaxTokens = 4 * kChunk;
+
+struct __align__(16) DirectSmem {
+  uint16_t ks[2][kChunk][kDim];
+  uint16_t qs[2][kChunk][kDim];
+  uint16_t vs[2][kChunk][kDim];
+  // chunk j's Tb in tb[j + 1]; its Aqk in tb[j], where the previous chunk's Tb
+  // is dead (every wave has read it before the barrier that chunk's Aqk needs)
+  uint16_t tb[kDirectTerms + 1][kMatElems];
+  float gt[kDirectTerms][4 * kChunk];
+  PrepassWaveSmem<1> w[kDirectTerms];    // scratch of the terms waves
 };
+// the terms' N blocks use K and V of buffer 1, the state's layout change Q of
+// a buffer that holds no live rows
+static_assert(kDirectTerms * sizeof(PrepassNt) <= 2 * kChunk * kDim * sizeof(uint16_t), "N blocks");
+static_assert(sizeof(DirectSmem) <= 160 * 1024, "one group per CU");
+
+// Calls of at most four chunks run on direct_kernel alone.  Measured against
+// the planned path: 4 sequences of 50 tokens 18.5 -> 13.3 us, one of 200 21.3
+// -> 21.0, one of 256 even (3.3 us per further chunk).
+// Larger calls of few, mostly short sequences take the direct path for the
+// sequences of at most kMixedChunks chunks, in the launch that plans and
+// prepasses the longer ones (mixed_kernel), which then run as ever: 8 sequences
+// of 50 tokens 20.9 -> 16.8 us, 24 of 60 30.8 -> 19.3, 32 of 60 35.1 -> 23.0;
+// one sequence of 500 or 1,889 tokens among tiny ones costs what it did (25,
+// 33 us).  Longer sequences gain from the split consumer's segments instead
+// (24 of 120 tokens: 34.0 planned, 37.4 mixed; 16 of 400: 38.8, 51.0).
+constexpr int kMixedChunks = 4;
+constexpr int kMixedMaxSeqs = kConsumerGroups / kVHeads;   // a CU for each (sequence, v-head)
+inline bool direct_batch(int num_seqs, long long tokens) {
+  return num_seqs <= kDirectMaxSeqs && tokens <= kDirectMaxTokens;
+}
+inline bool mixed_batch(int num_seqs, long long tokens) {
+  return num_seqs <= kMixedMaxSeqs && tokens <= 1ll * kChunk * num_seqs;
+}
+
+// One (sequence s, v-head h); nothing when the sequence has more than max_chunks
+// chunks (it runs elsewhere).
+__device__ __forceinline__ void direct_group(
+    DirectSmem& sm, int s, int h, int max_chunks, const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const float* __restrict__ state, const float* __restrict__ A_log, const uint16_t* __restrict__ a,
+    const float* __restrict__ dt_bias, const uint16_t* __restrict__ b, const void* __restrict__ cu, int is64,
+    long long T, float scale, uint16_t* __restrict__ out, float* __restrict__ new_state) {
+  const int hq = h / kGva;
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int vcol = 16 * w;
+  // the wave's 16 state rows: piece j = 2 q + i holds rows 8 i + lane / 8,
+  // columns 32 q + 4 (lane & 7)
+  auto soff_of = [&](int lane) {
+    return ((static_cast<size_t>(s) * kVHeads + h) * kDim + vcol + (lane >> 3)) * kDim + 4 * (lane & 7);
+  };
+  const size_t soff = soff_of(lane);
+  auto piece = [](int j) { return 8 * (j & 1) * kDim + 32 * (j >> 1); };
+  f32x4 rows[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) rows[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (state != nullptr) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      rows[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(state + soff + piece(j)));
+  }
+  long long t0, t1;
+  seq_bounds(cu, is64, s, T, t0, t1);
+  const int len = static_cast<int>(t1 - t0);   // 0 .. T
+  const int nch = (len + kChunk - 1) / kChunk;
+  if (nch > max_chunks) return;
+  if (len <= 0) {   // an empty sequence: zero state, no output rows
+    float* dst = new_state + soff;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      __builtin_nontemporal_store(f32x4{0.f, 0.f, 0.f, 0.f}, reinterpret_cast<f32x4*>(dst + piece(j)));
+    return;
+  }
+  // chunk j: first token t0 + 64 j, chunk_len(j) tokens
+  auto chunk_len = [&](int j) { return min(kChunk, len - kChunk * j); };
+  // chunk j's K / Q / V rows into buffer P (rows past its end repeat its last row)
+  auto copy = [&](int j, int P) __attribute__((always_inline)) {
+    const int lane = opaque_lane(tid);
+    const int r = 4 * w + (lane >> 4);
+    const uint32_t kq_col = 16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(r));
+    const uint32_t v_col = 16u * static_cast<uint32_t>((lane & 15) ^ v_swz(r));
+    const long long c0 = t0 + static_cast<long long>(kChunk) * j;
+    const size_t qk0 = (static_cast<size_t>(c0) * kQKHeads + hq) * kDim;
+    const char* kb = reinterpret_cast<const char*>(k + qk0);
+    const char* qb = reinterpret_cast<const char*>(q + qk0);
+    const char* vb = reinterpret_cast<const char*>(v + (static_cast<size_t>(c0) * kVHeads + h) * kDim);
+    const int last = chunk_len(j) - 1;
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      const uint32_t row = static_cast<uint32_t>(min(r + 32 * jj, last));
+      const uint32_t off = row * (kQKHeads * kDim * 2) + kq_col;
+      dma16(kb + off, &sm.ks[P][32 * jj + 4 * w][0]);
+      dma16(qb + off, &sm.qs[P][32 * jj + 4 * w][0]);
+      dma16<2>(vb + row * (kVHeads * kDim * 2) + v_col, &sm.vs[P][32 * jj + 4 * w][0]);
+    }
+  };
+  // wave w forms the terms of chunk b0 + w, slot w
+  auto terms = [&](int b0) __attribute__((always_inline)) {
+    if (w >= kDirectTerms || b0 + w >= nch) return;
+    const int c = chunk_len(b0 + w);
+    const long long c0 = t0 + static_cast<long long>(kChunk) * (b0 + w);
+    const size_t gi = static_cast<size_t>(c0 + min(lane, c - 1)) * kVHeads + h;
+    const float a1[kGva] = {bf2f(a[gi]), 0.0f}, b1[kGva] = {bf2f(b[gi]), 0.0f};
+    const float al1[kGva] = {A_log[h], 0.0f}, dt1[kGva] = {dt_bias[h], 0.0f};
+    // 4 KB each in K (waves 0-3) and V (4-6) of buffer 1
+    PrepassNt* nt = reinterpret_cast<PrepassNt*>(w < 4 ? &sm.ks[1][0][0] : &sm.vs[1][0][0]) + (w & 3);
+    // only the 16-token blocks that hold tokens are formed (c <= 16 nb)
+    auto blocks = [&](auto NBC) __attribute__((always_inline)) {
+      constexpr int NB = decltype(NBC)::value;
+      bf16x8 kf[4][4];
+      chunk_gram_loads<NB>(k, c0, c, hq, lane, kf);
+      float last[1];
+      prepass_gates<1>(sm.w[w], c, a1, b1, al1, dt1, &sm.gt[w][0], last);
+      f32x4 kk[4][4];
+      chunk_gram_products<NB>(kf, kk);
+      prepass_terms<1, 0, true, NB>(sm.w[w], nt, kk, c, last, &sm.tb[w + 1][0], &sm.gt[w][0]);
+    };
+    chunk_by_tiles(c, blocks);
+  };
+  auto out_rsrc = [&](int j) {
+    return __builtin_amdgcn_make_buffer_rsrc(out + ((static_cast<size_t>(t0) + kChunk * j) * kVHeads + h) * kDim, 0,
+                                             chunk_len(j) * (kVHeads * kDim * 2), 0x00020000);
+  };
+  // the state's layout change, 16 rows x 32 columns at a time: 16-byte piece p
+  // of row r at p ^ (r & 7); the C layout takes pieces 2 lg and 2 lg + 1
+  auto scratch = [&](int P) { return reinterpret_cast<f32x4*>(&sm.qs[P][0][0]) + 128 * w; };
+  f32x4 st[8];
+
+  // runs chunk j (slot i of its batch) from buffer P
+  auto chunk = [&](int j, int i, int P, auto NBC) __attribute__((always_inline)) {
+    const ChunkLds lds = {sm.ks[P], sm.qs[P], sm.vs[P], sm.tb[i + 1], sm.tb[i], sm.gt[i]};
+    const int lane = opaque_lane(tid);
+    consumer_chunk<decltype(NBC)::value>(lds, chunk_len(j), st, w, lane, scale, out_rsrc(j),
+                                         2u * static_cast<uint32_t>(vcol + 4 * (lane >> 4)));
+  };
+  int pl = 0;   // the last chunk's buffer
+  for (int b0 = 0; b0 < nch; b0 += kDirectTerms) {   // batches of chunks whose terms are formed together
+    copy(b0, 0);   // past the first batch every wave is behind its last barrier: both buffers are free
+    terms(b0);
+    if (b0 == 0) {
+      const int lane = opaque_lane(tid), l16 = lane & 15, lg = lane >> 4;
+      f32x4* sc = scratch(1);
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) sc[8 * (8 * i + (lane >> 3)) + ((lane & 7) ^ (lane >> 3))] = rows[2 * qd + i];
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) st[2 * qd + i] = sc[8 * l16 + ((2 * lg + i) ^ (l16 & 7))];
+        wave_lds_sync();
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);   // the batch's first copies and its terms have landed
+    __syncthreads();
+    if (nch == 1) {
+      // a lone chunk (short prompts): only its tiles that hold tokens
+      chunk_by_tiles(len, [&](auto NBC) __attribute__((always_inline)) { chunk(0, 0, 0, NBC); });
+      break;
+    }
+    const int nb = min(kDirectTerms, nch - b0);
+    for (int i = 0; i < nb; ++i) {
+      const int P = i & 1;
+      if (i + 1 < nb) copy(b0 + i + 1, P ^ 1);   // that buffer is free
+      chunk(b0 + i, i, P, std::integral_constant<int, 4>{});
+      pl = P;
+      // the copies have landed (only the chunk's four output stores are
+      // younger) and this chunk's operands are dead, in every wave
+      if (b0 + i + 1 < nch) split_barrier<4>(false);
+    }
+  }
+  {
+    const int lane = opaque_lane(tid), l16 = lane & 15, lg = lane >> 4;
+    float* dst = new_state + soff_of(lane);
+    f32x4* sc = scratch(pl ^ 1);   // its last reader is past the last chunk's barrier
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) sc[8 * l16 + ((2 * lg + i) ^ (l16 & 7))] = st[2 * qd + i];
+      wave_lds_sync();
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        __builtin_nontemporal_store(sc[8 * (8 * i + (lane >> 3)) + ((lane & 7) ^ (lane >> 3))],
+                                    reinterpret_cast<f32x4*>(dst + piece(2 * qd + i)));
+      wave_lds_sync();
+    }
+  }
+}
 
 __global__ __launch_bounds__(kConsumerThreads) void direct_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
@@ -1949,107 +2223,42 @@ __global__ __launch_bounds__(kConsumerThreads) void direct_kernel(
     const float* __restrict__ dt_bias, const uint16_t* __restrict__ b, const void* __restrict__ cu, int is64,
     long long T, float scale, uint16_t* __restrict__ out, float* __restrict__ new_state) {
   __shared__ DirectSmem sm;
-  const int s = static_cast<int>(blockIdx.x) / kVHeads;
-  const int h = static_cast<int>(blockIdx.x) % kVHeads;
-  const int hq = h / kGva;
-  long long t0, t1;
-  seq_bounds(cu, is64, s, T, t0, t1);
-  const int len = static_cast<int>(t1 - t0);   // 0 .. T <= 128
-  const int nch = (len + kChunk - 1) / kChunk;
-  const int tid = threadIdx.x;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int l16 = lane & 15, lg = lane >> 4;
-  const int vcol = 16 * w;
-  auto kappa0 = [](int kt) { return 32 * (kt >> 1) + 4 * (kt & 1); };
-  const size_t soff = ((static_cast<size_t>(s) * kVHeads + h) * kDim + vcol + l16) * kDim + 8 * lg;
-  float* dst = new_state + soff;
-  if (len <= 0) {   // an empty sequence: zero state, no output rows
-#pragma unroll
-    for (int kt = 0; kt < 8; ++kt)
-      __builtin_nontemporal_store(f32x4{0.f, 0.f, 0.f, 0.f}, reinterpret_cast<f32x4*>(dst + kappa0(kt)));
-    return;
-  }
-  // chunk j: first token t0 + 64 j, c_j tokens
-  auto chunk_len = [&](int j) { return min(kChunk, len - kChunk * j); };
-  // chunk j's K / Q / V rows into buffer j (rows past c_j repeat its last row)
-  auto copy = [&](auto JC) {
-    constexpr int J = decltype(JC)::value;
-    const int r = 4 * w + (lane >> 4);
-    const uint32_t kq_col = 16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(r));
-    const uint32_t v_col = 16u * static_cast<uint32_t>((lane & 15) ^ v_swz(r));
-    const long long c0 = t0 + static_cast<long long>(kChunk) * J;
-    const size_t qk0 = (static_cast<size_t>(c0) * kQKHeads + hq) * kDim;
-    const char* kb = reinterpret_cast<const char*>(k + qk0);
-    const char* qb = reinterpret_cast<const char*>(q + qk0);
-    const char* vb = reinterpret_cast<const char*>(v + (static_cast<size_t>(c0) * kVHeads + h) * kDim);
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const uint32_t row = static_cast<uint32_t>(min(r + 32 * jj, chunk_len(J) - 1));
-      const uint32_t off = row * (kQKHeads * kDim * 2) + kq_col;
-      dma16(kb + off, &sm.c.ks[J][32 * jj + 4 * w][0]);
-      dma16(qb + off, &sm.c.qs[J][32 * jj + 4 * w][0]);
-      dma16<2>(vb + row * (kVHeads * kDim * 2) + v_col, &sm.c.vs[J][32 * jj + 4 * w][0]);
-    }
-  };
-  copy(std::integral_constant<int, 0>{});
-  if (nch > 1) copy(std::integral_constant<int, 1>{});
-  f32x4 st[8];
-  if (state != nullptr) {
-#pragma unroll
-    for (int kt = 0; kt < 8; ++kt)
-      st[kt] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(state + soff + kappa0(kt)));
+  direct_group(sm, static_cast<int>(blockIdx.x) / kVHeads, static_cast<int>(blockIdx.x) % kVHeads, 1 << 30, q, k, v,
+               state, A_log, a, dt_bias, b, cu, is64, T, scale, out, new_state);
+}
+
+// Work-group 0 plans the longer sequences, the next 8 num_seqs run the shorter
+// ones directly, the rest are the prepass of the longer ones (a record's eight
+// v-heads per group).
+constexpr int kMixedWaves = kConsumerThreads / 64;
+union MixedSmem {
+  DirectSmem direct;
+  PrepassSmem<kMixedWaves> pre;
+  int plan[kPlanScratch];
+};
+
+__global__ __launch_bounds__(kConsumerThreads) void mixed_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const float* __restrict__ state, const float* __restrict__ A_log, const uint16_t* __restrict__ a,
+    const float* __restrict__ dt_bias, const uint16_t* __restrict__ b, const void* __restrict__ cu, int is64,
+    int num_seqs, long long T, int R, int gcap, float scale, int* __restrict__ rec_start, int* __restrict__ lists,
+    uint16_t* __restrict__ ws_frag, float* __restrict__ ws_gam, uint16_t* __restrict__ out,
+    float* __restrict__ new_state) {
+  __shared__ MixedSmem sm;
+  const int bid = static_cast<int>(blockIdx.x);
+  if (bid == 0) {
+    int total_recs;
+    plan_batch<kConsumerThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, sm.plan, total_recs,
+                                 false, kMixedChunks);
+  } else if (bid <= num_seqs * kVHeads) {
+    direct_group(sm.direct, (bid - 1) / kVHeads, (bid - 1) % kVHeads, kMixedChunks, q, k, v, state, A_log, a, dt_bias,
+                 b, cu, is64, T, scale, out, new_state);
   } else {
-#pragma unroll
-    for (int kt = 0; kt < 8; ++kt) st[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int first = 1 + num_seqs * kVHeads;
+    prepass_items<false, kMixedWaves>(sm.pre, bid - first,
+                                      static_cast<int>(gridDim.x) - first, k, A_log, a, dt_bias, b, nullptr, cu, is64,
+                                      num_seqs, T, R, 1, kMixedChunks, rec_start, ws_frag, ws_gam);
   }
-  // wave j < nch forms chunk j's terms into buffer j
-  auto terms = [&](auto JC) {
-    constexpr int J = decltype(JC)::value;
-    const int c = chunk_len(J);
-    const long long c0 = t0 + static_cast<long long>(kChunk) * J;
-    const size_t gi = static_cast<size_t>(c0 + min(lane, c - 1)) * kVHeads + h;
-    const float a1[kGva] = {bf2f(a[gi]), 0.0f}, b1[kGva] = {bf2f(b[gi]), 0.0f};
-    const float al1[kGva] = {A_log[h], 0.0f}, dt1[kGva] = {dt_bias[h], 0.0f};
-    // only the 16-token blocks that hold tokens are formed (c <= 16 nb)
-    auto blocks = [&](auto NBC) {
-      constexpr int NB = decltype(NBC)::value;
-      bf16x8 kf[4][4];
-      chunk_gram_loads<NB>(k, c0, c, hq, lane, kf);
-      float last[1];
-      prepass_gates<1, true>(sm.w[J], c, a1, b1, al1, dt1, &sm.c.gt[J][0], last);
-      f32x4 kk[4][4];
-      chunk_gram_products<NB>(kf, kk);
-      prepass_terms<1, 0, true, NB>(sm.w[J], kk, c, last, &sm.c.frag[J][0][0], &sm.c.gt[J][0]);
-    };
-    switch ((c + 15) >> 4) {
-      case 1: blocks(std::integral_constant<int, 1>{}); break;
-      case 2: blocks(std::integral_constant<int, 2>{}); break;
-      case 3: blocks(std::integral_constant<int, 3>{}); break;
-      default: blocks(std::integral_constant<int, 4>{}); break;
-    }
-  };
-  if (w == 0) terms(std::integral_constant<int, 0>{});
-  if (w == 1 && nch > 1) terms(std::integral_constant<int, 1>{});
-  __builtin_amdgcn_s_waitcnt(0);   // copies, state loads and the terms have landed
-  __syncthreads();
-  const uint32_t ocol = 2u * static_cast<uint32_t>(vcol + 4 * lg);
-  auto out_rsrc = [&](int j) {
-    return __builtin_amdgcn_make_buffer_rsrc(out + ((static_cast<size_t>(t0) + kChunk * j) * kVHeads + h) * kDim, 0,
-                                             chunk_len(j) * (kVHeads * kDim * 2), 0x00020000);
-  };
-  // each wave carries its own state tile: no barrier between the chunks
-  if (nch > 1) {
-    consumer_chunk<0, 4>(sm.c, chunk_len(0), st, w, lane, scale, out_rsrc(0), ocol);
-    consumer_chunk<1, 4>(sm.c, chunk_len(1), st, w, lane, scale, out_rsrc(1), ocol);
-  } else {
-    // a lone chunk (short prompts): only its tiles that hold tokens
-    chunk_by_tiles(chunk_len(0), [&](auto NBC) {
-      consumer_chunk<0, decltype(NBC)::value>(sm.c, chunk_len(0), st, w, lane, scale, out_rsrc(0), ocol);
-    });
-  }
-#pragma unroll
-  for (int kt = 0; kt < 8; ++kt) __builtin_nontemporal_store(st[kt], reinterpret_cast<f32x4*>(dst + kappa0(kt)));
 }
 
 // ============================================================================
@@ -2073,27 +2282,6 @@ constexpr int kSplitThreads = 512;
 constexpr int kHalfV = 64;                 // value rows per split work-group (4 tiles)
 constexpr int kSideStores = 4;             // output stores a side wave issues per chunk, after its copies
 static_assert(kSideStores == kChunk / 16, "side_chunk stores one 8-byte row piece per 16-token block");
-
-// Barrier of the split consumer: every wave's LDS writes are visible, and each
-// side wave has at most kPending vector memory operations outstanding.  The
-// chain waves issue no vector memory operation a later phase depends on: their
-// state loads are waited for where the state is first used, and their
-// final-state stores need not have completed for the next item to start.
-// At the chunk's end (B3), kPending = kSideStores: a side wave issues its
-// copies at the chunk's start and its kSideStores output stores at the end,
-// and vector memory operations complete in issue order, so every copy has
-// landed while the output stores stay in flight into the next chunk.
-template <int kPending>
-__device__ __forceinline__ void split_barrier(bool chain) {
-  static_assert(kPending >= 0 && kPending < 16, "vmcnt field");
-  asm volatile("" ::: "memory");
-  if (chain)
-    __builtin_amdgcn_s_waitcnt(0xc07f);             // lgkmcnt(0)
-  else
-    __builtin_amdgcn_s_waitcnt(0x0070 | kPending);  // vmcnt(kPending), lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 struct __align__(16) SplitSmem {
   uint16_t ks[2][kChunk][kDim];
@@ -2651,7 +2839,6 @@ __device__ __forceinline__ void split_items(
   // barrier, with the next chunk's copies), and fills them at its end; blocks
   // past `formed` are left empty.  The finish then takes a block with a single
   // descriptor load.  The entry repeats the later-segment table's.
-  const int fix_max = fin_blocks(n);
   int fix_pos = 0;
 
   // An M-run stops once the bound of its map falls below kNegligibleLog2: its
@@ -2670,7 +2857,7 @@ __device__ __forceinline__ void split_items(
       split_dma<0>(sm, chunk_ref(0), dl, wt, h, hq, mrun, q, k, v, ws_frag, ws_gam);
     }
     split_barrier<0>(chain);   // the first chunk's copies and every S fragment in place
-    if (mrun && hv == 0 && tid == kFixLane) fix_pos = atomicAdd(lv.hdr + 9 + zero_v, fix_max);
+    if (mrun && hv == 0 && tid == kFixLane) fix_pos = atomicAdd(lv.hdr + 9 + zero_v, fin_blocks(n));
     for (int i = 0; i < n; i += 2) {
       {
         if (i + 1 >= n) claim();
@@ -2719,7 +2906,8 @@ __device__ __forceinline__ void split_items(
     mval[static_cast<size_t>(slot) * kVHeads + h] = formed | (formed < n ? kMNegligible : 0);
     *seg_ready(slotm, slot - jseg, jseg, h) = 0;
   }
-  if (mrun && hv == 0 && tid == kFixLane && fix_max > 0) {
+  if (mrun && hv == 0 && tid == kFixLane && n > 0) {
+    const int fix_max = fin_blocks(n);
     const int4 seg = make_int4(rb.x, rb.y, ((nrun - 1) * kChunk + last_tok) | (jseg << 17), slot - 1);
     const int bsz = fin_block_chunks(n, formed);
     for (int b = 0; b < fix_max && fix_pos + b < fix_cap; ++b) {
@@ -2827,15 +3015,6 @@ constexpr int kWideGroups = 512;           // two per CU
 constexpr int kWideStores = 4;             // output stores of a wave per chunk (one per 16-token block)
 
 __host__ __device__ constexpr int wide_row(int e, int i) { return 8 * (i >> 2) + 4 * e + (i & 3); }
-
-// The lane index through an opaque move: keeps the compiler from computing the
-// lane-dependent addresses of every phase once, outside the chunk and item
-// loops, and spilling them.
-__device__ __forceinline__ int opaque_lane(int lane) {
-  int l;
-  asm volatile("v_and_b32 %0, 63, %1" : "=v"(l) : "v"(lane));
-  return l;
-}
 
 struct __align__(16) WideSmem {
   uint16_t ks[2][kChunk][kDim];
@@ -3883,8 +4062,8 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
   auto* ob = static_cast<uint16_t*>(output);
   const int Ri = static_cast<int>(R), gc = static_cast<int>(gcap);
 
-  // at most two chunks in the whole call: one launch, no workspace traffic
-  if (total_tokens <= static_cast<long long>(kDirectMaxChunks) * kChunk && num_seqs <= kDirectMaxSeqs) {
+  // small calls: one launch, no workspace traffic
+  if (direct_batch(num_seqs, total_tokens)) {
     direct_kernel<<<dim3(static_cast<unsigned>(num_seqs * kVHeads)), dim3(kConsumerThreads), 0, st>>>(
         qb, kb, vb, state, A_log, ab, dt_bias, bb, cu_seqlens, cu_seqlens_is_int64, total_tokens, scale, ob,
         new_state);
@@ -3906,7 +4085,14 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
   // wave per (record, q/k head): the gram and the K loads are then not
   // repeated per v-head, and up to 512 records start at once.
   const long long items_v = R * kVHeads;
-  if (items_v <= kPrepassMaxGroups * kPrepassWaves) {
+  const bool mixed = mixed_batch(num_seqs, total_tokens);
+  if (mixed) {
+    // records of the longer sequences only: more than kMixedChunks chunks each
+    const long long g_mixed = 1 + static_cast<long long>(num_seqs) * kVHeads + total_tokens / kChunk + num_seqs;
+    mixed_kernel<<<dim3(static_cast<unsigned>(g_mixed)), dim3(kConsumerThreads), 0, st>>>(
+        qb, kb, vb, state, A_log, ab, dt_bias, bb, cu_seqlens, cu_seqlens_is_int64, num_seqs, total_tokens, Ri, gc,
+        scale, rec_start, lists, frag, gam, ob, new_state);
+  } else if (items_v <= kPrepassMaxGroups * kPrepassWaves) {
     const long long g_pre = (items_v + kPrepassWaves - 1) / kPrepassWaves;
     prepass_kernel<false, 2><<<dim3(static_cast<unsigned>(g_pre + fused_plan)), dim3(kPrepassThreads), 0, st>>>(
         kb, A_log, ab, dt_bias, bb, recs, cu_seqlens, cu_seqlens_is_int64, num_seqs, total_tokens,
@@ -3932,13 +4118,15 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
   } else {
     const long long g_long =
         total_tokens > kChunk ? std::min<long long>(max_runs(num_seqs, gcap) * 2 * kVHeads, kConsumerGroups) : 0;
-    const long long g_short = std::min<long long>(static_cast<long long>(num_seqs) * kVHeads, kConsumerGroups);
+    // a mixed batch has run its short sequences already
+    const long long g_short =
+        mixed ? 0 : std::min<long long>(static_cast<long long>(num_seqs) * kVHeads, kConsumerGroups);
     consumer_kernel<<<dim3(static_cast<unsigned>(g_long + g_short)), dim3(kSplitThreads), 0, st>>>(
         qb, kb, vb, state, Ri, gc, scale, lists, num_seqs, static_cast<int>(g_long), frag, gam, ob, new_state, oi,
         slotb, slotm, mval, fix);
   }
-  // a second segment needs more than kMinSegChunks chunks in one sequence and a slot
-  if (gcap > 0 && total_tokens > static_cast<long long>(kMinSegChunks) * kChunk) {
+  // M-runs need a sequence of more than kMaxWholeChunks chunks and slots
+  if (gcap > 0 && total_tokens > static_cast<long long>(kMaxWholeChunks) * kChunk) {
     const long long g_fin = std::min<long long>(R * kVHeads, kFinGroups);
     finish_kernel<<<dim3(static_cast<unsigned>(g_fin)), dim3(kFinThreads), 0, st>>>(
         lists, num_seqs, gc, fix, static_cast<int>(R * kVHeads), slotb, slotm, mval, oi, ob, new_state);
