@@ -2262,6 +2262,68 @@ __global__ __launch_bounds__(kConsumerThreads) void mixed_kernel(
 }
 
 // ============================================================================
+// global-to-LDS copies of the run consumers
+// ============================================================================
+constexpr uint32_t kKqRow = kQKHeads * kDim * 2, kVRow = kVHeads * kDim * 2;          // bytes per token
+constexpr uint32_t kFragRec = kVHeads * kMatElems * 2, kGamRec = kVHeads * kGamStride * 4;   // bytes per record
+
+__device__ __forceinline__ u32x4 rsrc_words(const void* base, uint32_t bytes) {
+  const uint64_t b = reinterpret_cast<uint64_t>(base);
+  return u32x4{static_cast<uint32_t>(b), static_cast<uint32_t>(b >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
+}
+
+// The copies are issued in assembly blocks, which hold no output register:
+// through the builtin the compiler makes every transposed LDS read wait for
+// every copy in flight (it cannot tell their LDS ranges apart), which ends the
+// overlap.  The waits are the barriers' own.  Unknown operations in
+// flight only make the compiler's own vmcnt waits stricter.  The leading nops
+// cover a resource word written by a VALU instruction just before.
+//
+// One 1 KB piece: lane i's 16 bytes at voff go to lds + 16 i.
+__device__ __forceinline__ void lds_dma1(const u32x4& rs, uint32_t voff, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\ts_nop 4\n\t"
+      "buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
+      : "memory", "m0");
+}
+
+// Four pieces: rows voff + j step, j < 4, to lds + 4096 j.
+template <bool kNt>
+__device__ __forceinline__ void lds_dma4(const u32x4& rs, uint32_t voff, uint32_t step, uint32_t lds) {
+  const uint32_t v1 = voff + step, v2 = voff + 2 * step, v3 = voff + 3 * step;
+  if constexpr (kNt)
+    asm volatile(
+        "s_mov_b32 m0, %5\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %4, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen nt lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen nt lds" ::"v"(voff),
+        "v"(v1), "v"(v2), "v"(v3), "s"(rs), "s"(lds)
+        : "memory", "m0", "scc");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %5\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
+        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen lds" ::"v"(voff),
+        "v"(v1), "v"(v2), "v"(v3), "s"(rs), "s"(lds)
+        : "memory", "m0", "scc");
+}
+
+// Two pieces: rows voff + j step, j < 2, to lds + 4096 j (streamed).
+__device__ __forceinline__ void lds_dma2_nt(const u32x4& rs, uint32_t voff, uint32_t step, uint32_t lds) {
+  const uint32_t v1 = voff + step;
+  asm volatile(
+      "s_mov_b32 m0, %3\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %2, 0 offen nt lds\n\t"
+      "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"v"(voff),
+      "v"(v1), "s"(rs), "s"(lds)
+      : "memory", "m0", "scc");
+}
+
+// ============================================================================
 // split consumer: one work-group per (seq, v-head, half of the value rows)
 // ============================================================================
 // For sequences of several chunks the recurrence is a chain through the state,
@@ -2311,60 +2373,49 @@ __device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t rs, uint32_t vo
                                            voff, 0, 0, AUX);
 }
 
-// Per-lane byte offsets of the side-wave copies; chunk-invariant because each
-// chunk's base address lives in the (scalar) buffer resource.
+// Per-lane byte offsets of the side-wave copies (chunk-invariant) and the
+// resources they go through.  Resources are formed once per kSplitRebase chunks
+// of an item, so that a chunk's copies differ only in a 32-bit offset: forming
+// them per chunk was half of what a side wave issued before its first product.
+// Rows past the run's last token fall outside and arrive as zeros.
 struct SplitDmaLane {
-  uint32_t kq[4];     // K / Q row (kr + 16 j), source chunk of this lane
-  uint32_t v[2];      // V row (vr + 32 j), this half's source chunk
+  uint32_t kq;        // K / Q row kr (+ 16 j), source chunk of this lane
+  uint32_t v;         // V row vr (+ 32 j), this half's source chunk
   uint32_t fr;        // fragment bytes of pass 0 (+4 KB per pass)
   uint32_t g;         // gate block
 };
+struct SplitRes {
+  u32x4 k, q, v, fr, g;
+  __amdgpu_buffer_rsrc_t out;   // output rows
+};
+constexpr int kSplitRebase = 4096;
+static_assert((kSplitRebase + 2ll) * kChunk * kVRow < (1ll << 31), "32-bit offsets");
 
 __device__ __forceinline__ SplitDmaLane split_dma_lane(int ws, int lane, int hv) {
   SplitDmaLane o;
   const int kr = 4 * ws + (lane >> 4);    // + 16 j keeps kr & 15
-  const uint32_t kcol = 16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(kr));
-#pragma unroll
-  for (int j = 0; j < 4; ++j) o.kq[j] = static_cast<uint32_t>(kr + 16 * j) * (kQKHeads * kDim * 2) + kcol;
+  o.kq = static_cast<uint32_t>(kr) * kKqRow + 16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(kr));
   const int vr = 8 * ws + (lane >> 3);    // + 32 j keeps vr & 3
-  const uint32_t vcol = 2u * kHalfV * hv + 16u * static_cast<uint32_t>((lane & 7) ^ vh_swz(vr));
-#pragma unroll
-  for (int j = 0; j < 2; ++j) o.v[j] = static_cast<uint32_t>(vr + 32 * j) * (kVHeads * kDim * 2) + vcol;
+  o.v = static_cast<uint32_t>(vr) * kVRow + 2u * kHalfV * hv + 16u * static_cast<uint32_t>((lane & 7) ^ vh_swz(vr));
   o.fr = static_cast<uint32_t>(64 * ws + lane) * 16u;
   o.g = 16u * static_cast<uint32_t>(lane);
   return o;
 }
 
-// Side-wave copies of one chunk's operands into buffer P (4 side waves).
-// Rows t >= c fall outside the K / Q / V resources and arrive as zeros.
+// Side-wave copies of chunk i (counted from the resources' first) into buffer P
+// (4 side waves).
 template <int P>
-__device__ __forceinline__ void split_dma(SplitSmem& sm, const ChunkRef& cr, const SplitDmaLane& dl, int ws,
-                                          int h, int hq, bool zero_v, const uint16_t* __restrict__ q,
-                                          const uint16_t* __restrict__ k,
-                                          const uint16_t* __restrict__ v,
-                                          const uint16_t* __restrict__ ws_frag,
-                                          const float* __restrict__ ws_gam) {
-  const size_t qk0 = (static_cast<size_t>(cr.c0) * kQKHeads + hq) * kDim;
-  const uint32_t kq_bytes = static_cast<uint32_t>(cr.c) * (kQKHeads * kDim * 2);
-  const __amdgpu_buffer_rsrc_t kr = buf_rsrc(k + qk0, kq_bytes);
-  const __amdgpu_buffer_rsrc_t qr = buf_rsrc(q + qk0, kq_bytes);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    dma16_buf(kr, dl.kq[j], &sm.ks[P][16 * j + 4 * ws][0]);
-    dma16_buf(qr, dl.kq[j], &sm.qs[P][16 * j + 4 * ws][0]);
-  }
-  // an M-run reads V = 0: an empty resource makes every V copy a zero fill
-  const __amdgpu_buffer_rsrc_t vr = buf_rsrc(v + (static_cast<size_t>(cr.c0) * kVHeads + h) * kDim,
-                                             zero_v ? 0u : static_cast<uint32_t>(cr.c) * (kVHeads * kDim * 2));
-#pragma unroll
-  for (int j = 0; j < 2; ++j) dma16_buf<2>(vr, dl.v[j], &sm.vs[P][32 * j + 8 * ws][0]);   // V: read once
-  const size_t rh = static_cast<size_t>(cr.rec) * kVHeads + h;
+__device__ __forceinline__ void split_dma(SplitSmem& sm, const SplitRes& rs, int i, const SplitDmaLane& dl, int ws) {
+  const uint32_t rows = static_cast<uint32_t>(i) * kChunk;
+  lds_dma4<false>(rs.k, dl.kq + rows * kKqRow, 16 * kKqRow, lds_addr(&sm.ks[P][0][0]) + 1024u * ws);
+  lds_dma4<false>(rs.q, dl.kq + rows * kKqRow, 16 * kKqRow, lds_addr(&sm.qs[P][0][0]) + 1024u * ws);
+  lds_dma2_nt(rs.v, dl.v + rows * kVRow, 32 * kVRow, lds_addr(&sm.vs[P][0][0]) + 1024u * ws);   // V: read once
   // the 6 Tb fragments of 1 KB: side wave ws copies ws and ws + 4 (< 6); the
   // side waves form Aqk themselves
-  const __amdgpu_buffer_rsrc_t fr = buf_rsrc(ws_frag + rh * kMatElems, kMatElems * 2);
-  dma16_buf(fr, dl.fr, &sm.frag[P][0][0] + 64 * ws * 8);
-  if (ws + 4 < kMatFrags) dma16_buf(fr, dl.fr + 4096u, &sm.frag[P][0][0] + (256 + 64 * ws) * 8);
-  if (ws == 0) dma16_buf(buf_rsrc(ws_gam + rh * kGamStride, kGamStride * 4), dl.g, &sm.gt[P][0]);
+  const uint32_t fr = dl.fr + static_cast<uint32_t>(i) * kFragRec, tb = lds_addr(&sm.frag[P][0][0]) + 1024u * ws;
+  lds_dma1(rs.fr, fr, tb);
+  if (ws + 4 < kMatFrags) lds_dma1(rs.fr, fr + 4096u, tb + 4096u);
+  if (ws == 0) lds_dma1(rs.g, dl.g + static_cast<uint32_t>(i) * kGamRec, lds_addr(&sm.gt[P][0]));
 }
 
 // bf16 B-operand fragments of the state tile: slots of depth chunk d are
@@ -2634,14 +2685,19 @@ __device__ __forceinline__ void side_front(SplitSmem& sm, int lane, f32x4 (&YT)[
     }
 }
 
-// Side wave, one chunk: outputs of the chunk (tile of chain wave ws).
+// Side wave, one chunk: outputs of the chunk (tile of chain wave ws).  A warm-up
+// chunk (emit false) has none: only the copies and the barrier.
 template <int P, typename Copy>
-__device__ __forceinline__ void side_chunk(SplitSmem& sm, int ws, int lane, float scale,
-                                           __amdgpu_buffer_rsrc_t orc, uint32_t ocol, Copy&& copy_next) {
+__device__ __forceinline__ void side_chunk(SplitSmem& sm, int ws, int lane, float scale, bool emit,
+                                           const __amdgpu_buffer_rsrc_t& orc, uint32_t ocol, Copy&& copy_next) {
   const int l16 = lane & 15;
   // the copies go first: they then have the whole chunk to land, and Y^T runs
   // while the chain wave is in its VALU-heavy R / Delta phase instead of X
-  copy_next();
+  const uint32_t orow = copy_next();   // and the chunk's first output row in orc, in bytes
+  if (!emit) {   // uniform
+    lds_barrier();   // B2
+    return;
+  }
   f32x4 YT[4];
   switch (ws) {   // uniform
     case 0: side_front<0, P>(sm, lane, YT); break;
@@ -2675,7 +2731,7 @@ __device__ __forceinline__ void side_chunk(SplitSmem& sm, int ws, int lane, floa
     const int t = 16 * m + l16;
     const u32x2 pk = {pack_bf2(sg[m] * YT[m][0] + scale * OT[m][0], sg[m] * YT[m][1] + scale * OT[m][1]),
                       pack_bf2(sg[m] * YT[m][2] + scale * OT[m][2], sg[m] * YT[m][3] + scale * OT[m][3])};
-    __builtin_amdgcn_raw_buffer_store_b64(pk, orc, static_cast<uint32_t>(t) * (kVHeads * kDim * 2) + ocol, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(pk, orc, orow + static_cast<uint32_t>(t) * kVRow + ocol, 0, 0);
   }
 }
 
@@ -2804,10 +2860,7 @@ __device__ __forceinline__ void split_items(
   const int l16 = lane & 15, lg = lane >> 4;
   const int vcol = kHalfV * hv + 16 * wt;
   // chunk i of the item is chunk i - warmup of the run (negative: warm-up chunks, all full)
-  auto chunk_ref = [&](int i) {
-    const int li = i - warmup;
-    return ChunkRef{c0r + static_cast<long long>(li) * kChunk, li == nrun - 1 ? last_tok : kChunk, rfirst + li};
-  };
+  auto chunk_len = [&](int i) { return i - warmup == nrun - 1 ? last_tok : kChunk; };
   auto kappa = [&](int kt, int rr) { return 32 * (kt >> 1) + 8 * lg + 4 * (kt & 1) + rr; };
 
   f32x4 st[8];
@@ -2825,14 +2878,36 @@ __device__ __forceinline__ void split_items(
       for (int kt = 0; kt < 8; ++kt) st[kt] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(sp + kappa(kt, 0)));
     }
   }
-  uint16_t* obase = mrun ? oi : out;
   const uint32_t ocol = 2u * static_cast<uint32_t>(vcol + 4 * lg);
-  // output rows of chunk i: none for warm-up chunks (the stores fall outside the resource)
-  auto out_rsrc = [&](int i, const ChunkRef& cr) {
-    return buf_rsrc(obase + (static_cast<size_t>(cr.c0) * kVHeads + h) * kDim,
-                    i < warmup ? 0u : static_cast<uint32_t>(cr.c) * (kVHeads * kDim * 2));
-  };
   const SplitDmaLane dl = split_dma_lane(wt, lane, hv);
+  // resources for the copies of chunks i0 .. and the outputs of chunks
+  // i0 - 1 .. of the item (a chunk's outputs follow the next one's copies),
+  // counted from chunk rs0
+  SplitRes rs;
+  int rs0 = 0;
+  auto rebase = [&](int i0) {
+    rs0 = max(i0 - 1, 0);
+    const long long cb = c0r + static_cast<long long>(rs0 - warmup) * kChunk;
+    const int left = min(warmup + nrun - 1 - rs0, kSplitRebase + 1);   // full chunks
+    const uint32_t rows = static_cast<uint32_t>(left) * kChunk + (left <= kSplitRebase ? last_tok : 0);
+    const size_t kq0 = (static_cast<size_t>(cb) * kQKHeads + hq) * kDim;
+    const size_t r0 = static_cast<size_t>(rfirst + rs0 - warmup) * kVHeads + h;
+    const uint32_t recs = static_cast<uint32_t>(min(n - rs0, kSplitRebase + 1));
+    rs.k = rsrc_words(k + kq0, rows * kKqRow);
+    rs.q = rsrc_words(q + kq0, rows * kKqRow);
+    // an M-run reads V = 0: an empty resource makes every V copy a zero fill
+    const size_t v0 = (static_cast<size_t>(cb) * kVHeads + h) * kDim;
+    rs.v = rsrc_words(v + v0, mrun ? 0u : rows * kVRow);
+    rs.out = buf_rsrc((mrun ? oi : out) + v0, rows * kVRow);
+    rs.fr = rsrc_words(ws_frag + r0 * kMatElems, recs * kFragRec);
+    rs.g = rsrc_words(ws_gam + r0 * kGamStride, recs * kGamRec);
+  };
+  auto copy = [&](int i, auto PC) {   // side waves: chunk i's operands
+    if (i - rs0 > kSplitRebase) rebase(i);
+    split_dma<decltype(PC)::value>(sm, rs, i - rs0, dl, wt);
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
   // Correction blocks of the segment: chunks [0, formed) get O0 + OI S_j^T in
   // the finish.  Each M-run (once per v-head) reserves its blocks (fin_blocks)
   // during its first chunk (the atomic returns before that chunk's closing
@@ -2854,23 +2929,29 @@ __device__ __forceinline__ void split_items(
 #pragma unroll
       for (int d = 0; d < 4; ++d) sm.sbx[wt][d][lane] = __builtin_bit_cast(u32x4, sb[d]);
     } else {
-      split_dma<0>(sm, chunk_ref(0), dl, wt, h, hq, mrun, q, k, v, ws_frag, ws_gam);
+      rebase(0);
+      copy(0, B0{});
     }
     split_barrier<0>(chain);   // the first chunk's copies and every S fragment in place
     if (mrun && hv == 0 && tid == kFixLane) fix_pos = atomicAdd(lv.hdr + 9 + zero_v, fin_blocks(n));
     for (int i = 0; i < n; i += 2) {
       {
         if (i + 1 >= n) claim();
-        const ChunkRef cr = chunk_ref(i);
         if (chain) {
-          chain_chunk<0>(sm, cr.c, st, wt, lane);
+          chain_chunk<0>(sm, chunk_len(i), st, wt, lane);
         } else {
-          side_chunk<0>(sm, wt, lane, scale, out_rsrc(i, cr), ocol, [&] {
-            if (i + 1 < n) split_dma<1>(sm, chunk_ref(i + 1), dl, wt, h, hq, mrun, q, k, v, ws_frag, ws_gam);
+          side_chunk<0>(sm, wt, lane, scale, i >= warmup, rs.out, ocol, [&] {
+            if (i + 1 < n) copy(i + 1, B1{});
+            return static_cast<uint32_t>(i - rs0) * kChunk * kVRow;
           });
         }
         lbound += sm.gt[0][kBoundAt];
-        split_barrier<kSideStores>(chain);   // B3: buffer 0 free, buffer 1 landed
+        // B3: buffer 0 free, buffer 1 landed (a warm-up chunk has no output
+        // stores younger than its copies)
+        if (i >= warmup)
+          split_barrier<kSideStores>(chain);
+        else
+          split_barrier<0>(chain);
       }
       if (mrun && lbound < kNegligibleLog2) {
         formed = i + 1;
@@ -2878,16 +2959,19 @@ __device__ __forceinline__ void split_items(
       }
       if (i + 1 < n) {
         if (i + 2 >= n) claim();
-        const ChunkRef cr = chunk_ref(i + 1);
         if (chain) {
-          chain_chunk<1>(sm, cr.c, st, wt, lane);
+          chain_chunk<1>(sm, chunk_len(i + 1), st, wt, lane);
         } else {
-          side_chunk<1>(sm, wt, lane, scale, out_rsrc(i + 1, cr), ocol, [&] {
-            if (i + 2 < n) split_dma<0>(sm, chunk_ref(i + 2), dl, wt, h, hq, mrun, q, k, v, ws_frag, ws_gam);
+          side_chunk<1>(sm, wt, lane, scale, i + 1 >= warmup, rs.out, ocol, [&] {
+            if (i + 2 < n) copy(i + 2, B0{});
+            return static_cast<uint32_t>(i + 1 - rs0) * kChunk * kVRow;
           });
         }
         lbound += sm.gt[1][kBoundAt];
-        split_barrier<kSideStores>(chain);
+        if (i + 1 >= warmup)
+          split_barrier<kSideStores>(chain);
+        else
+          split_barrier<0>(chain);
         if (mrun && lbound < kNegligibleLog2) {
           formed = i + 2;
           break;
@@ -3035,57 +3119,9 @@ struct WideItem {
   u32x4 k, q, v, fr, g;
   __amdgpu_buffer_rsrc_t out;
 };
-constexpr uint32_t kKqRow = kQKHeads * kDim * 2, kVRow = kVHeads * kDim * 2;          // bytes per token
-constexpr uint32_t kFragRec = kVHeads * kMatElems * 2, kGamRec = kVHeads * kGamStride * 4;   // bytes per record
 // an item's rows of V, the widest stream, must fit the 32-bit offsets
 constexpr long long kWideMaxTokens = 1 << 20;
 static_assert((kWideMaxTokens + 2 * kChunk) * kVRow < (1ll << 32), "32-bit offsets");
-
-__device__ __forceinline__ u32x4 rsrc_words(const void* base, uint32_t bytes) {
-  const uint64_t b = reinterpret_cast<uint64_t>(base);
-  return u32x4{static_cast<uint32_t>(b), static_cast<uint32_t>(b >> 32) & 0xffffu, bytes, 0x00020000u};
-}
-
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
-}
-
-// The copies are issued in assembly blocks, which hold no output register:
-// through the builtin the compiler makes every transposed LDS read wait for
-// every copy in flight (it cannot tell their LDS ranges apart), which ends the
-// overlap.  The waits are the barriers' own (W2).  Unknown operations in
-// flight only make the compiler's own vmcnt waits stricter.  The leading nops
-// cover a resource word written by a VALU instruction just before.
-//
-// One 1 KB piece: lane i's 16 bytes at voff go to lds + 16 i.
-__device__ __forceinline__ void wide_dma1(const u32x4& rs, uint32_t voff, uint32_t lds) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\ts_nop 4\n\t"
-      "buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
-      : "memory", "m0");
-}
-
-// Four pieces: rows voff + j step, j < 4, to lds + 4096 j.
-template <bool kNt>
-__device__ __forceinline__ void wide_dma4(const u32x4& rs, uint32_t voff, uint32_t step, uint32_t lds) {
-  const uint32_t v1 = voff + step, v2 = voff + 2 * step, v3 = voff + 3 * step;
-  if constexpr (kNt)
-    asm volatile(
-        "s_mov_b32 m0, %5\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %4, 0 offen nt lds\n\t"
-        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen nt lds\n\t"
-        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen nt lds\n\t"
-        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen nt lds" ::"v"(voff),
-        "v"(v1), "v"(v2), "v"(v3), "s"(rs), "s"(lds)
-        : "memory", "m0", "scc");
-  else
-    asm volatile(
-        "s_mov_b32 m0, %5\n\ts_nop 4\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds\n\t"
-        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
-        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
-        "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen lds" ::"v"(voff),
-        "v"(v1), "v"(v2), "v"(v3), "s"(rs), "s"(lds)
-        : "memory", "m0", "scc");
-}
 
 // Copies of chunk i's operands: wave w copies rows 4 w + lane / 16 + 16 j of K,
 // Q and V (1 KB per instruction).
@@ -3096,9 +3132,9 @@ __device__ __forceinline__ void wide_dma_k(WideSmem& sm, int P, const WideItem& 
   const int row = 4 * w + (lane >> 4);
   const uint32_t off = static_cast<uint32_t>(i * kChunk + row) * kKqRow +
                        16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(row));
-  wide_dma4<false>(it.k, off, 16 * kKqRow, lds_addr(&sm.ks[0][0][0]) + 16384u * P + 1024u * w);
+  lds_dma4<false>(it.k, off, 16 * kKqRow, lds_addr(&sm.ks[0][0][0]) + 16384u * P + 1024u * w);
   if (w == kWideWaves - 1)
-    wide_dma1(it.g, 16u * static_cast<uint32_t>(lane) + i * kGamRec, lds_addr(&sm.gt[0][0]) + 1024u * P);
+    lds_dma1(it.g, 16u * static_cast<uint32_t>(lane) + i * kGamRec, lds_addr(&sm.gt[0][0]) + 1024u * P);
 }
 
 // Q and V rows and the Tb fragments.
@@ -3107,13 +3143,13 @@ __device__ __forceinline__ void wide_dma_qvt(WideSmem& sm, const WideItem& it, i
   const int row = 4 * w + (lane >> 4);
   const uint32_t r = static_cast<uint32_t>(i * kChunk + row);
   // V first: the only stream the prepass has not touched
-  wide_dma4<true>(it.v, r * kVRow + 16u * static_cast<uint32_t>((lane & 15) ^ v_swz(row)), 16 * kVRow,
+  lds_dma4<true>(it.v, r * kVRow + 16u * static_cast<uint32_t>((lane & 15) ^ v_swz(row)), 16 * kVRow,
                   lds_addr(&sm.vs[0][0]) + 1024u * w);
-  wide_dma4<false>(it.q, r * kKqRow + 16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(row)), 16 * kKqRow,
+  lds_dma4<false>(it.q, r * kKqRow + 16u * static_cast<uint32_t>((lane & 15) ^ kq_swz(row)), 16 * kKqRow,
                    lds_addr(&sm.qs[0][0]) + 1024u * w);
   const uint32_t foff = static_cast<uint32_t>(64 * w + lane) * 16u + i * kFragRec;
-  wide_dma1(it.fr, foff, lds_addr(sm.tb) + 1024u * w);
-  if (w + kWideWaves < kMatFrags) wide_dma1(it.fr, foff + 4096u, lds_addr(sm.tb) + 4096u + 1024u * w);
+  lds_dma1(it.fr, foff, lds_addr(sm.tb) + 1024u * w);
+  if (w + kWideWaves < kMatFrags) lds_dma1(it.fr, foff + 4096u, lds_addr(sm.tb) + 4096u + 1024u * w);
 }
 
 // A 32 x 128 fp32 state tile (two 16-row tiles of a wave) between memory and
@@ -3951,7 +3987,7 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
     if (my < last) load_chunk(my);
     if (tid == 0) {
       int* rd = seg_ready(slotm, g0, j, h);
-      while (__hip_atomic_load(rd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kFinReady) __builtin_amdgcn_s_sleep(2);
+      while (__hip_atomic_load(rd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kFinReady) __builtin_amdgcn_s_sleep(8);
     }
     __syncthreads();
     // S_j's fragments, published over the slot of segment j - 1: part p's 8 KB
