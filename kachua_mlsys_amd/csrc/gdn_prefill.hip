@@ -132,7 +132,8 @@ __host__ __device__ inline long long max_segments(long long tokens) {
 //   [3] multi-segment sequences, [4] segments >= 1 over all sequences,
 //   [5] 1 when the batch uses warm-up segments (no M-runs, no finish work),
 //   [8] split-consumer work queue (items claimed past each group's first),
-//   [9] correction blocks appended by the consumer's M-runs, [10] finish queue
+//   [9] correction blocks appended by the consumer's M-runs, [10] finish queue,
+//   [11] most segments of any sequence
 //   multi[e]   = (seq, first slot, segments, 0)
 //   segs[i]    = (first token lo, hi, tokens in the segment | j << 17, slot of
 //                 segment j - 1) for every segment j >= 1 (L <= 1024 chunks:
@@ -170,7 +171,7 @@ constexpr int kSlotNone = -2;
 // it starts: pairs of chunks in shorter segments (more groups at work), four
 // chunks in longer ones (the state's fragments are fetched once per block),
 // and spreads the chunks it formed over them at its end.
-__host__ __device__ constexpr int fin_blocks(int n) { return n <= 24 ? (n + 1) / 2 : (n + 3) / 4; }
+__host__ __device__ constexpr int fin_blocks(int n) { return n <= 14 ? (n + 1) / 2 : (n + 3) / 4; }
 __host__ __device__ constexpr int fin_block_chunks(int n, int formed) {
   const int nb = fin_blocks(n), even = nb > 0 ? (formed + nb - 1) / nb : 0;
   return even > 2 ? even : 2;
@@ -259,9 +260,10 @@ __host__ __device__ inline WsLayout ws_layout(int num_seqs, long long tokens, lo
 // segment map per v-head).  The planner's best segmentings of the benchmark
 // batches use at most a few dozen (16 sequences of 16384 tokens: 10).
 constexpr long long kDefaultSlots = 48;
-// A sequence's segments are counted ready in one slot's 64 KB (seg_ready).
-constexpr long long kMaxSlots = 16384;
-static_assert(kMaxSlots * sizeof(int) <= kMSlotElems * sizeof(uint16_t), "a count per segment");
+// A sequence's segments are counted ready in the first half of one slot's 64 KB
+// (seg_ready).
+constexpr long long kMaxSlots = 8192;
+static_assert(kMaxSlots * sizeof(int) <= kMSlotElems * sizeof(uint16_t) / 2, "a count per segment");
 
 // The most slots (up to what the batch can use) whose layout fits `bytes`, or
 // -1 when not even the layout without slots fits.
@@ -671,6 +673,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     if (lane == 0) {
       ps[kPsMisc] = seg_cand(63 - (best & 63));
       ps[kPsMisc + 1] = warm ? 1 : 0;
+      ps[kPsMisc + 2] = ml > 0 ? (ml - 1) / seg_cand(63 - (best & 63)) + 1 : 0;
     }
   }
   __syncthreads();
@@ -713,6 +716,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       lv.hdr[8] = 0;   // work queue
       lv.hdr[9] = 0;   // correction blocks
       lv.hdr[10] = 0;  // finish queue
+      lv.hdr[11] = ps[kPsMisc + 2];
     }
     if (lane == 63) {
       lv.hdr[0] = tot[4] + inc;
@@ -3735,8 +3739,8 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
 //        alone after an M-run that stopped early, whose map is negligible) and
 //        publishes S_j as bf16 correction fragments; S_nseg goes to new_state.
 //   a correction block (segment j >= 1, v-head, a few chunks whose OI was
-//        formed), as the consumer's M-run appended it: waits
-//        until S_j is published, then out = bf16(O0 + OI S_j^T), wave w taking
+//        formed), as the consumer's M-run appended it: waits until S_j is
+//        published (S_1 is the first segment's slot itself), then out = bf16(O0 + OI S_j^T), wave w taking
 //        16-token tile w of each chunk (the other chunks keep O0).
 // Scan items precede every block in the queue and wait for nothing, so a block
 // only ever waits for items that running groups hold, whatever share of the
@@ -3846,7 +3850,11 @@ __device__ __forceinline__ void scan_item(FinishLds& sm, const int4& me, int h, 
     // publish S_j: natural-order A fragments, 8 bytes per row tile.  Value row
     // 16 rt + l16 of the part goes to row i of v-tile e, 16 rt + l16 =
     // wide_row(e, i), so that a block's lanes hold eight consecutive columns
-    auto* pub = reinterpret_cast<unsigned long long*>(slotb + head(j - 1) * kHeadState + r0 * kDim);
+    // (S_1 is its slot's state itself, which the blocks of segment 1 read as it
+    // is: its fragments go unused to the second half of the counts' area)
+    auto* pub = j > 1 ? reinterpret_cast<unsigned long long*>(slotb + head(j - 1) * kHeadState + r0 * kDim)
+                      : reinterpret_cast<unsigned long long*>(slotm + head(0) * kMSlotElems + kMSlotElems / 2) +
+                            part * (kFinRows * kDim / 4);
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
       const u32x2 pk = {pack_bf2(s[rt][0], s[rt][1]), pack_bf2(s[rt][2], s[rt][3])};
@@ -3854,7 +3862,7 @@ __device__ __forceinline__ void scan_item(FinishLds& sm, const int4& me, int h, 
       __hip_atomic_store(pub + ((e * 4 + (w >> 1)) * 64 + 16 * (2 * (w & 1) + (lg >> 1)) + i) * 2 + (lg & 1),
                          __builtin_bit_cast(unsigned long long, pk), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
-    if constexpr (!kLong) {
+    if (!kLong && j > 1) {
       __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
       asm volatile("" ::: "memory");
       raise(j);
@@ -3927,25 +3935,35 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int l16 = lane & 15, lg = lane >> 4;
-  const int nscan = nmulti * kVHeads * kFinParts;
+  if (nmulti + ncorr == 0) return;
+  // The next claim is requested while an item is worked on.  A group that waits
+  // in a block holds at most another block: claims only grow.  Where no sequence
+  // has a third segment nothing waits, and every group starts with its own
+  // item (256 first claims cost about 1.5 us) and scans two parts at a time (at
+  // most one round of items for a few sequences).
+  const bool waits = lv.hdr[11] > 2;
+  const int parts = waits ? 1 : 2;
+  const int nscan = nmulti * kVHeads * (kFinParts / parts);
   const int nitem = ncorr + nscan;
-  if (nitem == 0) return;
-  // the next claim is requested while an item is worked on.  A group that waits
-  // in a block holds at most another block: claims only grow
+  const int base = waits ? 0 : static_cast<int>(gridDim.x);
   int zero_v;   // as in split_items: a plain single-lane atomic, waited for at its use
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero_v));
-  int next = 0;
-  if (tid == 0) next = atomicAdd(lv.hdr + 10 + zero_v, 1);
+  int next = static_cast<int>(blockIdx.x);
+  if (waits && tid == 0) next = atomicAdd(lv.hdr + 10 + zero_v, 1);
   for (;;) {
     if (tid == 0) claimed = next;
     __syncthreads();   // also: the previous item's readers of sm are done
     const int it = __builtin_amdgcn_readfirstlane(claimed);
     __syncthreads();   // every wave has the claim before the next one
     if (it >= nitem) break;
-    if (tid == 0) next = atomicAdd(lv.hdr + 10 + zero_v, 1);
+    if (tid == 0) next = base + atomicAdd(lv.hdr + 10 + zero_v, 1);
     if (it < nscan) {
-      scan_item(sm, lv.multi[it / (kVHeads * kFinParts)], (it / kFinParts) % kVHeads, it % kFinParts, slotb, slotm,
-                mval, new_state, w, lane);
+      const int per = kFinParts / parts;
+      for (int pt = 0; pt < parts; ++pt) {
+        if (pt > 0) __syncthreads();
+        scan_item(sm, lv.multi[it / (kVHeads * per)], (it / per) % kVHeads, (it % per) * parts + pt, slotb, slotm, mval,
+                  new_state, w, lane);
+      }
       continue;
     }
     // block: (first token lo, hi, tokens | j << 17, slot of segment j - 1) and
@@ -3985,21 +4003,30 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
     };
     const int my = first + (w >> 2);
     if (my < last) load_chunk(my);
-    if (tid == 0) {
-      int* rd = seg_ready(slotm, g0, j, h);
-      while (__hip_atomic_load(rd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kFinReady) __builtin_amdgcn_s_sleep(8);
-    }
-    __syncthreads();
-    // S_j's fragments, published over the slot of segment j - 1: part p's 8 KB
-    // (v-tiles 2 p, 2 p + 1) at its rows' place
-    const __amdgpu_buffer_rsrc_t src =
-        buf_rsrc(slotb + (static_cast<size_t>(sg.w) * kVHeads + h) * kHeadState, kHeadState * 4);
-    u32x4 fr[4];
+    const float* slot = slotb + (static_cast<size_t>(sg.w) * kVHeads + h) * kHeadState;
+    u32x4 fr[4];   // wave w brings v-tile w's fragments
+    if (j == 1) {
+      // S_1: the first segment's state, as its run left it
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int vt = w, d = e;   // wave w brings v-tile w's fragments
-      fr[e] = __builtin_amdgcn_raw_buffer_load_b128(
-          src, (vt >> 1) * (kFinRows * kDim * 4) + (((vt & 1) * 4 + d) * 64 + lane) * 16, 0, kSc01);
+      for (int d = 0; d < 4; ++d) {
+        const float* sp = slot + (32 * (w >> 1) + wide_row(w & 1, l16)) * kDim + 32 * d + 8 * lg;
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(sp), x1 = *reinterpret_cast<const f32x4*>(sp + 4);
+        fr[d] = u32x4{pack_bf2(x0[0], x0[1]), pack_bf2(x0[2], x0[3]), pack_bf2(x1[0], x1[1]), pack_bf2(x1[2], x1[3])};
+      }
+    } else {
+      if (tid == 0) {
+        int* rd = seg_ready(slotm, g0, j, h);
+        while (__hip_atomic_load(rd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kFinReady)
+          __builtin_amdgcn_s_sleep(8);
+      }
+      __syncthreads();
+      // S_j's fragments, published over the slot of segment j - 1: part p's 8 KB
+      // (v-tiles 2 p, 2 p + 1) at its rows' place
+      const __amdgpu_buffer_rsrc_t src = buf_rsrc(slot, kHeadState * 4);
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        fr[d] = __builtin_amdgcn_raw_buffer_load_b128(
+            src, (w >> 1) * (kFinRows * kDim * 4) + (((w & 1) * 4 + d) * 64 + lane) * 16, 0, kSc01);
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) sm.frag[w][e][lane] = fr[e];
