@@ -222,15 +222,17 @@ def cpu_prefill_baseline(torch, p, max_tokens=1 << 30):
                       f"({tot} tokens) of the workload, {t:.2f} s"}
 
 
-def time_prefill(p_cpu, args, torch, dev, traffic=None, warm=None) -> dict:
+def time_prefill(p_cpu, args, torch, dev, traffic=None, warm=None, split=True) -> dict:
     """One prefill workload: µs per call (HIP-graph replay, rotated buffer
-    sets unless warm), tokens/s and its roofline."""
+    sets unless warm), tokens/s and its roofline.  split=False gives the
+    smallest workspace, whose lack of segment slots keeps sequences whole."""
     from kachua_mlsys_amd import prefill
 
     warm = args.warm_cache if warm is None else warm
     p = p_cpu.to(dev)
     T, N = p.q.shape[0], len(p.lengths)
-    ws = torch.empty(prefill.workspace_bytes(N, T), dtype=torch.uint8, device=dev)
+    need = prefill.workspace_bytes(N, T) if split else prefill.workspace_min_bytes(N, T)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
     per_set = prefill_bytes(T, N) + ws.numel()
     nsets = 1 if warm else max(2, math.ceil(2 * MALL_BYTES / per_set) + 1)
     sets = []
@@ -287,7 +289,7 @@ def planned_segment_chunks(ws, N, T, torch):
     that used workspace `ws`, or None when no sequence was split.  The list
     header sits after the Tb fragments, the gate blocks and rec_start
     (ws_layout in csrc/gdn_prefill.hip); header[2] is L."""
-    if T <= 2 * 64:          # the direct path: no plan
+    if T <= 4 * 64 and N <= 64:   # the direct path: no plan
         return None
     def a256(x):
         return (x + 255) // 256 * 256
@@ -299,22 +301,22 @@ def planned_segment_chunks(ws, N, T, torch):
 
 
 def chain_step_us(args, torch, dev) -> dict:
-    """Time of one chunk step of the consumer's sequential state chain: one
-    sequence of 4 chunks against one of 3 (warm cache; too long for the direct
-    path, so the difference is one chunk step of the chain as long as the
-    planner cuts neither into segments, which it normally does not at these
-    lengths: `us` is None when it did)."""
+    """Time of one chunk step of the split consumer's sequential state chain: one
+    sequence of 9 chunks against one of 8 (warm cache; too long for the direct
+    path, and a workspace without segment slots keeps both whole, so the
+    difference is one chunk step of the chain; `us` is None if the planner cut
+    either all the same)."""
     from kachua_mlsys_amd.inputs import prefill_inputs_from_lengths
 
     t, seg = {}, {}
-    for nch in (3, 4):
+    for nch in (8, 9):
         p = prefill_inputs_from_lengths([64 * nch], seed=11)
-        r = time_prefill(p, args, torch, dev, warm=True)
+        r = time_prefill(p, args, torch, dev, warm=True, split=False)
         t[nch], seg[nch] = r["us_per_call"], r["segment_chunks"]
-    unsplit = all(seg[n] is None or seg[n] >= n for n in (3, 4))
-    return {"us": round(t[4] - t[3], 3) if unsplit else None, "us_per_call_3_chunks": t[3],
-            "us_per_call_4_chunks": t[4], "segment_chunks": [seg[3], seg[4]],
-            "method": "t(1 x 256 tokens) - t(1 x 192 tokens), warm cache, neither split"}
+    unsplit = all(seg[n] is None or seg[n] >= n for n in (8, 9))
+    return {"us": round(t[9] - t[8], 3) if unsplit else None, "us_per_call_8_chunks": t[8],
+            "us_per_call_9_chunks": t[9], "segment_chunks": [seg[8], seg[9]],
+            "method": "t(1 x 576 tokens) - t(1 x 512 tokens), warm cache, neither split"}
 
 
 # Prefill workloads beside the three configurations: configuration 3 with

@@ -14,6 +14,11 @@
 // (solution/triton/kernel.py:421-425) divides by G.
 //
 // Launches, all on the caller's stream, no host synchronisation:
+//   direct   : calls of at most four chunks run as this launch alone, one
+//              work-group per (sequence, v-head).
+//   mixed    : calls of few, mostly short sequences: the direct path for the
+//              sequences of at most four chunks, and beside it the plan and the
+//              prepass of the longer ones.
 //   plan     : (batches of more than 512 sequences only) 1 work-group: chunk
 //              records, segment length and work lists from cu_seqlens.  For
 //              smaller batches work-group 0 of the prepass plans and the other
@@ -34,9 +39,13 @@
 //              in MFMA registers.  Short sequences run one work-group per
 //              (sequence, v-head).  Chunk operands are copied from global
 //              memory straight into double-buffered LDS.
+//   wide     : in place of the consumer for batches of many sequences: one
+//              work-group of four waves per (run or short sequence, v-head),
+//              two per CU.
 //   finish   : the state before each segment (S_{j+1} = S_j M_j + B_j), the
 //              output correction O = O0 + OI S_j^T for segments >= 1, and the
-//              final state of multi-segment sequences.
+//              final state of multi-segment sequences.  Not launched when no
+//              sequence can take M-runs.
 //
 // Precision policy (fp32 accumulation everywhere): K, Q, V are bf16 inputs, so
 // their products are exact.  S enters Q S^T as a single bf16 and K S^T as a
@@ -3740,8 +3749,8 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
 //        publishes S_j as bf16 correction fragments; S_nseg goes to new_state.
 //   a correction block (segment j >= 1, v-head, a few chunks whose OI was
 //        formed), as the consumer's M-run appended it: waits until S_j is
-//        published (S_1 is the first segment's slot itself), then out = bf16(O0 + OI S_j^T), wave w taking
-//        16-token tile w of each chunk (the other chunks keep O0).
+//        published (S_1 is the first segment's slot itself), then
+//        out = bf16(O0 + OI S_j^T) for its chunks (the others keep O0).
 // Scan items precede every block in the queue and wait for nothing, so a block
 // only ever waits for items that running groups hold, whatever share of the
 // grid is resident.
