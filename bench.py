@@ -493,7 +493,7 @@ def main():
         ach = total_b / (step_ms * 1e-3) / 1e9
         result["roofline"] = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBPS,
                               "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBPS, 4),
-                              "traffic": traffic, "kernel": "gdn::decode_kernel<32>",
+                              "traffic": traffic, "kernel": "gdn::decode_kernel<32, true>",
                               "algorithmic_bytes_per_launch": total_b,
                               "mean_launch_us": round(step_ms * 1e3, 3)}
         # decode B = 1 (configuration 0), launch-latency bound

@@ -32,8 +32,23 @@ __device__ __forceinline__ void reduce_scatter_step(float* v, bool upper) {
   }
 }
 
+// log_decay with both sides of the softplus threshold formed and selected, so
+// that no load can be moved behind a branch.
+__device__ __forceinline__ float log_decay_flat(float A_log, float a, float dt_bias) {
+  const float x = a + dt_bias;
+  const float y = log1pf(expf(x > 20.0f ? 0.0f : x));
+  return -expf(A_log) * (x > 20.0f ? x : y);
+}
+
 // ROWS rows of one head per wave (ROWS/2 per half-wave).
-template <int ROWS>
+// kEarly: every load is requested in one memory round trip.  Left to the
+// compiler, b is loaded behind the softplus branch and v behind the reduction,
+// two more dependent round trips: what bounds small batches.  With 16 rows the
+// few small loads go first (a wave's loads return in order), so that the gates
+// are formed while the state is in flight; with 32 rows, where the state's
+// bandwidth matters, they follow it.  24 captured steps of 4 sequences 84.4 ->
+// 74.5 us; the sizes and both sides are at the dispatch.
+template <int ROWS, bool kEarly>
 __global__ __launch_bounds__(64) void decode_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, const float* __restrict__ state,
@@ -57,25 +72,53 @@ __global__ __launch_bounds__(64) void decode_kernel(
   const int hq = h / kGva;
   const int row0 = vt * ROWS + half * NL;
 
-  // ---- issue the state loads first (the only large traffic) ----
+  constexpr bool kSmallFirst = kEarly && ROWS == 16;
+  constexpr int kShift = (NV == 32) ? 0 : 1;
+  const int idx = lam >> kShift;          // value index held by this lane after the reduction
+  const int row_i = idx & (NL - 1);       // row within the half
+  const bool is_q = idx >= NL;
+
+  // ---- the state (the only large traffic) ----
   // Non-temporal: every state byte is read exactly once, so the loads stream
   // instead of allocating in L2 / MALL (measured on MI355X at B = 64: 11.84 ->
   // 10.84 us per step with plain vs non-temporal loads, same outputs).
   const float* src = state + static_cast<size_t>(nh) * kHeadState + row0 * kDim + lam * 4;
   f32x4 s[NL];
+  auto load_state = [&] {
 #pragma unroll
-  for (int i = 0; i < NL; ++i) s[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + i * kDim));
+    for (int i = 0; i < NL; ++i) s[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + i * kDim));
+  };
+  if constexpr (!kSmallFirst) load_state();
+  if constexpr (kEarly && !kSmallFirst) __builtin_amdgcn_sched_barrier(0);
 
-  // ---- q, k for this lane's 4 columns; gates for this (n, h) ----
+  // ---- q, k for this lane's 4 columns; gates for this (n, h); the v value of
+  // the row this lane holds after the reduction ----
   const size_t qk_off = (static_cast<size_t>(n) * kQKHeads + hq) * kDim + lam * 4;
+  const size_t v_off = static_cast<size_t>(nh) * kDim + row0 + row_i;
   const uint2 kraw = *reinterpret_cast<const uint2*>(k + qk_off);
   const uint2 qraw = *reinterpret_cast<const uint2*>(q + qk_off);
+  float g, beta;
+  uint16_t vraw = 0;
+  if constexpr (kEarly) {
+    const uint16_t araw = a[nh], braw = b[nh];
+    vraw = v[v_off];
+    const float alog = A_log[h], dtb = dt_bias[h];
+    if constexpr (kSmallFirst) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_state();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    g = expf(log_decay_flat(alog, bf2f(araw), dtb));
+    beta = sigmoidf(bf2f(braw));
+  } else {
+    g = expf(log_decay(A_log[h], bf2f(a[nh]), dt_bias[h]));
+    beta = sigmoidf(bf2f(b[nh]));
+  }
   const float kc[4] = {bf_lo(kraw.x), bf_hi(kraw.x), bf_lo(kraw.y), bf_hi(kraw.y)};
   const float qc[4] = {bf_lo(qraw.x), bf_hi(qraw.x), bf_lo(qraw.y), bf_hi(qraw.y)};
-  const float g = expf(log_decay(A_log[h], bf2f(a[nh]), dt_bias[h]));
-  const float beta = sigmoidf(bf2f(b[nh]));
   float kq = kc[0] * qc[0] + kc[1] * qc[1] + kc[2] * qc[2] + kc[3] * qc[3];
   kq = half_wave_allreduce(kq);
+  if constexpr (kSmallFirst) __builtin_amdgcn_sched_barrier(0);   // formed before the state is waited for
 
   // ---- partial row dots: vals[i] = S_i . k, vals[NL + i] = S_i . q ----
   float vals[NV];
@@ -97,13 +140,8 @@ __global__ __launch_bounds__(64) void decode_kernel(
   } else {
     red = xor_sum<1>(vals[0]);
   }
-  constexpr int kShift = (NV == 32) ? 0 : 1;
-  const int idx = lam >> kShift;          // value index held by this lane
-  const int row_i = idx & (NL - 1);       // row within the half
-  const bool is_q = idx >= NL;
-
   // p-lanes: delta_i = beta (v_i - g p_i); q-lanes fetch it from lane lam ^ 16
-  const float vrow = bf2f(v[static_cast<size_t>(nh) * kDim + row0 + row_i]);
+  const float vrow = bf2f(kEarly ? vraw : v[v_off]);
   const float delta = beta * (vrow - g * red);
   const float delta_x = xor_lane<16>(delta);
   if (!is_q && ((lam & kShift) == 0)) delta_lds[half][row_i] = delta;
@@ -149,7 +187,12 @@ extern "C" int gdn_decode_fwd(const void* q, const void* k, const void* v, const
   if ((reinterpret_cast<uintptr_t>(A_log) | reinterpret_cast<uintptr_t>(dt_bias)) & 3u) return GDN_ERR_UNALIGNED;
   if (state == new_state) return GDN_ERR_ALIASING;
   if (!(scale > 0.0f) && !(scale < 0.0f)) scale = 0.08838834764831845f;  // 0 / NaN -> 1/sqrt(128)
-  if (rows_per_wave == 0) rows_per_wave = (batch >= 16) ? 32 : 16;
+  // Rows per wave, us per step in captured steps over rotated buffers (16 rows
+  // early / 32 early / 32 late): batch 8: 3.57 / 4.29 / 4.11, 32: 6.40 / 7.49 /
+  // 7.02, 48: 10.59 / 8.79 / 8.95, 64: 13.58 / 11.12 / 11.34, 96: 19.05 / 19.52 /
+  // 17.79, 128: 24.60 / 24.79 / 24.46, 192: 35.14 / 36.18 / 35.62, 256: 45.52 /
+  // 46.94 / 46.65.
+  if (rows_per_wave == 0) rows_per_wave = (batch <= 32 || batch >= 160) ? 16 : 32;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const auto* qb = static_cast<const uint16_t*>(q);
   const auto* kb = static_cast<const uint16_t*>(k);
@@ -161,12 +204,15 @@ extern "C" int gdn_decode_fwd(const void* q, const void* k, const void* v, const
   if (rows_per_wave == 32) {
     const long grid = heads * (kDim / 32);
     if (grid > 0x7fffffffL) return GDN_ERR_INVALID_ARGUMENT;
-    decode_kernel<32><<<dim3(static_cast<unsigned>(grid)), dim3(64), 0, st>>>(
-        qb, kb, vb, state, A_log, ab, dt_bias, bb, scale, ob, new_state);
+    const dim3 gr(static_cast<unsigned>(grid));
+    if (batch <= 64)
+      decode_kernel<32, true><<<gr, dim3(64), 0, st>>>(qb, kb, vb, state, A_log, ab, dt_bias, bb, scale, ob, new_state);
+    else
+      decode_kernel<32, false><<<gr, dim3(64), 0, st>>>(qb, kb, vb, state, A_log, ab, dt_bias, bb, scale, ob, new_state);
   } else if (rows_per_wave == 16) {
     const long grid = heads * (kDim / 16);
     if (grid > 0x7fffffffL) return GDN_ERR_INVALID_ARGUMENT;
-    decode_kernel<16><<<dim3(static_cast<unsigned>(grid)), dim3(64), 0, st>>>(
+    decode_kernel<16, true><<<dim3(static_cast<unsigned>(grid)), dim3(64), 0, st>>>(
         qb, kb, vb, state, A_log, ab, dt_bias, bb, scale, ob, new_state);
   } else {
     return GDN_ERR_INVALID_ARGUMENT;

@@ -167,3 +167,13 @@ def test_decode_random_steps(gpu, seed):
     o_ref, s_ref = decode_ref(*d.args())
     out, ns = _run(d, gpu, rows_per_wave=rows)
     assert_parity(out, ns, o_ref, s_ref, label)
+
+
+# The automatic choice of rows per wave and of the load order changes at batches
+# of 33, 65 and 160: both sides of each edge, checked against the oracle.
+@pytest.mark.parametrize("batch", [32, 33, 64, 65, 159, 160])
+def test_decode_dispatch_edges(gpu, batch):
+    d = decode_inputs(batch, seed=300 + batch)
+    o_ref, s_ref = decode_ref(*d.args())
+    out, ns = _run(d, gpu)
+    assert_parity(out, ns, o_ref, s_ref, f"decode B={batch}, automatic rows")
