@@ -3779,6 +3779,11 @@ constexpr int kFinRows = 32;                      // value rows of a scan item
 constexpr int kFinParts = kDim / kFinRows;        // scan items per (sequence, v-head)
 constexpr int kFinReady = kFinParts * (kFinThreads / 64);   // waves that publish a segment's state
 constexpr int kScanAhead = 3;                     // steps between a step's loads and their use
+// Polls of a block's wait, at least 512 cycles each: about a second.  A block
+// waits for one scan at most, and the longest scan (kMaxSlots steps) takes 14
+// ms, so the bound is met only where another call on the same workspace has
+// overwritten the counts: its results are then undefined, but it ends.
+constexpr int kFinSpins = 1 << 22;
 constexpr int kSc01 = 1 | 16;                     // cache policy bits sc0 and sc1
 
 union FinishLds {
@@ -4025,8 +4030,10 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
     } else {
       if (tid == 0) {
         int* rd = seg_ready(slotm, g0, j, h);
-        while (__hip_atomic_load(rd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < kFinReady)
+        for (int i = 0; i < kFinSpins; ++i) {
+          if (__hip_atomic_load(rd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= kFinReady) break;
           __builtin_amdgcn_s_sleep(8);
+        }
       }
       __syncthreads();
       // S_j's fragments, published over the slot of segment j - 1: part p's 8 KB
