@@ -3769,7 +3769,13 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
 // B_j).  Wave w forms k tile w of both row tiles: as a B operand in permuted
 // order they are half of depth chunk w / 2 of the next step, so the waves trade
 // 8-byte halves of fragments through LDS.  The correction multiplies OI (bf16)
-// by S as a single bf16, as the chunk recurrence does in Q S^T.
+// by S as hi / lo, where the chunk recurrence's Q S^T takes a single bf16: a
+// corrected row carries two roundings more (OI's and O0's), and the more
+// segments, the more such rows.  Relative output error against a 32-bit
+// recurrence, near-1 decay, S single -> hi / lo: 1 x 2000 tokens 3.19e-3 ->
+// 3.02e-3, 2 x 1000 3.15e-3 -> 2.99e-3, 1 x 32768 2.86e-3 -> 2.84e-3; 0.5 to
+// 1 us of a call of up to 8,192 tokens (1 x 1000: 42.5 -> 43.0 us), nothing
+// at 1 x 32768 (242 -> 240).
 //
 // Published data crosses XCDs within the launch: it is stored and loaded past
 // the XCD's own L2 (sc0 sc1), and the count of finished waves is raised only
@@ -3788,9 +3794,9 @@ constexpr int kSc01 = 1 | 16;                     // cache policy bits sc0 and s
 
 union FinishLds {
   u32x4 x[2][2][4][2][64];   // scan: [parity][row tile][depth chunk][hi / lo][lane]
-  // block: S as A fragments: [v-tile][d][lane], slot s of v-tile 2 p + e =
-  // S[32 p + wide_row(e, l16)][32 d + 8 lg + s]
-  u32x4 frag[8][4][64];
+  // block: S as A fragments: [hi / lo][v-tile][d][lane], slot s of v-tile
+  // 2 p + e = S[32 p + wide_row(e, l16)][32 d + 8 lg + s]
+  u32x4 frag[2][8][4][64];
 };
 
 // Operands of scan step i: M_i^T fragments of the wave's k tile and B_i (the
@@ -3846,13 +3852,16 @@ __device__ __forceinline__ void scan_item(FinishLds& sm, const int4& me, int h, 
     constexpr bool kLong = decltype(LC)::value;
     const int P = j & 1;
     // S_j into LDS: half e = w & 1 of the fragments of depth chunk w / 2
+    u32x2 sx[2][2];   // [row tile][hi / lo]
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
       const uint32_t h0 = pack_bf2(s[rt][0], s[rt][1]), h1 = pack_bf2(s[rt][2], s[rt][3]);
-      const u32x2 lo = {pack_bf2(s[rt][0] - bf_lo(h0), s[rt][1] - bf_hi(h0)),
+      sx[rt][0] = u32x2{h0, h1};
+      sx[rt][1] = u32x2{pack_bf2(s[rt][0] - bf_lo(h0), s[rt][1] - bf_hi(h0)),
                         pack_bf2(s[rt][2] - bf_lo(h1), s[rt][3] - bf_hi(h1))};
-      *(reinterpret_cast<u32x2*>(&sm.x[P][rt][w >> 1][0][lane]) + (w & 1)) = u32x2{h0, h1};
-      *(reinterpret_cast<u32x2*>(&sm.x[P][rt][w >> 1][1][lane]) + (w & 1)) = lo;
+#pragma unroll
+      for (int hl = 0; hl < 2; ++hl)
+        *(reinterpret_cast<u32x2*>(&sm.x[P][rt][w >> 1][hl][lane]) + (w & 1)) = sx[rt][hl];
     }
     // this step's operands; the state published kScanAhead steps ago, issued
     // before them, is out as well
@@ -3861,21 +3870,28 @@ __device__ __forceinline__ void scan_item(FinishLds& sm, const int4& me, int h, 
                  : "memory");
     if (kLong && j > kScanAhead) raise(j - kScanAhead);
     lds_barrier();   // S_j in LDS; every wave holds its rows of B_{j-1}, whose place S_j takes
-    // publish S_j: natural-order A fragments, 8 bytes per row tile.  Value row
-    // 16 rt + l16 of the part goes to row i of v-tile e, 16 rt + l16 =
-    // wide_row(e, i), so that a block's lanes hold eight consecutive columns
-    // (S_1 is its slot's state itself, which the blocks of segment 1 read as it
-    // is: its fragments go unused to the second half of the counts' area)
-    auto* pub = j > 1 ? reinterpret_cast<unsigned long long*>(slotb + head(j - 1) * kHeadState + r0 * kDim)
-                      : reinterpret_cast<unsigned long long*>(slotm + head(0) * kMSlotElems + kMSlotElems / 2) +
-                            part * (kFinRows * kDim / 4);
+    // publish S_j: natural-order A fragments, 8 KB of hi and 8 KB of lo, 8 bytes
+    // of each per row tile.  Value row 16 rt + l16 of the part goes to row i of
+    // v-tile e, 16 rt + l16 = wide_row(e, i), so that a block's lanes hold eight
+    // consecutive columns (S_1 is its slot's state itself, which the blocks of
+    // segment 1 read as it is: its fragments go unused to the second half of the
+    // counts' area, lo over hi)
+    constexpr int kPubBytes = kFinRows * kDim * 2;   // of hi or lo
+    const __amdgpu_buffer_rsrc_t pub =
+        j > 1 ? buf_rsrc(slotb + head(j - 1) * kHeadState + r0 * kDim, 2 * kPubBytes)
+              : buf_rsrc(slotm + head(0) * kMSlotElems + kMSlotElems / 2 + part * (kPubBytes / 2), kPubBytes);
+    const int lo_at = j > 1 ? kPubBytes : 0;
+    const uint32_t at =
+        ((((l16 >> 2) & 1) * 4 + (w >> 1)) * 64 + 16 * (2 * (w & 1) + (lg >> 1)) + 4 * (l16 >> 3) + (l16 & 3)) * 16 +
+        8 * (lg & 1);
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      const u32x2 pk = {pack_bf2(s[rt][0], s[rt][1]), pack_bf2(s[rt][2], s[rt][3])};
-      const int e = (l16 >> 2) & 1, i = 4 * (2 * rt + (l16 >> 3)) + (l16 & 3);
-      __hip_atomic_store(pub + ((e * 4 + (w >> 1)) * 64 + 16 * (2 * (w & 1) + (lg >> 1)) + i) * 2 + (lg & 1),
-                         __builtin_bit_cast(unsigned long long, pk), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int hl = 0; hl < 2; ++hl)
+        __builtin_amdgcn_raw_buffer_store_b64(sx[rt][hl], pub, at + 128 * rt, hl * lo_at, kSc01);
+    // the loads below stay behind these stores (raise relies on that order)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     if (!kLong && j > 1) {
       __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
       asm volatile("" ::: "memory");
@@ -4018,14 +4034,18 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
     const int my = first + (w >> 2);
     if (my < last) load_chunk(my);
     const float* slot = slotb + (static_cast<size_t>(sg.w) * kVHeads + h) * kHeadState;
-    u32x4 fr[4];   // wave w brings v-tile w's fragments
+    u32x4 fr[2][4];   // [hi / lo]: wave w brings v-tile w's fragments
     if (j == 1) {
       // S_1: the first segment's state, as its run left it
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
         const float* sp = slot + (32 * (w >> 1) + wide_row(w & 1, l16)) * kDim + 32 * d + 8 * lg;
         const f32x4 x0 = *reinterpret_cast<const f32x4*>(sp), x1 = *reinterpret_cast<const f32x4*>(sp + 4);
-        fr[d] = u32x4{pack_bf2(x0[0], x0[1]), pack_bf2(x0[2], x0[3]), pack_bf2(x1[0], x1[1]), pack_bf2(x1[2], x1[3])};
+        const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+        bf16x8 hi, lo;
+        split_frag(x, hi, lo);
+        fr[0][d] = __builtin_bit_cast(u32x4, hi);
+        fr[1][d] = __builtin_bit_cast(u32x4, lo);
       }
     } else {
       if (tid == 0) {
@@ -4036,19 +4056,24 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
         }
       }
       __syncthreads();
-      // S_j's fragments, published over the slot of segment j - 1: part p's 8 KB
+      // S_j's fragments, published over the slot of segment j - 1: part p's 16 KB
       // (v-tiles 2 p, 2 p + 1) at its rows' place
       const __amdgpu_buffer_rsrc_t src = buf_rsrc(slot, kHeadState * 4);
 #pragma unroll
-      for (int d = 0; d < 4; ++d)
-        fr[d] = __builtin_amdgcn_raw_buffer_load_b128(
-            src, (w >> 1) * (kFinRows * kDim * 4) + (((w & 1) * 4 + d) * 64 + lane) * 16, 0, kSc01);
+      for (int hl = 0; hl < 2; ++hl)
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          fr[hl][d] = __builtin_amdgcn_raw_buffer_load_b128(
+              src, (w >> 1) * (kFinRows * kDim * 4) + (((2 * hl + (w & 1)) * 4 + d) * 64 + lane) * 16, 0, kSc01);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sm.frag[w][e][lane] = fr[e];
+    for (int hl = 0; hl < 2; ++hl)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sm.frag[hl][w][e][lane] = fr[hl][e];
     __syncthreads();
     for (int ci = my; ci < last; ci += 2) {
       if (ci > my) load_chunk(ci);
+      const int ln = opaque_lane(lane);   // the lo fragments are read per chunk (both kinds would not fit in registers)
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         f32x4 acc[2];
@@ -4056,8 +4081,10 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
         for (int e = 0; e < 2; ++e) {
           acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int d = 0; d < 4; ++d)
-            acc[e] = mfma16(__builtin_bit_cast(bf16x8, sm.frag[2 * p + e][d][lane]), b[d], acc[e]);
+          for (int hl = 1; hl >= 0; --hl)   // the small terms first
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+              acc[e] = mfma16(__builtin_bit_cast(bf16x8, sm.frag[hl][2 * p + e][d][hl ? ln : lane]), b[d], acc[e]);
         }
         const u32x4 o = o0[p];
         u32x4 o1;
