@@ -1705,7 +1705,12 @@ __device__ __forceinline__ void chunk_by_tiles(int c, F&& f) {
 //         (zero columns of Tb, zero rows of Delta); their products are not
 //         formed (their R rows count as zero, also for R's range scale), and
 //         the state update skips the second 32-token depth half when NB <= 2.
-template <int NB>
+//   kResidue: in slowly decaying chunks the state's rounding residue enters X
+//         too (see chain_chunk).  It keeps roundings from accumulating over the
+//         chunks of a sequence, so sequences of one chunk go without: it adds
+//         3% to their calls (24 sequences of 70 tokens, near-1 decay: 32.8
+//         with it, 32.2 us without) for a state error of 3.05e-4 against 3.06e-4.
+template <int NB, bool kResidue>
 __device__ __forceinline__ void consumer_chunk(const ChunkLds& sm, int c, f32x4 (&st)[8], int w,
                                                int lane, float scale, __amdgpu_buffer_rsrc_t orc,
                                                uint32_t ocol) {
@@ -1755,7 +1760,7 @@ __device__ __forceinline__ void consumer_chunk(const ChunkLds& sm, int c, f32x4 
     }
   }
 
-  if (sm.gt[kBoundAt] > kHiLoBoundLog2) {   // uniform: slow decay (see chain_chunk)
+  if (kResidue && sm.gt[kBoundAt] > kHiLoBoundLog2) {   // uniform
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       float x[8];
@@ -1984,7 +1989,7 @@ __device__ __forceinline__ void full_head_items(
       const ChunkLds lds = {sm.ks[P], sm.qs[P], sm.vs[P], sm.frag[P][0], sm.frag[P][1], sm.gt[P]};
       // all four tiles: batches of many short sequences are bound by their
       // state traffic, and one body keeps the loop's code small
-      consumer_chunk<4>(lds, cur.c, st, w, lane, scale, orc, ocol);
+      consumer_chunk<4, false>(lds, cur.c, st, w, lane, scale, orc, ocol);
     }
     // an empty sequence leaves new_state zero (st is zero); a chunk without a
     // record (malformed cu_seqlens) passes the state through.  State bytes are
@@ -2174,7 +2179,7 @@ __device__ __forceinline__ void direct_group(
   auto chunk = [&](int j, int i, int P, auto NBC) __attribute__((always_inline)) {
     const ChunkLds lds = {sm.ks[P], sm.qs[P], sm.vs[P], sm.tb[i + 1], sm.tb[i], sm.gt[i]};
     const int lane = opaque_lane(tid);
-    consumer_chunk<decltype(NBC)::value>(lds, chunk_len(j), st, w, lane, scale, out_rsrc(j),
+    consumer_chunk<decltype(NBC)::value, true>(lds, chunk_len(j), st, w, lane, scale, out_rsrc(j),
                                          2u * static_cast<uint32_t>(vcol + 4 * (lane >> 4)));
   };
   int pl = 0;   // the last chunk's buffer
