@@ -1359,7 +1359,10 @@ __device__ __forceinline__ void prepass_items(
     __syncthreads();
     total = min(sm.seq.incl[64 * nblk - 1], R);
   } else {
-    total = min(rec_start[num_seqs], R);
+    // written by the plan launch, constant here.  Through the constant address
+    // space, as the compiler merges this read with the LDS one above into one
+    // of either memory otherwise, which waits for every load in flight.
+    total = min(((const __attribute__((address_space(4))) int*)rec_start)[num_seqs], R);
   }
 
   // items: (record r, v-head h) = 8 r + h, or (record r, q/k head hq) = 4 r + hq
