@@ -134,19 +134,14 @@ __host__ __device__ inline long long max_segments(long long tokens) {
   return tokens / (32 * kMinSegChunks) + 1;
 }
 
-// lists: header, multi-segment entries, later-segment table, runs (two int4
-// each), short sequences.  Everything a kernel needs about one work item sits
+// lists: header, multi-segment entries, runs (two int4 each), short sequences.  Everything a kernel needs about one work item sits
 // in one entry, so an item costs one dependent load before its data.
 //   hdr[0] runs, [1] short sequences, [2] segment length L (chunks),
-//   [3] multi-segment sequences, [4] segments >= 1 over all sequences,
-//   [5] 1 when the batch uses warm-up segments (no M-runs, no finish work),
+//   [3] multi-segment sequences (none when the batch uses warm-up segments),
 //   [8] split-consumer work queue (items claimed past each group's first),
 //   [9] correction blocks appended by the consumer's M-runs, [10] finish queue,
 //   [11] most segments of any sequence
 //   multi[e]   = (seq, first slot, segments, 0)
-//   segs[i]    = (first token lo, hi, tokens in the segment | j << 17, slot of
-//                 segment j - 1) for every segment j >= 1 (L <= 1024 chunks:
-//                 at most 65536 tokens)
 //   runs[2i]   = (seq, flags | tokens of the run's last chunk << 8 | segment
 //                 j << 16, final-state slot or -1 for new_state, first record)
 //   runs[2i+1] = (first token lo, hi, chunks with records, chunks)
@@ -200,7 +195,6 @@ __host__ __device__ inline long long max_runs(int num_seqs, long long gcap) { re
 struct ListView {
   int* hdr;
   int4* multi;
-  int4* segs;
   int4* runs;
   int4* shorts;
 };
@@ -209,15 +203,13 @@ __host__ __device__ inline ListView list_view(int* lists, int num_seqs, long lon
   ListView v;
   v.hdr = lists;
   v.multi = reinterpret_cast<int4*>(lists + kListHdr);
-  v.segs = v.multi + num_seqs;
-  v.runs = v.segs + gcap;
+  v.runs = v.multi + num_seqs;
   v.shorts = v.runs + 2 * max_runs(num_seqs, gcap);
   return v;
 }
 
 __host__ __device__ inline size_t list_ints(int num_seqs, long long gcap) {
-  return kListHdr + 4 * static_cast<size_t>(num_seqs) + 4 * static_cast<size_t>(gcap) +
-         8 * static_cast<size_t>(max_runs(num_seqs, gcap)) + 4 * static_cast<size_t>(num_seqs);
+  return kListHdr + 4 * static_cast<size_t>(num_seqs) + 8 * static_cast<size_t>(max_runs(num_seqs, gcap)) + 4 * static_cast<size_t>(num_seqs);
 }
 
 // ---- workspace layout -------------------------------------------------------
@@ -231,7 +223,7 @@ struct WsLayout {
   size_t slotm_off;    // u16  [G][8][kMSlotElems] M_j^T fragments
   size_t oi_off;       // u16  [T][8][128]       M-run outputs OI (rows of segments >= 1)
   size_t mval_off;     // i32  [G][8]            M-run chunks whose outputs OI were formed | kMNegligible
-  size_t fix_off;      // i32x4[8 R][2]          correction blocks (segs entry; v-head, first, last chunk)
+  size_t fix_off;      // i32x4[8 R][2]          correction blocks (see split_items)
   size_t total;
 };
 
@@ -493,8 +485,7 @@ constexpr int kPlanScratch = kPsMisc + 4;
 // i owning a contiguous range of sequences: rec_start (chunk record of each
 // sequence's first chunk), the segment length, and the work lists of the
 // split consumer (runs, longest first), the full-head consumer (short
-// sequences), the scan (multi-segment sequences) and the correction (segments
-// >= 1).
+// sequences) and the scan (multi-segment sequences).
 //
 // Segment length: for each candidate L an estimate of the split consumer's
 // critical path in chunk steps, the smallest winning (ties to the longer L).
@@ -732,8 +723,6 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       lv.hdr[1] = tot[1];
       lv.hdr[2] = L;
       lv.hdr[3] = tot[2];
-      lv.hdr[4] = tot[3] - tot[2];
-      lv.hdr[5] = warm ? 1 : 0;
       rec_start[num_seqs] = min(tot[0], R);
     }
   }
@@ -761,14 +750,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     }
     const int g0 = p.multi ? gb : 0;
     if (p.multi) {
-      // later-segment table: entries gb - mp .. (one per segment >= 1)
       lv.multi[mp] = make_int4(s, gb, p.nseg, 0);
-      for (int j = 1; j < p.nseg; ++j) {
-        const long long c0 = t0 + static_cast<long long>(j) * L * kChunk;
-        const int tok = static_cast<int>(min(t1 - c0, static_cast<long long>(L) * kChunk));
-        lv.segs[gb - mp + j - 1] = make_int4(static_cast<int>(c0 & 0xffffffffLL), static_cast<int>(c0 >> 32),
-                                             tok | (j << 17), gb + j - 1);
-      }
       ++mp;
       gb += p.nseg;
     }
@@ -2934,7 +2916,9 @@ __device__ __forceinline__ void split_items(
   // during its first chunk (the atomic returns before that chunk's closing
   // barrier, with the next chunk's copies), and fills them at its end; blocks
   // past `formed` are left empty.  The finish then takes a block with a single
-  // descriptor load.  The entry repeats the later-segment table's.
+  // descriptor load: (first token of the segment lo, hi, its tokens | j << 17
+  // (L <= 1024 chunks: at most 65536 tokens), slot of segment j - 1) and
+  // (v-head, first chunk, end chunk, 0).
   int fix_pos = 0;
 
   // An M-run stops once the bound of its map falls below kNegligibleLog2: its
