@@ -3832,8 +3832,7 @@ __device__ __forceinline__ void scan_item(FinishLds& sm, const int4& me, int h, 
         o.m[d][hl] = *reinterpret_cast<const bf16x8*>(mp + ((w * 4 + d) * 2 + hl) * kFragTile);
     scan_load_b(slotb + hd * kHeadState, r0, w, lane, o.b);
   };
-#pragma unroll
-  for (int k = 0; k < kScanAhead; ++k) load_ops(1 + k, op[k]);
+  load_ops(1, op[0]);
   auto raise = [&](int j) {   // this wave's share of S_j is out
     if (lane == 0)
       __hip_atomic_fetch_add(seg_ready(slotm, g0, j, h), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -3908,7 +3907,16 @@ __device__ __forceinline__ void scan_item(FinishLds& sm, const int4& me, int h, 
   };
   constexpr int kBlock = 64 / kScanAhead * kScanAhead;   // steps per read_neg
   const bool lng = nseg > kScanAhead + 1;
-  if (!lng) {
+  if (nseg > 2) {
+#pragma unroll
+    for (int k = 1; k < kScanAhead; ++k) load_ops(1 + k, op[k]);
+  }
+  if (nseg == 2) {
+    // a single step, with no other step's operands in flight (a group reads 80
+    // KB per step)
+    read_neg();
+    step(1, op[0], std::false_type{});
+  } else if (!lng) {
     read_neg();
 #pragma unroll
     for (int k = 0; k < kScanAhead; ++k)
@@ -3960,11 +3968,13 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
   if (nmulti + ncorr == 0) return;
   // The next claim is requested while an item is worked on.  A group that waits
   // in a block holds at most another block: claims only grow.  Where no sequence
-  // has a third segment nothing waits, and every group starts with its own
-  // item (256 first claims cost about 1.5 us) and scans two parts at a time (at
-  // most one round of items for a few sequences).
+  // has a third segment nothing waits, and every group starts with its own item
+  // (256 first claims cost about 1.5 us).  It scans two parts at a time if the
+  // items would not be one round otherwise (the second part's loads follow the
+  // first part's stores: 1 x 1000 tokens in two segments 12.5 us, one part each
+  // 8.4).
   const bool waits = lv.hdr[11] > 2;
-  const int parts = waits ? 1 : 2;
+  const int parts = waits || nmulti * kVHeads * kFinParts + ncorr <= static_cast<int>(gridDim.x) ? 1 : 2;
   const int nscan = nmulti * kVHeads * (kFinParts / parts);
   const int nitem = ncorr + nscan;
   const int base = waits ? 0 : static_cast<int>(gridDim.x);
