@@ -57,6 +57,7 @@
 // bf16 hi+lo pair; Aqk Delta (output only) is single bf16.  The fp32 state
 // never leaves registers between chunks.
 #include "gdn_common.h"
+#include "gdn_plan_model.h"
 #include <algorithm>
 #include <type_traits>
 #include "../../include/gdn_mi355x.h"
@@ -473,7 +474,7 @@ __device__ __forceinline__ SeqPlan seq_plan(int nch, int L, bool warm) {
 }
 
 // Scratch ints used by plan_batch.
-constexpr int kPsVals = 3 * kSegCands + 3;
+constexpr int kPsVals = 3 * kSegCands + 4;
 constexpr int kPsCand = 0;                                   // [waves][kPsVals]
 constexpr int kPsScan = kPsCand + (kPlanThreads / 64) * kPsVals;   // [waves][5]
 constexpr int kPsHist = kPsScan + (kPlanThreads / 64) * 5;
@@ -487,14 +488,9 @@ constexpr int kPlanScratch = kPsMisc + 4;
 // split consumer (runs, longest first), the full-head consumer (short
 // sequences) and the scan (multi-segment sequences).
 //
-// Segment length: for each candidate L an estimate of the split consumer's
-// critical path in chunk steps, the smallest winning (ties to the longer L).
-// With M-runs: max(L + o, (16 W(L) + 16 o runs(L)) / groups), W(L) = sum over
-// long sequences of (2 nch - min(nch, L)) chunk runs per (value half, v-head),
-// o the per-item overhead, plus about half a step per segment for the scan and
-// 1.5 for segmenting at all (and a scan term for slowly decaying heads).  With
-// warm-up runs: the runs' list schedule on groups / 16 machines (longest run
-// or balanced load plus a last-round tail; see the evaluation below).
+// Segment length: for each candidate L an estimate of the call's time, the
+// smallest winning (ties to the longer L): with M-runs plan_split_mrun_us, with
+// warm-up runs the runs' list schedule (see the evaluation below).
 // Candidates whose segments would not fit the workspace slots are skipped.
 // Returns the thread's first record index.  t0_first / t1_first: bounds of the
 // thread's first sequence when the caller already read them (t1_first < 0:
@@ -540,10 +536,13 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
   int A[kSegCands], B[kSegCands], C[kSegCands];
 #pragma unroll
   for (int i = 0; i < kSegCands; ++i) A[i] = B[i] = C[i] = 0;
-  int suml = 0, maxl = 0, nlong = 0;
+  int suml = 0, maxl = 0, nlong = 0, nshort = 0;
   for (int s = s_begin; s < s_end; ++s) {
     const int nch = chunks(s);
-    if (nch < kLongChunks) continue;
+    if (nch < kLongChunks) {
+      nshort += nch >= 0 ? 1 : 0;
+      continue;
+    }
     suml += nch;
     maxl = max(maxl, nch);
     ++nlong;
@@ -568,6 +567,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     maxl = wave_max0(maxl);
     nlong = wave_sum(nlong);
   }
+  nshort = wave_sum(nshort);
   if (lane == 0) {
     int* pw = ps + kPsCand + wv * kPsVals;
 #pragma unroll
@@ -579,6 +579,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     pw[3 * kSegCands] = suml;
     pw[3 * kSegCands + 1] = maxl;
     pw[3 * kSegCands + 2] = nlong;
+    pw[3 * kSegCands + 3] = nshort;
   }
   for (int i = tid; i < 2 * kBuckets; i += NT) ps[kPsHist + i] = 0;
   __syncthreads();
@@ -593,12 +594,9 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     const int wh = hb < kNegligibleLog2 ? 1 : (hb < 0.f ? static_cast<int>(ceilf(kNegligibleLog2 / hb)) : 1 << 20);
     const int w_est = wave_max0(min(wh, 1 << 20));
     const bool warm = w_est <= kWarmMaxChunks;
-    // lane i < kSegCands evaluates candidate i, in chunk steps of the split
-    // consumer: the longest run and the average work-group load (chunk runs
-    // plus a per-item overhead) bound the critical path; the scan adds half a
-    // step per segment and segmenting at all 1.5 steps.  The minimum over the
-    // lanes wins, ties to the longer segments.
-    float sl = 0.f, a = 0.f, runs = 0.f, nl = 0.f;
+    // lane i < kSegCands evaluates candidate i; the minimum over the lanes wins,
+    // ties to the longer segments
+    float sl = 0.f, a = 0.f, runs = 0.f, nl = 0.f, ns = 0.f;
     long long slots = 0;
     int ml = 0;
     const int ci = min(lane, kSegCands - 1);
@@ -607,6 +605,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       sl += static_cast<float>(pj[3 * kSegCands]);
       ml = max(ml, pj[3 * kSegCands + 1]);
       nl += static_cast<float>(pj[3 * kSegCands + 2]);
+      ns += static_cast<float>(pj[3 * kSegCands + 3]);
       a += static_cast<float>(pj[ci]);
       slots += pj[kSegCands + ci];
       runs += static_cast<float>(pj[2 * kSegCands + ci]);
@@ -637,27 +636,25 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       est = fmaxf(longest + kWarmItem, balanced + tail) + (nseg_max > 1 ? kSegmented : 0.f);
     } else {
       // M-run scheme: a later segment runs twice, its M-run per v-head only
-      // until the head's map is negligible (about wh chunks).  The same list
-      // schedule over all runs; the finish adds its scan (0.4 steps per segment
-      // of the longest sequence), the corrections (48 KB of traffic per
-      // corrected chunk and v-head) and 6 steps for having any.  Measured with
-      // forced lengths (mixed or near-1 gates, us per call at this estimate's
-      // choice / unsegmented): 1 x 1024 tokens 42 / 48, 1 x 8192 91 / 227,
-      // 1 x 32768 195 / 830; 32 x 256 50 unsegmented, 61 at L <= 10.
-      constexpr float kRunItem = 1.5f, kTailShare = 0.25f, kCorrShare = 0.04f, kScan = 0.4f, kFinish = 6.0f;
-      const float kMachines = static_cast<float>(kConsumerGroups / (wide ? 8 : 16));
+      // until the head's map is negligible (about wh chunks)
       float mfrac = 0.f;
 #pragma unroll
       for (int hh = 0; hh < kVHeads; ++hh)
         mfrac += static_cast<float>(min(__builtin_amdgcn_readlane(wh, hh), Lc)) / (kVHeads * static_cast<float>(Lc));
-      const float mwork = (sl - a) * mfrac;
-      const float longest = static_cast<float>(min(Lc, ml));
-      const float balanced = (sl + mwork + kRunItem * runs) / kMachines;
-      const float tail = runs > kMachines ? kTailShare * ((sl + mwork) / fmaxf(runs, 1.f) + kRunItem) : 0.f;
-      est = fmaxf(longest + kRunItem, balanced + tail) +
-            (nseg_max > 1 ? kScan * static_cast<float>(nseg_max - 1) + kFinish + kCorrShare * mwork : 0.f);
+      if (wide) {
+        constexpr float kRunItem = 1.5f, kTailShare = 0.25f, kCorrShare = 0.04f, kScan = 0.4f, kFinish = 6.0f;
+        const float kMachines = static_cast<float>(kConsumerGroups / 8);
+        const float mwork = (sl - a) * mfrac;
+        const float longest = static_cast<float>(min(Lc, ml));
+        const float balanced = (sl + mwork + kRunItem * runs) / kMachines;
+        const float tail = runs > kMachines ? kTailShare * ((sl + mwork) / fmaxf(runs, 1.f) + kRunItem) : 0.f;
+        est = fmaxf(longest + kRunItem, balanced + tail) +
+              (nseg_max > 1 ? kScan * static_cast<float>(nseg_max - 1) + kFinish + kCorrShare * mwork : 0.f);
+      } else {
+        est = plan_split_mrun_us(PlanStats{sl, a, 0.5f * (runs + nl), nl, ns, mfrac, ml, Lc});
+      }
     }
-    // key: estimate in 1/16 steps, then the longer candidate; invalid lanes hold
+    // key: estimate in 1/16, then the longer candidate; invalid lanes hold
     // the maximum.  No slot is written in the warm-up scheme, but the slot
     // bound still applies: the run table holds max_runs(N, gcap) = N + 2 gcap
     // runs, and with at most gcap later segments the runs (one per segment)
