@@ -39,9 +39,9 @@
 //              in MFMA registers.  Short sequences run one work-group per
 //              (sequence, v-head).  Chunk operands are copied from global
 //              memory straight into double-buffered LDS.
-//   wide     : in place of the consumer for batches of many sequences: one
-//              work-group of four waves per (run or short sequence, v-head),
-//              two per CU.
+//              Batches of more than 32 sequences may run on the wide consumer
+//              instead, as the planner decides: half a work-group of four waves
+//              per (run or short sequence, v-head), two such items per CU.
 //   finish   : the state before each segment (S_{j+1} = S_j M_j + B_j), the
 //              output correction O = O0 + OI S_j^T for segments >= 1, and the
 //              final state of multi-segment sequences.  Not launched when no
@@ -141,7 +141,7 @@ __host__ __device__ inline long long max_segments(long long tokens) {
 //   [3] multi-segment sequences (none when the batch uses warm-up segments),
 //   [8] split-consumer work queue (items claimed past each group's first),
 //   [9] correction blocks appended by the consumer's M-runs, [10] finish queue,
-//   [11] most segments of any sequence
+//   [11] most segments of any sequence, [12] the wide consumer runs the call
 //   multi[e]   = (seq, first slot, segments, 0)
 //   runs[2i]   = (seq, flags | tokens of the run's last chunk << 8 | segment
 //                 j << 16, final-state slot or -1 for new_state, first record)
@@ -480,7 +480,7 @@ constexpr int kPsScan = kPsCand + (kPlanThreads / 64) * kPsVals;   // [waves][5]
 constexpr int kPsHist = kPsScan + (kPlanThreads / 64) * 5;
 constexpr int kPsCur = kPsHist + kBuckets;
 constexpr int kPsMisc = kPsCur + kBuckets;
-constexpr int kPlanScratch = kPsMisc + 4;
+constexpr int kPlanScratch = kPsMisc + 8;
 
 // Plans the call for the whole batch with one work-group of NT threads, thread
 // i owning a contiguous range of sequences: rec_start (chunk record of each
@@ -489,8 +489,8 @@ constexpr int kPlanScratch = kPsMisc + 4;
 // sequences) and the scan (multi-segment sequences).
 //
 // Segment length: for each candidate L an estimate of the call's time, the
-// smallest winning (ties to the longer L): with M-runs plan_split_mrun_us, with
-// warm-up runs the runs' list schedule (see the evaluation below).
+// smallest winning (ties to the longer L).  may_wide: for either consumer, whose
+// choice goes to the header too.
 // Candidates whose segments would not fit the workspace slots are skipped.
 // Returns the thread's first record index.  t0_first / t1_first: bounds of the
 // thread's first sequence when the caller already read them (t1_first < 0:
@@ -498,7 +498,7 @@ constexpr int kPlanScratch = kPsMisc + 4;
 template <int NT>
 __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, long long T, int R, int gcap,
                           const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-                          int* __restrict__ rec_start, int* __restrict__ lists, int* ps, int& total_recs, bool wide, int skip,
+                          int* __restrict__ rec_start, int* __restrict__ lists, int* ps, int& total_recs, bool may_wide, int skip,
                           long long t0_first = 0, long long t1_first = -1) {
   constexpr int kW = NT / 64;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -583,7 +583,8 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
   }
   for (int i = tid; i < 2 * kBuckets; i += NT) ps[kPsHist + i] = 0;
   __syncthreads();
-  if (wv == 0) {
+  // wave 0 for the split consumer, wave 1 for the wide one
+  if (wv == 0 || (may_wide && wv == 1)) {
     // per v-head (lanes 0-7) the log2 bound of one chunk's map, estimated from
     // the per-head constants (a = 0): 64 log2 g = -64 log2(e) exp(A_log) softplus(dt_bias)
     const float hb = lane < kVHeads
@@ -612,49 +613,21 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     }
     const int Lc = seg_cand(ci);
     const int nseg_max = ml > 0 ? (ml - 1) / Lc + 1 : 0;
-    float est;
-    if (warm) {
-      // Warm-up scheme: one run per segment (T of them), each later segment
-      // W chunks longer; the work-groups take a run's 16 items together, so
-      // the packing is that of T runs on kConsumerGroups / 16 machines:
-      // the longest run, or the balanced load plus a quarter of an average
-      // run for the last round when there is more than one.  Item overhead
-      // (descriptor, warm-up bounds, first copies, final stores) about 1.5
-      // chunk steps.  Fitted with a list-scheduling model of the consumer
-      // against its measured step and item costs (c3: L = 18, 2 x 8192
-      // tokens: 16, 4 x 16384: 64, all measured faster than the earlier
-      // estimate's 20, 28 and 96).
-      constexpr float kWarmItem = 1.5f, kTailShare = 0.25f, kSegmented = 0.75f;
-      // the split consumer takes a run's 16 items on 256 groups, the wide one
-      // its 8 on 256 CUs (two groups of a CU share its throughput)
-      const float kMachines = static_cast<float>(kConsumerGroups / (wide ? 8 : 16));
-      const float T = 0.5f * (runs + nl);                      // runs = sum of 2 nseg - 1
-      const float work = sl + static_cast<float>(w_est) * (T - nl);
-      const float longest = ml > Lc ? static_cast<float>(Lc + w_est) : static_cast<float>(ml);
-      const float balanced = (work + kWarmItem * T) / kMachines;
-      const float tail = T > kMachines ? kTailShare * (work / fmaxf(T, 1.f) + kWarmItem) : 0.f;
-      est = fmaxf(longest + kWarmItem, balanced + tail) + (nseg_max > 1 ? kSegmented : 0.f);
-    } else {
-      // M-run scheme: a later segment runs twice, its M-run per v-head only
-      // until the head's map is negligible (about wh chunks)
-      float mfrac = 0.f;
+    // the share of a segment that its M-run forms: per v-head until the map is
+    // negligible (about wh chunks)
+    float mfrac = 0.f;
+    if (!warm) {
 #pragma unroll
       for (int hh = 0; hh < kVHeads; ++hh)
         mfrac += static_cast<float>(min(__builtin_amdgcn_readlane(wh, hh), Lc)) / (kVHeads * static_cast<float>(Lc));
-      if (wide) {
-        constexpr float kRunItem = 1.5f, kTailShare = 0.25f, kCorrShare = 0.04f, kScan = 0.4f, kFinish = 6.0f;
-        const float kMachines = static_cast<float>(kConsumerGroups / 8);
-        const float mwork = (sl - a) * mfrac;
-        const float longest = static_cast<float>(min(Lc, ml));
-        const float balanced = (sl + mwork + kRunItem * runs) / kMachines;
-        const float tail = runs > kMachines ? kTailShare * ((sl + mwork) / fmaxf(runs, 1.f) + kRunItem) : 0.f;
-        est = fmaxf(longest + kRunItem, balanced + tail) +
-              (nseg_max > 1 ? kScan * static_cast<float>(nseg_max - 1) + kFinish + kCorrShare * mwork : 0.f);
-      } else {
-        est = plan_split_mrun_us(PlanStats{sl, a, 0.5f * (runs + nl), nl, ns, mfrac, ml, Lc});
-      }
     }
-    // key: estimate in 1/16, then the longer candidate; invalid lanes hold
+    const PlanStats ps_c = {sl, a, 0.5f * (runs + nl), nl, ns, mfrac, ml, Lc, static_cast<float>(w_est), may_wide};
+    float est;
+    if (wv == 0)   // uniform
+      est = warm ? plan_split_warm_us(ps_c) : plan_split_mrun_us(ps_c);
+    else
+      est = warm ? plan_wide_warm_us(ps_c) : plan_wide_mrun_us(ps_c);
+    // key: estimate in 1/16 us, then the longer candidate; invalid lanes hold
     // the maximum.  No slot is written in the warm-up scheme, but the slot
     // bound still applies: the run table holds max_runs(N, gcap) = N + 2 gcap
     // runs, and with at most gcap later segments the runs (one per segment)
@@ -668,14 +641,19 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     // minimum over the lanes: the maximum of the complements
     const int best = 0x7fffffff - wave_max0(0x7fffffff - key);
     if (lane == 0) {
-      ps[kPsMisc] = seg_cand(63 - (best & 63));
-      ps[kPsMisc + 1] = warm ? 1 : 0;
-      ps[kPsMisc + 2] = ml > 0 ? (ml - 1) / seg_cand(63 - (best & 63)) + 1 : 0;
+      const int cand = seg_cand(63 - (best & 63));
+      int* pm = ps + kPsMisc + 4 * wv;
+      pm[0] = cand;
+      pm[1] = warm ? 1 : 0;
+      pm[2] = ml > 0 ? (ml - 1) / cand + 1 : 0;
+      pm[3] = best >> 6;
     }
   }
   __syncthreads();
-  const int L = ps[kPsMisc];
-  const bool warm = ps[kPsMisc + 1] != 0;
+  const bool take_wide = may_wide && ps[kPsMisc + 7] < ps[kPsMisc + 3];
+  const int* choice = ps + kPsMisc + (take_wide ? 4 : 0);
+  const int L = choice[0];
+  const bool warm = choice[1] != 0;
 
   // ---- pass 2: per-sequence counts and their prefix sums ----
   // v: records, short sequences, multi-segment sequences, slots, full runs
@@ -713,7 +691,8 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
       lv.hdr[8] = 0;   // work queue
       lv.hdr[9] = 0;   // correction blocks
       lv.hdr[10] = 0;  // finish queue
-      lv.hdr[11] = ps[kPsMisc + 2];
+      lv.hdr[11] = choice[2];
+      lv.hdr[12] = take_wide ? 1 : 0;
     }
     if (lane == 63) {
       lv.hdr[0] = tot[4] + inc;
@@ -787,7 +766,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     const void* __restrict__ cu, int is64, int num_seqs, long long T, int R, int gcap,
     const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-    int* __restrict__ rec_start, int4* __restrict__ recs, int* __restrict__ lists, int wide) {
+    int* __restrict__ rec_start, int4* __restrict__ recs, int* __restrict__ lists, int may_wide) {
   __shared__ int ps[kPlanScratch];
   const int tid = threadIdx.x;
   const int per = (num_seqs + kPlanThreads - 1) / kPlanThreads;
@@ -795,7 +774,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   const int s_end = min(num_seqs, s_begin + per);
   int total_recs;
   int base = plan_batch<kPlanThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, ps,
-                                      total_recs, wide != 0, -1);
+                                      total_recs, may_wide != 0, -1);
   for (int s = s_begin; s < s_end; ++s) {
     long long t0, t1;
     seq_bounds(cu, is64, s, T, t0, t1);
@@ -1436,14 +1415,14 @@ __global__ __launch_bounds__(kPrepassThreads, kGroups) void prepass_kernel(
     const float* __restrict__ dt_bias, const uint16_t* __restrict__ b,
     const int4* __restrict__ recs, const void* __restrict__ cu, int is64, int num_seqs, long long T, int R,
     int gcap, int fused_plan, int* __restrict__ rec_start, int* __restrict__ lists,
-    uint16_t* __restrict__ ws_frag, float* __restrict__ ws_gam, int wide) {
+    uint16_t* __restrict__ ws_frag, float* __restrict__ ws_gam, int may_wide) {
   __shared__ PrepassSmem<kPrepassWaves> sm;
   if (fused_plan && blockIdx.x == 0) {
     // work-group 0 plans the batch (lists for the consumer) while the others
     // run the records
     int total_recs;
     plan_batch<kPrepassThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, sm.u.plan,
-                                total_recs, wide != 0, -1);
+                                total_recs, may_wide != 0, -1);
     return;
   }
   prepass_items<kPair, kPrepassWaves>(sm, static_cast<int>(blockIdx.x) - fused_plan,
@@ -3044,51 +3023,25 @@ __device__ __forceinline__ void split_items(
   }
 }
 
-// Consumer entry: work-groups [0, g_long) run the split consumer over the
-// run list, the rest the full-head consumer over the short-sequence list, so
-// both regimes of a mixed batch run concurrently.  Lists come from the plan
-// (no host synchronisation); an empty list costs one short round of groups.
-union ConsumerLds {
-  ConsumerSmem full;
-  SplitSmem split;
-};
-
-__global__ __launch_bounds__(kSplitThreads)
-void consumer_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-                     const uint16_t* __restrict__ v, const float* __restrict__ state,
-                     int R, int gcap, float scale, int* __restrict__ lists, int num_seqs,
-                     int g_long, const uint16_t* __restrict__ ws_frag, const float* __restrict__ ws_gam,
-                     uint16_t* __restrict__ out, float* __restrict__ new_state, uint16_t* __restrict__ oi,
-                     float* __restrict__ slotb, uint16_t* __restrict__ slotm, int* __restrict__ mval,
-                     int4* __restrict__ fix) {
-  __shared__ ConsumerLds sm;
-  const int bid = blockIdx.x;
-  const ListView lv = list_view(lists, num_seqs, gcap);
-  if (bid < g_long) {
-    split_items(sm.split, bid, g_long, lv, q, k, v, state, scale, ws_frag, ws_gam, out, new_state, oi, slotb,
-                slotm, mval, fix, R * kVHeads);
-    // an M-run that stopped early may leave its next chunk's copies into LDS in
-    // flight: they land before the work-group releases its LDS
-    __builtin_amdgcn_s_waitcnt(0);
-  } else {
-    full_head_items(sm.full, bid - g_long, static_cast<int>(gridDim.x) - g_long, lv.shorts, lv.hdr[1],
-                    q, k, v, state, scale, ws_frag, ws_gam, out, new_state);
-  }
-}
-
 // ============================================================================
-// wide consumer: one work-group per (run or short sequence, v-head)
+// wide consumer: half a work-group per (run or short sequence, v-head)
 // ============================================================================
-// For batches with work for every CU.  A group of four waves carries a whole
+// For batches with work for every CU.  Four waves carry a whole
 // head, wave w the value rows 32 w .. 32 w + 31 as two 16-row tiles (row i of
 // tile e is value row 32 w + wide_row(e, i): a lane then holds eight
 // consecutive value columns of an output token over the two tiles), and runs
 // everything a chunk needs (X, Y^T, Aqk tiles, R, Delta, O^T, S') itself: no
 // state or Delta leaves the wave's registers, and every K / Q / Tb / Aqk
-// fragment read from LDS feeds both tiles.  Two groups share a CU (78 KB of
-// LDS, 256 VGPRs per wave, two waves per SIMD) and are independent of each
-// other, so one group's barriers, copies, item starts and state traffic run
-// under the other's products.
+// fragment read from LDS feeds both tiles.  The halves of a work-group (78 KB of
+// LDS each, 256 VGPRs per wave, two waves per SIMD) are independent of each
+// other, with barriers of their own (HalfBarrier), so one half's barriers,
+// copies, item starts and state traffic run under the other's products.  Half a
+// group and not a launch of its own, so that the planner, which alone knows the
+// lengths and gates, can choose between this and the split consumer.  As a
+// launch of 256-thread groups chosen on the host it was 0 to 2% faster (512 x 34
+// tokens 144.3 us, now 145.7; 64 x 128 42.6, 43.5; 96 x 400 119, 121), but by
+// number of sequences and mean length alone up to 47% slower than the split
+// consumer (figures at plan_wide_mrun_us).
 //
 // LDS: K rows and the gate block are double-buffered (K is read to the end of
 // the chunk by the state update); Q, V, Tb and Aqk have one buffer each.  Two
@@ -3097,7 +3050,7 @@ void consumer_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict_
 // W2 at the end (the next chunk's operands have landed).
 constexpr int kWideThreads = 256;
 constexpr int kWideWaves = kWideThreads / 64;
-constexpr int kWideGroups = 512;           // two per CU
+constexpr int kWideGroups = 512;           // halves: two per CU
 constexpr int kWideStores = 4;             // output stores of a wave per chunk (one per 16-token block)
 
 __host__ __device__ constexpr int wide_row(int e, int i) { return 8 * (i >> 2) + 4 * e + (i & 3); }
@@ -3111,7 +3064,7 @@ struct __align__(16) WideSmem {
   float gt[2][4 * kChunk];
   int next_item;
 };
-static_assert(2 * sizeof(WideSmem) <= 160 * 1024, "two groups per CU");
+static_assert(2 * sizeof(WideSmem) <= 160 * 1024, "two halves per CU");
 
 // Resources over an item's rows and records, formed once per item: a chunk's
 // copies and stores then differ only in a 32-bit offset.  Row i 64 + t of an
@@ -3310,11 +3263,40 @@ __device__ __forceinline__ void wide_front(WideSmem& sm, int P, const f32x4 (&st
   }
 }
 
+// Barriers of one half (four waves) of a 512-thread work-group: the halves run
+// unrelated items, so the hardware barrier, which counts all eight waves, cannot
+// serve them.  A wave adds itself to a count in LDS once its own operations are
+// done and polls until its half's four waves have; the waves of a group are
+// resident together and make the same number of calls within a half, so every
+// wait ends.  Only where another call overwrites the workspace meanwhile may the
+// waves read different plans: a wave that has polled kHalfSpins times (at least
+// 64 cycles each, more than 0.1 s) therefore stops waiting, here and at every
+// later barrier, so that such calls end, with undefined results.  Each wave first waits for its LDS operations, and for its vector
+// memory operations but the kPending youngest (kLdsOnly: none of them).
+constexpr int kLdsOnly = -1;
+constexpr int kHalfSpins = 1 << 22;
+struct HalfBarrier {
+  int* count;
+  int target;
+  template <int kPending>
+  __device__ __forceinline__ void wait() {
+    static_assert(kPending >= kLdsOnly && kPending < 16, "vmcnt field");
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(kPending == kLdsOnly ? 0xc07f : (0x0070 | kPending));
+    if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    target += kWideWaves;
+    for (int spins = 0;
+         __builtin_amdgcn_readfirstlane(__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < target;)
+      if (++spins == kHalfSpins) target = -(1 << 30);   // and later targets: below any count
+    asm volatile("" ::: "memory");
+  }
+};
+
 // One chunk of a wave's two tiles (see chain_chunk for the numerics, which are
 // the same).  emit: the chunk has outputs (a warm-up chunk has none).  copy_k /
 // copy_qvt issue the next chunk's copies.
 template <typename CopyK, typename CopyQvt>
-__device__ __forceinline__ void wide_chunk(WideSmem& sm, int P, int c, f32x4 (&st)[2][8], int w, int lane, float scale,
+__device__ __forceinline__ void wide_chunk(WideSmem& sm, HalfBarrier& bar, int P, int c, f32x4 (&st)[2][8], int w, int lane, float scale,
                                            bool emit, __amdgpu_buffer_rsrc_t orc, uint32_t obase,
                                            CopyK&& copy_k, CopyQvt&& copy_qvt) {
   lane = opaque_lane(lane);
@@ -3401,7 +3383,7 @@ __device__ __forceinline__ void wide_chunk(WideSmem& sm, int P, int c, f32x4 (&s
 #pragma unroll
       for (int m = 0; m < 4; ++m) D[e][m] = D[e][m] * inv;
     }
-  lds_barrier();   // W1: every wave's Aqk tiles are in LDS; Q, V and Tb are dead
+  bar.template wait<kLdsOnly>();   // W1: every wave's Aqk tiles are in LDS; Q, V and Tb are dead
   copy_qvt();
 
   // ---- O^T = scale (Y^T diag(gam) + Delta^T Aqk^T): lane (lg, l16) holds
@@ -3477,45 +3459,23 @@ __device__ __forceinline__ void wide_chunk(WideSmem& sm, int P, int c, f32x4 (&s
   }
 }
 
-// Which batches run on the wide consumer: those whose (sequence, v-head) items
-// fill the chip by themselves.  More items than CUs (N > 32) of at most four
-// chunks on average, or two rounds of items (N >= 64) of any length.  Below
-// that the split consumer's shorter chunk step (1.9 us for a half head on a CU
-// of its own against 3.6 us for a whole head here) wins.  Measured per call,
-// split -> wide (fast gates, mean length x sequences): 30 x 48 30.2 -> 26.6 us,
-// 120 x 48 51.2 -> 41.3, 60 x 64 49.8 -> 34.2, 60 x 128 77.3 -> 55.1, 400 x 96
-// 143 -> 112, 34 x 512 169 -> 139; but 60 x 16 24.0 -> 29.2, 400 x 24 46 -> 48,
-// 400 x 48 77 -> 83.
+// Batches for which the planner weighs the wide consumer against the split one:
+// more (sequence, v-head) items than CUs, so that there are two for some.  (Every
+// such batch has the 256 groups of short sequences in its consumer grid.)
 inline bool wide_batch(int num_seqs, long long tokens) {
-  return tokens <= kWideMaxTokens &&
-         (num_seqs >= kWideGroups / kVHeads ||
-          (num_seqs > kConsumerGroups / kVHeads && tokens <= 4ll * kChunk * num_seqs));
-}
-
-// Barrier W2: every wave's copies have landed (at most kPending vector-memory
-// operations, the chunk's output stores, are younger) and its LDS reads are done.
-template <int kPending>
-__device__ __forceinline__ void wide_barrier() {
-  static_assert(kPending >= 0 && kPending < 16, "vmcnt field");
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0x0070 | kPending);
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+  return tokens <= kWideMaxTokens && num_seqs > kConsumerGroups / kVHeads;
 }
 
 // Work items: (run, v-head) of the run list in list order (longest first),
-// then (short sequence, v-head).  Group g starts with item g; later items are
+// then (short sequence, v-head).  Half-group g starts with item g; later items are
 // claimed from the queue counter, the claim issued during the item's last
 // chunk.  See split_items for what a run is and where its results go.
-__global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    const float* __restrict__ state, int R, int gcap, float scale, int* __restrict__ lists, int num_seqs,
+__device__ __forceinline__ void wide_items(
+    WideSmem& sm, HalfBarrier bar, int group, const ListView lv, int fix_cap, const uint16_t* __restrict__ q,
+    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const float* __restrict__ state, float scale,
     const uint16_t* __restrict__ ws_frag, const float* __restrict__ ws_gam, uint16_t* __restrict__ out,
     float* __restrict__ new_state, uint16_t* __restrict__ oi, float* __restrict__ slotb,
     uint16_t* __restrict__ slotm, int* __restrict__ mval, int4* __restrict__ fix) {
-  __shared__ WideSmem sm;
-  const ListView lv = list_view(lists, num_seqs, gcap);
-  const int fix_cap = R * kVHeads;
   // written by earlier launches, constant here: scalar loads
   const auto* runs_c = (const __attribute__((address_space(4))) u32x4*)lv.runs;
   const auto* shorts_c = (const __attribute__((address_space(4))) u32x4*)lv.shorts;
@@ -3523,16 +3483,15 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
   const auto* gam_c = (const __attribute__((address_space(4))) float*)ws_gam;
   const int nruns = hdr_c[0], nshort = hdr_c[1], seg_len = hdr_c[2];
   const int nitems = (nruns + nshort) * kVHeads;
-  const int nwg = static_cast<int>(gridDim.x);
   int* queue = lv.hdr + 8;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x & (kWideThreads - 1);
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane0 = tid & 63;
   const int vrow0 = 32 * w;                      // first value row of the wave
   int zero_v;   // see split_items
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero_v));
 
-  for (int item = static_cast<int>(blockIdx.x); item < nitems;) {
+  for (int item = group; item < nitems;) {
     int claimed = 0;
     bool has_claim = false;
     auto claim = [&] {
@@ -3640,7 +3599,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
     int formed = n;
     int pl = 0;   // K buffer of the last chunk run
     if (n > 0) {
-      wide_barrier<0>();
+      bar.template wait<0>();
       if (mrun && tid == 64) fix_pos = atomicAdd(lv.hdr + 9 + zero_v, fix_max);
       for (int i = 0;; ++i) {
         const int P = i & 1;
@@ -3648,7 +3607,7 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
         if (!more) claim();
         const int c = i - warmup == nrun - 1 ? last_tok : kChunk;
         wide_chunk(
-            sm, P, c, st, w, lane0, scale, i >= warmup, wi.out, static_cast<uint32_t>(i) * kChunk * kVRow,
+            sm, bar, P, c, st, w, lane0, scale, i >= warmup, wi.out, static_cast<uint32_t>(i) * kChunk * kVRow,
             [&] {
               if (more) wide_dma_k(sm, P ^ 1, wi, i + 1, lane0, w);
             },
@@ -3658,9 +3617,9 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
         lbound += sm.gt[P][kBoundAt];
         // W2: a warm-up chunk has no output stores younger than its copies
         if (i >= warmup)
-          wide_barrier<kWideStores>();
+          bar.template wait<kWideStores>();
         else
-          wide_barrier<0>();
+          bar.template wait<0>();
         pl = P;
         if (mrun && lbound < kNegligibleLog2) {
           formed = i + 1;
@@ -3672,10 +3631,10 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
       // into the other buffer, which serves as scratch below: they landed at
       // the chunk's closing barrier
     } else {
-      lds_barrier();   // every wave has read this item's index before it is replaced
+      bar.template wait<kLdsOnly>();   // every wave has read this item's index before it is replaced
     }
     claim();
-    if (tid == 0) sm.next_item = nwg + claimed;
+    if (tid == 0) sm.next_item = kWideGroups + claimed;
     if (mrun && tid == 0) {
       mval[static_cast<size_t>(slot) * kVHeads + h] = formed | (formed < n ? kMNegligible : 0);
       *seg_ready(slotm, slot - jseg, jseg, h) = 0;
@@ -3721,8 +3680,77 @@ __global__ __launch_bounds__(kWideThreads, 2) void wide_kernel(
             }
       }
     }
-    lds_barrier();   // publishes the next item; the item's stores stay in flight
+    bar.template wait<kLdsOnly>();   // publishes the next item; the item's stores stay in flight
     item = __builtin_amdgcn_readfirstlane(sm.next_item);
+  }
+}
+
+// ============================================================================
+// consumer entry
+// ============================================================================
+// Lists come from the plan (no host synchronisation).  Work-groups [0, g_long)
+// run the split consumer over the run list, the rest the full-head consumer over
+// the short-sequence list, so both regimes of a batch run concurrently; an empty
+// list costs one short round of groups.
+//
+// kMayWide (batches of more items than CUs, wide_batch): the planner has chosen
+// between that and the wide consumer, whose two items per CU are the halves of
+// each of the first 256 groups.  (One grid of 256 groups, which run their share
+// of the short sequences after their runs, was slower for the former by up to 25%:
+// one sequence of 2,896 tokens among 72 72 -> 91 us.)
+union ConsumerLds {
+  ConsumerSmem full;
+  SplitSmem split;
+};
+template <bool kMayWide>
+struct EntryLds;
+template <>
+struct EntryLds<false> {
+  ConsumerLds c;
+};
+template <>
+struct EntryLds<true> {
+  union {
+    ConsumerLds c;
+    WideSmem wide[2];
+  };
+  int count[2];   // HalfBarrier
+};
+static_assert(sizeof(EntryLds<true>) <= 160 * 1024, "one group per CU");
+static_assert(kSplitThreads == 2 * kWideThreads && kWideGroups == 2 * kConsumerGroups, "two wide items per group");
+
+template <bool kMayWide>
+__global__ __launch_bounds__(kSplitThreads)
+void consumer_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                     const uint16_t* __restrict__ v, const float* __restrict__ state,
+                     int R, int gcap, float scale, int* __restrict__ lists, int num_seqs,
+                     int g_long, const uint16_t* __restrict__ ws_frag, const float* __restrict__ ws_gam,
+                     uint16_t* __restrict__ out, float* __restrict__ new_state, uint16_t* __restrict__ oi,
+                     float* __restrict__ slotb, uint16_t* __restrict__ slotm, int* __restrict__ mval,
+                     int4* __restrict__ fix) {
+  __shared__ EntryLds<kMayWide> sm;
+  const int bid = blockIdx.x;
+  const ListView lv = list_view(lists, num_seqs, gcap);
+  if constexpr (kMayWide) {
+    if (((const __attribute__((address_space(4))) int*)lv.hdr)[12] != 0) {
+      if (bid >= kConsumerGroups) return;
+      if (threadIdx.x < 2) sm.count[threadIdx.x] = 0;
+      __syncthreads();
+      const int half = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWideThreads);
+      wide_items(sm.wide[half], HalfBarrier{&sm.count[half], 0}, bid + kConsumerGroups * half, lv, R * kVHeads, q, k, v,
+                 state, scale, ws_frag, ws_gam, out, new_state, oi, slotb, slotm, mval, fix);
+      return;
+    }
+  }
+  if (bid < g_long) {
+    split_items(sm.c.split, bid, g_long, lv, q, k, v, state, scale, ws_frag, ws_gam, out, new_state, oi, slotb,
+                slotm, mval, fix, R * kVHeads);
+    // an M-run that stopped early may leave its next chunk's copies into LDS in
+    // flight: they land before the work-group releases its LDS
+    __builtin_amdgcn_s_waitcnt(0);
+  } else {
+    full_head_items(sm.c.full, bid - g_long, static_cast<int>(gridDim.x) - g_long, lv.shorts, lv.hdr[1],
+                    q, k, v, state, scale, ws_frag, ws_gam, out, new_state);
   }
 }
 
@@ -4219,22 +4247,17 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
         kb, A_log, ab, dt_bias, bb, recs, cu_seqlens, cu_seqlens_is_int64, num_seqs, total_tokens,
         Ri, gc, fused_plan, rec_start, lists, frag, gam, wide);
   }
-  // persistent grids: two wide groups per CU, or one group per CU per kind of
-  // the split launch; a sequence needs 2 chunks (65 tokens) to be long
-  if (wide) {
-    const long long g_wide = std::min<long long>(max_runs(num_seqs, gcap) * kVHeads, kWideGroups);
-    wide_kernel<<<dim3(static_cast<unsigned>(g_wide)), dim3(kWideThreads), 0, st>>>(
-        qb, kb, vb, state, Ri, gc, scale, lists, num_seqs, frag, gam, ob, new_state, oi, slotb, slotm, mval, fix);
-  } else {
-    const long long g_long =
-        total_tokens > kChunk ? std::min<long long>(max_runs(num_seqs, gcap) * 2 * kVHeads, kConsumerGroups) : 0;
-    // a mixed batch has run its short sequences already
-    const long long g_short =
-        mixed ? 0 : std::min<long long>(static_cast<long long>(num_seqs) * kVHeads, kConsumerGroups);
-    consumer_kernel<<<dim3(static_cast<unsigned>(g_long + g_short)), dim3(kSplitThreads), 0, st>>>(
-        qb, kb, vb, state, Ri, gc, scale, lists, num_seqs, static_cast<int>(g_long), frag, gam, ob, new_state, oi,
-        slotb, slotm, mval, fix);
-  }
+  // persistent grids: one group per CU per kind; a sequence needs 2 chunks (65
+  // tokens) to be long
+  const long long g_long =
+      total_tokens > kChunk ? std::min<long long>(max_runs(num_seqs, gcap) * 2 * kVHeads, kConsumerGroups) : 0;
+  // a mixed batch has run its short sequences already
+  const long long g_short =
+      mixed ? 0 : std::min<long long>(static_cast<long long>(num_seqs) * kVHeads, kConsumerGroups);
+  auto* consumer = wide ? consumer_kernel<true> : consumer_kernel<false>;
+  consumer<<<dim3(static_cast<unsigned>(g_long + g_short)), dim3(kSplitThreads), 0, st>>>(
+      qb, kb, vb, state, Ri, gc, scale, lists, num_seqs, static_cast<int>(g_long), frag, gam, ob, new_state, oi,
+      slotb, slotm, mval, fix);
   // M-runs need a sequence of more than kMaxWholeChunks chunks and slots
   if (gcap > 0 && total_tokens > static_cast<long long>(kMaxWholeChunks) * kChunk) {
     const long long g_fin = std::min<long long>(R * kVHeads, kFinGroups);

@@ -1,7 +1,6 @@
-"""GPU parity of the wide consumer (batches of many sequences: one work-group
-per (run or short sequence, v-head), two per CU) at the edges of its range:
-the smallest batches that take it, one on either side of the rule, chunk and
-16-token tile boundaries, empty sequences, warm-up and M-run segments beside
+"""GPU parity of batches of many sequences around the wide consumer's range (half
+a work-group per (run or short sequence, v-head)): 32 and 33 sequences (the
+planner weighs it from 33 on), chunk and 16-token tile boundaries, empty sequences, warm-up and M-run segments beside
 short sequences, no initial state, an output that is only 8-byte aligned, and
 the plan launch's batches.  Bar: the oracle tolerances of gpu_util (fixed
 there; the bounds on outputs and states of every prefill test)."""
@@ -27,7 +26,7 @@ CASES = {
     "33 sequences": (_tile(33), {}),
     "32 sequences (split consumer)": (_tile(32), {}),
     "33 x 256 tokens": ([256] * 33, {}),
-    "33 x 257 tokens (split consumer)": ([257] * 33, {}),
+    "33 x 257 tokens": ([257] * 33, {}),
     "64 sequences, one long": (_tile(64, [1500]), {}),
     "63 sequences, one long": (_tile(63, [900]), {}),
     "70 sequences, near-1 decay": (_tile(70, [700, 1100]), {"weak": True}),
