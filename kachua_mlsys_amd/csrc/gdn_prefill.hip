@@ -1997,16 +1997,15 @@ __device__ __forceinline__ void split_barrier(bool chain) {
 // Latency-bound calls run as one launch with no plan and no workspace: one
 // work-group per (sequence, v-head).  Wave j forms chunk j's terms (the prepass
 // of one item, written to LDS instead of the workspace) while chunk 0's K / Q /
-// V copies and the state land, up to kDirectTerms chunks at once; the eight
-// waves then run the chunks one after the other as the full-head consumer does,
+// V copies and the state land; the eight waves then run the chunks one after the other as the full-head consumer does,
 // the state staying in registers and the next chunk's copies landing in the
 // other buffer.  The state moves as 8 rows x 128 contiguous bytes per
 // instruction and changes to the C layout through 2 KB of LDS per wave (see
 // load_state_rows for what the direct access pattern costs); its loads need
 // only the sequence index and are requested before the sequence's bounds.
-constexpr int kDirectTerms = 7;
+constexpr int kDirectChunks = 4;   // the longest sequence that runs directly
 constexpr int kDirectMaxSeqs = 64;
-constexpr int kDirectMaxTokens = 4 * kChunk;
+constexpr int kDirectMaxTokens = kDirectChunks * kChunk;
 
 struct __align__(16) DirectSmem {
   uint16_t ks[2][kChunk][kDim];
@@ -2014,26 +2013,25 @@ struct __align__(16) DirectSmem {
   uint16_t vs[2][kChunk][kDim];
   // chunk j's Tb in tb[j + 1]; its Aqk in tb[j], where the previous chunk's Tb
   // is dead (every wave has read it before the barrier that chunk's Aqk needs)
-  uint16_t tb[kDirectTerms + 1][kMatElems];
-  float gt[kDirectTerms][4 * kChunk];
-  PrepassWaveSmem<1> w[kDirectTerms];    // scratch of the terms waves
+  uint16_t tb[kDirectChunks + 1][kMatElems];
+  float gt[kDirectChunks][4 * kChunk];
+  PrepassWaveSmem<1> w[kDirectChunks];   // scratch of the terms waves
 };
-// the terms' N blocks use K and V of buffer 1, the state's layout change Q of
-// a buffer that holds no live rows
-static_assert(kDirectTerms * sizeof(PrepassNt) <= 2 * kChunk * kDim * sizeof(uint16_t), "N blocks");
+// the terms' N blocks use K of buffer 1, the state's layout change Q of a buffer
+// that holds no live rows
+static_assert(kDirectChunks * sizeof(PrepassNt) <= kChunk * kDim * sizeof(uint16_t), "N blocks");
 static_assert(sizeof(DirectSmem) <= 160 * 1024, "one group per CU");
 
 // Calls of at most four chunks run on direct_kernel alone.  Measured against
 // the planned path: 4 sequences of 50 tokens 18.5 -> 13.3 us, one of 200 21.3
 // -> 21.0, one of 256 even (3.3 us per further chunk).
 // Larger calls of few, mostly short sequences take the direct path for the
-// sequences of at most kMixedChunks chunks, in the launch that plans and
+// sequences of at most kDirectChunks chunks, in the launch that plans and
 // prepasses the longer ones (mixed_kernel), which then run as ever: 8 sequences
 // of 50 tokens 20.9 -> 16.8 us, 24 of 60 30.8 -> 19.3, 32 of 60 35.1 -> 23.0;
 // one sequence of 500 or 1,889 tokens among tiny ones costs what it did (25,
 // 33 us).  Longer sequences gain from the split consumer's segments instead
 // (24 of 120 tokens: 34.0 planned, 37.4 mixed; 16 of 400: 38.8, 51.0).
-constexpr int kMixedChunks = 4;
 constexpr int kMixedMaxSeqs = kConsumerGroups / kVHeads;   // a CU for each (sequence, v-head)
 inline bool direct_batch(int num_seqs, long long tokens) {
   return num_seqs <= kDirectMaxSeqs && tokens <= kDirectMaxTokens;
@@ -2042,11 +2040,11 @@ inline bool mixed_batch(int num_seqs, long long tokens) {
   return num_seqs <= kMixedMaxSeqs && tokens <= 1ll * kChunk * num_seqs;
 }
 
-// One (sequence s, v-head h); nothing when the sequence has more than max_chunks
-// chunks (it runs elsewhere).
+// One (sequence s, v-head h); nothing when the sequence has more than
+// kDirectChunks chunks (it runs elsewhere).
 __device__ __forceinline__ void direct_group(
-    DirectSmem& sm, int s, int h, int max_chunks, const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    const float* __restrict__ state, const float* __restrict__ A_log, const uint16_t* __restrict__ a,
+    DirectSmem& sm, int s, int h, const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+    const uint16_t* __restrict__ v, const float* __restrict__ state, const float* __restrict__ A_log, const uint16_t* __restrict__ a,
     const float* __restrict__ dt_bias, const uint16_t* __restrict__ b, const void* __restrict__ cu, int is64,
     long long T, float scale, uint16_t* __restrict__ out, float* __restrict__ new_state) {
   const int hq = h / kGva;
@@ -2073,7 +2071,7 @@ __device__ __forceinline__ void direct_group(
   seq_bounds(cu, is64, s, T, t0, t1);
   const int len = static_cast<int>(t1 - t0);   // 0 .. T
   const int nch = (len + kChunk - 1) / kChunk;
-  if (nch > max_chunks) return;
+  if (nch > kDirectChunks) return;
   if (len <= 0) {   // an empty sequence: zero state, no output rows
     float* dst = new_state + soff;
 #pragma unroll
@@ -2104,16 +2102,15 @@ __device__ __forceinline__ void direct_group(
       dma16<2>(vb + row * (kVHeads * kDim * 2) + v_col, &sm.vs[P][32 * jj + 4 * w][0]);
     }
   };
-  // wave w forms the terms of chunk b0 + w, slot w
-  auto terms = [&](int b0) __attribute__((always_inline)) {
-    if (w >= kDirectTerms || b0 + w >= nch) return;
-    const int c = chunk_len(b0 + w);
-    const long long c0 = t0 + static_cast<long long>(kChunk) * (b0 + w);
+  // wave w forms the terms of chunk w
+  auto terms = [&]() __attribute__((always_inline)) {
+    if (w >= nch) return;
+    const int c = chunk_len(w);
+    const long long c0 = t0 + static_cast<long long>(kChunk) * w;
     const size_t gi = static_cast<size_t>(c0 + min(lane, c - 1)) * kVHeads + h;
     const float a1[kGva] = {bf2f(a[gi]), 0.0f}, b1[kGva] = {bf2f(b[gi]), 0.0f};
     const float al1[kGva] = {A_log[h], 0.0f}, dt1[kGva] = {dt_bias[h], 0.0f};
-    // 4 KB each in K (waves 0-3) and V (4-6) of buffer 1
-    PrepassNt* nt = reinterpret_cast<PrepassNt*>(w < 4 ? &sm.ks[1][0][0] : &sm.vs[1][0][0]) + (w & 3);
+    PrepassNt* nt = reinterpret_cast<PrepassNt*>(&sm.ks[1][0][0]) + w;   // 4 KB
     // only the 16-token blocks that hold tokens are formed (c <= 16 nb)
     auto blocks = [&](auto NBC) __attribute__((always_inline)) {
       constexpr int NB = decltype(NBC)::value;
@@ -2136,46 +2133,42 @@ __device__ __forceinline__ void direct_group(
   auto scratch = [&](int P) { return reinterpret_cast<f32x4*>(&sm.qs[P][0][0]) + 128 * w; };
   f32x4 st[8];
 
-  // runs chunk j (slot i of its batch) from buffer P
-  auto chunk = [&](int j, int i, int P, auto NBC) __attribute__((always_inline)) {
-    const ChunkLds lds = {sm.ks[P], sm.qs[P], sm.vs[P], sm.tb[i + 1], sm.tb[i], sm.gt[i]};
+  // runs chunk j from buffer P
+  auto chunk = [&](int j, int P, auto NBC) __attribute__((always_inline)) {
+    const ChunkLds lds = {sm.ks[P], sm.qs[P], sm.vs[P], sm.tb[j + 1], sm.tb[j], sm.gt[j]};
     const int lane = opaque_lane(tid);
     consumer_chunk<decltype(NBC)::value, true>(lds, chunk_len(j), st, w, lane, scale, out_rsrc(j),
                                          2u * static_cast<uint32_t>(vcol + 4 * (lane >> 4)));
   };
+  copy(0, 0);
+  terms();
+  {
+    const int lane = opaque_lane(tid), l16 = lane & 15, lg = lane >> 4;
+    f32x4* sc = scratch(1);
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) sc[8 * (8 * i + (lane >> 3)) + ((lane & 7) ^ (lane >> 3))] = rows[2 * qd + i];
+      wave_lds_sync();
+#pragma unroll
+      for (int i = 0; i < 2; ++i) st[2 * qd + i] = sc[8 * l16 + ((2 * lg + i) ^ (l16 & 7))];
+      wave_lds_sync();
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);   // the first copies and the terms have landed
+  __syncthreads();
   int pl = 0;   // the last chunk's buffer
-  for (int b0 = 0; b0 < nch; b0 += kDirectTerms) {   // batches of chunks whose terms are formed together
-    copy(b0, 0);   // past the first batch every wave is behind its last barrier: both buffers are free
-    terms(b0);
-    if (b0 == 0) {
-      const int lane = opaque_lane(tid), l16 = lane & 15, lg = lane >> 4;
-      f32x4* sc = scratch(1);
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) sc[8 * (8 * i + (lane >> 3)) + ((lane & 7) ^ (lane >> 3))] = rows[2 * qd + i];
-        wave_lds_sync();
-#pragma unroll
-        for (int i = 0; i < 2; ++i) st[2 * qd + i] = sc[8 * l16 + ((2 * lg + i) ^ (l16 & 7))];
-        wave_lds_sync();
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0);   // the batch's first copies and its terms have landed
-    __syncthreads();
-    if (nch == 1) {
-      // a lone chunk (short prompts): only its tiles that hold tokens
-      chunk_by_tiles(len, [&](auto NBC) __attribute__((always_inline)) { chunk(0, 0, 0, NBC); });
-      break;
-    }
-    const int nb = min(kDirectTerms, nch - b0);
-    for (int i = 0; i < nb; ++i) {
-      const int P = i & 1;
-      if (i + 1 < nb) copy(b0 + i + 1, P ^ 1);   // that buffer is free
-      chunk(b0 + i, i, P, std::integral_constant<int, 4>{});
-      pl = P;
+  if (nch == 1) {
+    // a lone chunk (short prompts): only its tiles that hold tokens
+    chunk_by_tiles(len, [&](auto NBC) __attribute__((always_inline)) { chunk(0, 0, NBC); });
+  } else {
+    for (int j = 0; j < nch; ++j) {
+      pl = j & 1;
+      if (j + 1 < nch) copy(j + 1, pl ^ 1);   // that buffer is free
+      chunk(j, pl, std::integral_constant<int, 4>{});
       // the copies have landed (only the chunk's four output stores are
       // younger) and this chunk's operands are dead, in every wave
-      if (b0 + i + 1 < nch) split_barrier<4>(false);
+      if (j + 1 < nch) split_barrier<4>(false);
     }
   }
   {
@@ -2202,8 +2195,7 @@ __global__ __launch_bounds__(kConsumerThreads) void direct_kernel(
     const float* __restrict__ dt_bias, const uint16_t* __restrict__ b, const void* __restrict__ cu, int is64,
     long long T, float scale, uint16_t* __restrict__ out, float* __restrict__ new_state) {
   __shared__ DirectSmem sm;
-  direct_group(sm, static_cast<int>(blockIdx.x) / kVHeads, static_cast<int>(blockIdx.x) % kVHeads, 1 << 30, q, k, v,
-               state, A_log, a, dt_bias, b, cu, is64, T, scale, out, new_state);
+  direct_group(sm, static_cast<int>(blockIdx.x) / kVHeads, static_cast<int>(blockIdx.x) % kVHeads, q, k, v, state, A_log, a, dt_bias, b, cu, is64, T, scale, out, new_state);
 }
 
 // Work-group 0 plans the longer sequences, the next 8 num_seqs run the shorter
@@ -2228,15 +2220,15 @@ __global__ __launch_bounds__(kConsumerThreads) void mixed_kernel(
   if (bid == 0) {
     int total_recs;
     plan_batch<kConsumerThreads>(cu, is64, num_seqs, T, R, gcap, A_log, dt_bias, rec_start, lists, sm.plan, total_recs,
-                                 false, kMixedChunks);
+                                 false, kDirectChunks);
   } else if (bid <= num_seqs * kVHeads) {
-    direct_group(sm.direct, (bid - 1) / kVHeads, (bid - 1) % kVHeads, kMixedChunks, q, k, v, state, A_log, a, dt_bias,
-                 b, cu, is64, T, scale, out, new_state);
+    direct_group(sm.direct, (bid - 1) / kVHeads, (bid - 1) % kVHeads, q, k, v, state, A_log, a, dt_bias, b, cu, is64, T,
+                 scale, out, new_state);
   } else {
     const int first = 1 + num_seqs * kVHeads;
     prepass_items<false, kMixedWaves>(sm.pre, bid - first,
                                       static_cast<int>(gridDim.x) - first, k, A_log, a, dt_bias, b, nullptr, cu, is64,
-                                      num_seqs, T, R, 1, kMixedChunks, rec_start, ws_frag, ws_gam);
+                                      num_seqs, T, R, 1, kDirectChunks, rec_start, ws_frag, ws_gam);
   }
 }
 
@@ -4225,7 +4217,7 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
   const long long items_v = R * kVHeads;
   const bool mixed = mixed_batch(num_seqs, total_tokens);
   if (mixed) {
-    // records of the longer sequences only: more than kMixedChunks chunks each
+    // records of the longer sequences only: more than kDirectChunks chunks each
     const long long g_mixed = 1 + static_cast<long long>(num_seqs) * kVHeads + total_tokens / kChunk + num_seqs;
     mixed_kernel<<<dim3(static_cast<unsigned>(g_mixed)), dim3(kConsumerThreads), 0, st>>>(
         qb, kb, vb, state, A_log, ab, dt_bias, bb, cu_seqlens, cu_seqlens_is_int64, num_seqs, total_tokens, Ri, gc,
