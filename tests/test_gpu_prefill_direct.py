@@ -1,9 +1,12 @@
-"""GPU parity of the direct path (small calls in one launch) at the edges of its
-rule and of its chunk batches: calls of 256 and 257 tokens, up to 512 tokens
-while they average at most 64 per sequence (one long sequence among tiny ones
-included: eight chunks, one more than a batch of terms), empty sequences, no
-state, int64 cu_seqlens, near-1 decay, and outputs and states that are views
-into larger buffers.  Bar: the oracle tolerances of gpu_util."""
+"""GPU parity of the direct path and of the mixed launch at the edges of their
+rules.  Direct: calls of at most 256 tokens and 64 sequences.  Mixed: longer
+calls of at most 32 sequences and 64 tokens per sequence on average, whose
+sequences of at most four chunks (256 tokens) run directly while the planner and
+the prepass take the longer ones: three- and four-chunk sequences beside five-
+and eight-chunk ones, together and among short ones.  Beside them calls just past
+either rule, which go through the planner.  Empty sequences, no state, int64
+cu_seqlens, near-1 decay, and outputs and states that are views into larger
+buffers.  Bar: the oracle tolerances of gpu_util."""
 
 import pytest
 import torch
@@ -21,15 +24,22 @@ CASES = {
     "255 and 1": ([255, 1], {"weak": True}),
     "three chunks, partial last": ([129], {"state_none": True}),
     "192, 0, 64": ([192, 0, 64], {"cu64": True}),
-    "500 among twelve": ([1] * 6 + [500] + [1] * 6, {}),
-    "500 among twelve, near-1": ([1] * 6 + [500] + [1] * 6, {"weak": True}),
-    "505 among seven ones": ([505] + [1] * 7, {"state_none": True, "cu64": True}),
-    "448 and 449 (batch edge)": ([448] + [0] * 6 + [1], {}),
-    "449 tokens, seven empty": ([449] + [0] * 7, {"weak": True}),
-    "8 x 64": ([64] * 8, {}),
+    "500 among twelve (mixed: planned beside short ones)": ([1] * 6 + [500] + [1] * 6, {}),
+    "500 among twelve, near-1 (mixed)": ([1] * 6 + [500] + [1] * 6, {"weak": True}),
+    "505 among seven ones (mixed)": ([505] + [1] * 7, {"state_none": True, "cu64": True}),
+    "448, one and six empty (mixed)": ([448] + [0] * 6 + [1], {}),
+    "449 tokens, seven empty (mixed)": ([449] + [0] * 7, {"weak": True}),
+    "8 x 64 (mixed, all direct)": ([64] * 8, {}),
     "513 over eight (planned)": ([64] * 7 + [65], {}),
-    "64 sequences of 8": ([8] * 64, {}),
+    "64 sequences of 8 (planned)": ([8] * 64, {}),
     "16-token tiles": ([15, 16, 17, 31, 33, 47, 49, 63, 65, 80], {}),
+    "64 sequences of 4": ([4] * 64, {}),
+    "192 to 320 (mixed, two planned)": ([192, 193, 256, 257, 320] + [3] * 20, {}),
+    "192 to 320, near-1, no state": ([320, 257, 256, 193, 192] + [2] * 20, {"weak": True, "state_none": True}),
+    "256 among short ones, near-1": ([60] * 4 + [256] + [50, 0, 70, 1] * 3, {"weak": True}),
+    "257 among short ones": ([60] * 4 + [257] + [50, 0, 70, 1] * 3, {"cu64": True}),
+    "193 alone among empty ones (mixed)": ([0, 0, 193, 0, 0, 128], {"state_none": True}),
+    "32 sequences, one of 256": ([9] * 16 + [256] + [64] * 15, {}),
 }
 
 
