@@ -2335,15 +2335,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, uin
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
 }
 
-// 16 bytes per lane through a buffer resource straight into LDS (lane i of the
-// wave writes bytes [16 i, 16 i + 16) after the wave-uniform LDS address).
-// AUX is the cache policy of the load: 2 (nt) streams data read exactly once.
-template <int AUX = 0>
-__device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t rs, uint32_t voff, void* lds_wave_base) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)lds_wave_base, 16,
-                                           voff, 0, 0, AUX);
-}
-
 // Per-lane byte offsets of the side-wave copies (chunk-invariant) and the
 // resources they go through.  Resources are formed once per kSplitRebase chunks
 // of an item, so that a chunk's copies differ only in a 32-bit offset: forming
