@@ -388,21 +388,8 @@ __device__ __forceinline__ float fp16_range_scale(float mx) {
   return __int_as_float((137 - e) << 23);           // 2^(10 - e)
 }
 
-// Inclusive prefix sum over the NT threads of the work-group (wave_tot: NT / 64 ints).
-template <int NT>
-__device__ __forceinline__ int block_scan(int x, int* wave_tot) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  x = wave_incl_sum(x);
-  if (lane == 63) wave_tot[wv] = x;
-  __syncthreads();
-  int add = 0;
-  for (int j = 0; j < wv; ++j) add += wave_tot[j];
-  __syncthreads();
-  return x + add;
-}
-
-// K prefix sums at once: x becomes the inclusive scan, total the block sums
-// (wave_tot: NT / 64 * K ints).
+// K prefix sums over the NT threads of the work-group at once: x becomes the
+// inclusive scan, total the block sums (wave_tot: NT / 64 * K ints).
 template <int NT, int K>
 __device__ __forceinline__ void block_scan_v(int (&x)[K], int* wave_tot, int (&total)[K]) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -798,10 +785,6 @@ __device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const 
 
 __device__ __forceinline__ f32x4 mfma16h(const f16x8& a, const f16x8& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ f32x4 mfma_f32(float a, float b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
 // K / Q rows in LDS keep natural column order; the 16-byte chunk j of row t is
