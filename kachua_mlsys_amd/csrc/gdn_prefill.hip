@@ -3768,11 +3768,14 @@ constexpr int kFinRows = 32;                      // value rows of a scan item
 constexpr int kFinParts = kDim / kFinRows;        // scan items per (sequence, v-head)
 constexpr int kFinReady = kFinParts * (kFinThreads / 64);   // waves that publish a segment's state
 constexpr int kScanAhead = 3;                     // steps between a step's loads and their use
-// Polls of a block's wait, at least 512 cycles each: about a second.  A block
-// waits for one scan at most, and the longest scan (kMaxSlots steps) takes 14
-// ms, so the bound is met only where another call on the same workspace has
-// overwritten the counts: its results are then undefined, but it ends.
-constexpr int kFinSpins = 1 << 22;
+// Polls of a group's waits.  A poll sleeps 512 cycles and loads past the L2, so
+// this many take more than 0.2 s.  The scan that a block needs may itself be queued
+// behind others; all scans together are at most kMaxSlots steps per (v-head,
+// part), in order on 256 groups: 30 ms for the longest (3.6 us a step) and 4 ms
+// for the others before it.  The bound is therefore met only where another call
+// on the same workspace has overwritten the counts.  The group then waits for no
+// later block either, so such a call ends about as soon, with undefined results.
+constexpr int kFinSpins = 1 << 20;
 constexpr int kSc01 = 1 | 16;                     // cache policy bits sc0 and sc1
 
 union FinishLds {
@@ -3976,6 +3979,7 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
   const int base = waits ? 0 : static_cast<int>(gridDim.x);
   int zero_v;   // as in split_items: a plain single-lane atomic, waited for at its use
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero_v));
+  bool gave_up = false;   // thread 0: kFinSpins polls were not enough
   int next = static_cast<int>(blockIdx.x);
   if (waits && tid == 0) next = atomicAdd(lv.hdr + 10 + zero_v, 1);
   for (;;) {
@@ -4048,8 +4052,9 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
     } else {
       if (tid == 0) {
         int* rd = seg_ready(slotm, g0, j, h);
-        for (int i = 0; i < kFinSpins; ++i) {
+        for (int i = 0; !gave_up; ++i) {
           if (__hip_atomic_load(rd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= kFinReady) break;
+          gave_up = i >= kFinSpins;
           __builtin_amdgcn_s_sleep(8);
         }
       }
