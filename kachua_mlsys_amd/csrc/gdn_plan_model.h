@@ -104,10 +104,11 @@ GDN_HD float plan_split_warm_us(const PlanStats& b) {
 // run's end) and kStep of a CU's time when both are busy, so the longest run and
 // the balanced load have steps of their own.
 //
-// Fitted together with the split consumer's estimate to 778 batches of 33 to 300
-// sequences timed on both consumers at every segment length (one to 16 sequences
-// of 150 to 16,000 tokens among short ones; uniform; log-uniform over a factor of
-// 4 to 36): consumer and length chosen are 0.7% slower than the best on average,
+// Fitted together with the split consumer's estimate to 1,355 batches of 33 to
+// 700 sequences timed on both consumers at every segment length (one to 16
+// sequences of 150 to 16,000 tokens among short ones; uniform; log-uniform over
+// a factor of 4 to 36): consumer and length chosen are 0.6% slower than the best
+// on average under mixed and near-1 gates, 1.0% under fast ones,
 // 19% at worst.  The rule before, by number of sequences and mean length, took
 // the wide consumer for skewed batches under mixed and slow gates: one of 256
 // tokens among 33 45.9 us (split 30.9), one of 4,000 among 64 92.4 (66.5), 66

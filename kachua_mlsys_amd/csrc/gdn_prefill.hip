@@ -4128,8 +4128,9 @@ int prefill_launch(const void* q, const void* k, const void* v, const float* sta
   if (!cu_seqlens || !new_state || !workspace || !A_log || !dt_bias)
     return GDN_ERR_INVALID_ARGUMENT;
   if (total_tokens > 0 && (!q || !k || !v || !a || !b || !output)) return GDN_ERR_INVALID_ARGUMENT;
-  // q, k, v: 16-byte copies straight into LDS; output: 8-byte stores; states:
-  // 16-byte accesses; a, b: 2-byte loads; cu_seqlens: 4- or 8-byte loads
+  // q, k, v: 16-byte copies straight into LDS; output: 8-byte stores, and 16-byte
+  // buffer accesses, which take any multiple of 4 bytes; states: 16-byte accesses;
+  // a, b: 2-byte loads; cu_seqlens: 4- or 8-byte loads
   if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15u)
     return GDN_ERR_UNALIGNED;
   if (reinterpret_cast<uintptr_t>(output) & 7u) return GDN_ERR_UNALIGNED;
