@@ -187,12 +187,14 @@ extern "C" int gdn_decode_fwd(const void* q, const void* k, const void* v, const
   if ((reinterpret_cast<uintptr_t>(A_log) | reinterpret_cast<uintptr_t>(dt_bias)) & 3u) return GDN_ERR_UNALIGNED;
   if (state == new_state) return GDN_ERR_ALIASING;
   if (!(scale > 0.0f) && !(scale < 0.0f)) scale = 0.08838834764831845f;  // 0 / NaN -> 1/sqrt(128)
-  // Rows per wave, us per step in captured steps over rotated buffers (16 rows
-  // early / 32 early / 32 late): batch 8: 3.57 / 4.29 / 4.11, 32: 6.40 / 7.49 /
-  // 7.02, 48: 10.59 / 8.79 / 8.95, 64: 13.58 / 11.12 / 11.34, 96: 19.05 / 19.52 /
-  // 17.79, 128: 24.60 / 24.79 / 24.46, 192: 35.14 / 36.18 / 35.62, 256: 45.52 /
-  // 46.94 / 46.65.
-  if (rows_per_wave == 0) rows_per_wave = (batch <= 32 || batch >= 160) ? 16 : 32;
+  // Rows per wave and load order, us per step in captured steps over rotated
+  // buffers (16 rows early / 32 early / 32 late): batch 8: 3.65 / 4.41 / 4.11, 32: 6.49 / 7.75 / 7.35, 33: 7.64 /
+  // 7.83 / 7.50, 40: 8.94 / 8.49 / 8.24, 44: 9.78 / 8.79 / 8.70, 48: 10.51 / 9.05 /
+  // 9.09, 56: 11.97 / 9.76 / 10.31, 64: 13.44 / 11.27 / 11.31, 65: 13.74 / 13.28 /
+  // 11.84, 96: 18.81 / 19.43 / 17.38, 120: 22.92 / 23.29 / 22.64, 128: 24.22 /
+  // 24.49 / 24.17, 136: 25.81 / 27.33 / 26.42, 159: 29.48 / 30.67 / 29.74, 192:
+  // 34.80 / 35.88 / 35.32, 256: 45.70 / 47.02 / 46.78.
+  if (rows_per_wave == 0) rows_per_wave = (batch <= 32 || batch >= 132) ? 16 : 32;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const auto* qb = static_cast<const uint16_t*>(q);
   const auto* kb = static_cast<const uint16_t*>(k);
@@ -205,7 +207,7 @@ extern "C" int gdn_decode_fwd(const void* q, const void* k, const void* v, const
     const long grid = heads * (kDim / 32);
     if (grid > 0x7fffffffL) return GDN_ERR_INVALID_ARGUMENT;
     const dim3 gr(static_cast<unsigned>(grid));
-    if (batch <= 64)
+    if (batch >= 46 && batch <= 64)
       decode_kernel<32, true><<<gr, dim3(64), 0, st>>>(qb, kb, vb, state, A_log, ab, dt_bias, bb, scale, ob, new_state);
     else
       decode_kernel<32, false><<<gr, dim3(64), 0, st>>>(qb, kb, vb, state, A_log, ab, dt_bias, bb, scale, ob, new_state);

@@ -170,8 +170,8 @@ def test_decode_random_steps(gpu, seed):
 
 
 # The automatic choice of rows per wave and of the load order changes at batches
-# of 33, 65 and 160: both sides of each edge, checked against the oracle.
-@pytest.mark.parametrize("batch", [32, 33, 64, 65, 159, 160])
+# of 33, 46, 65 and 132: both sides of each edge, checked against the oracle.
+@pytest.mark.parametrize("batch", [32, 33, 45, 46, 64, 65, 131, 132, 159, 160])
 def test_decode_dispatch_edges(gpu, batch):
     d = decode_inputs(batch, seed=300 + batch)
     o_ref, s_ref = decode_ref(*d.args())
