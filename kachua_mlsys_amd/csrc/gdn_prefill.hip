@@ -140,8 +140,10 @@ __host__ __device__ inline long long max_segments(long long tokens) {
 //   hdr[0] runs, [1] short sequences, [2] segment length L (chunks),
 //   [3] multi-segment sequences (none when the batch uses warm-up segments),
 //   [8] split-consumer work queue (items claimed past each group's first),
-//   [9] correction blocks appended by the consumer's M-runs, [10] finish queue,
-//   [11] most segments of any sequence, [12] the wide consumer runs the call
+//   [9] correction blocks of second segments (from the list's front), appended by
+//   the consumer's M-runs, [10] finish queue,
+//   [11] most segments of any sequence, [12] the wide consumer runs the call,
+//   [13] correction blocks of segments after a sequence's second (from the back)
 //   multi[e]   = (seq, first slot, segments, 0)
 //   runs[2i]   = (seq, flags | tokens of the run's last chunk << 8 | segment
 //                 j << 16, final-state slot or -1 for new_state, first record)
@@ -172,14 +174,25 @@ constexpr int kSlotNone = -2;
 
 // Finish work: a correction block is a few chunks of one (segment, v-head);
 // four waves of a finish group correct a chunk (16 tokens each), so a group
-// takes two at a time.  An M-run of n chunks reserves fin_blocks(n) blocks when
-// it starts: pairs of chunks in shorter segments (more groups at work), four
-// chunks in longer ones (the state's fragments are fetched once per block),
-// and spreads the chunks it formed over them at its end.
+// takes two at a time.  An M-run of n chunks spreads the chunks that it formed
+// over at most fin_blocks(n) blocks of two chunks or more: pairs of chunks in
+// shorter segments (more groups at work), four chunks in longer ones (the state's
+// fragments are fetched once per block).
 __host__ __device__ constexpr int fin_blocks(int n) { return n <= 14 ? (n + 1) / 2 : (n + 3) / 4; }
 __host__ __device__ constexpr int fin_block_chunks(int n, int formed) {
   const int nb = fin_blocks(n), even = nb > 0 ? (formed + nb - 1) / nb : 0;
   return even > 2 ? even : 2;
+}
+// Blocks of first later segments, which wait for nothing, fill the list from its
+// front, the others from its back, and the finish takes them in that order (in
+// the order of their M-runs' ends, short last segments' blocks came first and
+// groups waited in them: 13 sequences of 260 to 4,160 tokens 91 us, now 89).
+// Header word of the count, and place of block i.
+__host__ __device__ constexpr int fix_count(int j) { return j == 1 ? 9 : 13; }
+__host__ __device__ constexpr int fix_at(int j, int i, int cap) { return j == 1 ? i : cap - 1 - i; }
+__host__ __device__ constexpr int fin_count(int n, int formed) {
+  const int c = fin_block_chunks(n, formed);
+  return (formed + c - 1) / c;
 }
 // The count of waves that have published the state before segment j: in the
 // first slot's M area, which no M-run writes (segment 0 has none).  The
@@ -676,7 +689,7 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     }
     if (lane == 0) {
       lv.hdr[8] = 0;   // work queue
-      lv.hdr[9] = 0;   // correction blocks
+      lv.hdr[9] = lv.hdr[13] = 0;   // correction blocks
       lv.hdr[10] = 0;  // finish queue
       lv.hdr[11] = choice[2];
       lv.hdr[12] = take_wide ? 1 : 0;
@@ -2854,15 +2867,14 @@ __device__ __forceinline__ void split_items(
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
   // Correction blocks of the segment: chunks [0, formed) get O0 + OI S_j^T in
-  // the finish.  Each M-run (once per v-head) reserves its blocks (fin_blocks)
-  // during its first chunk (the atomic returns before that chunk's closing
-  // barrier, with the next chunk's copies), and fills them at its end; blocks
-  // past `formed` are left empty.  The finish then takes a block with a single
-  // descriptor load: (first token of the segment lo, hi, its tokens | j << 17
+  // the finish.  Each M-run appends its blocks (once per v-head) when it ends, and
+  // so knows how many it needs.  (Reserved during its first chunk, as many as the
+  // whole segment could need, most blocks of heads that forget soon were empty,
+  // each a claim for the finish: 8 x 2446 tokens, mixed gates, 102 us, now 91; 6 x
+  // 4000 114 -> 108; 1 x 32768 186 -> 180.)  The finish then takes a block with a
+  // single descriptor load: (first token of the segment lo, hi, its tokens | j << 17
   // (L <= 1024 chunks: at most 65536 tokens), slot of segment j - 1) and
   // (v-head, first chunk, end chunk, 0).
-  int fix_pos = 0;
-
   // An M-run stops once the bound of its map falls below kNegligibleLog2: its
   // outputs of later chunks are negligible (the correction skips them) and so
   // is its final state.  Every wave accumulates the same bounds in the same
@@ -2880,7 +2892,6 @@ __device__ __forceinline__ void split_items(
       copy(0, B0{});
     }
     split_barrier<0>(chain);   // the first chunk's copies and every S fragment in place
-    if (mrun && hv == 0 && tid == kFixLane) fix_pos = atomicAdd(lv.hdr + 9 + zero_v, fin_blocks(n));
     for (int i = 0; i < n; i += 2) {
       {
         if (i + 1 >= n) claim();
@@ -2938,12 +2949,14 @@ __device__ __forceinline__ void split_items(
     *seg_ready(slotm, slot - jseg, jseg, h) = 0;
   }
   if (mrun && hv == 0 && tid == kFixLane && n > 0) {
-    const int fix_max = fin_blocks(n);
+    const int fix_max = fin_count(n, formed);
+    const int fix_pos = atomicAdd(lv.hdr + fix_count(jseg) + zero_v, fix_max);
     const int4 seg = make_int4(rb.x, rb.y, ((nrun - 1) * kChunk + last_tok) | (jseg << 17), slot - 1);
     const int bsz = fin_block_chunks(n, formed);
     for (int b = 0; b < fix_max && fix_pos + b < fix_cap; ++b) {
-      fix[2 * (fix_pos + b)] = seg;
-      fix[2 * (fix_pos + b) + 1] = make_int4(h, b * bsz, min((b + 1) * bsz, formed), 0);
+      const int at = fix_at(jseg, fix_pos + b, fix_cap);
+      fix[2 * at] = seg;
+      fix[2 * at + 1] = make_int4(h, b * bsz, min((b + 1) * bsz, formed), 0);
     }
   }
 
@@ -3559,14 +3572,11 @@ __device__ __forceinline__ void wide_items(
           for (int rr = 0; rr < 4; ++rr)
             st[e][kt][rr] = mrun && kappa(kt, rr) == vrow0 + wide_row(e, l16) ? 1.0f : 0.0f;
     }
-    const int fix_max = fin_blocks(n);
-    int fix_pos = 0;
     float lbound = 0.0f;
     int formed = n;
     int pl = 0;   // K buffer of the last chunk run
     if (n > 0) {
       bar.template wait<0>();
-      if (mrun && tid == 64) fix_pos = atomicAdd(lv.hdr + 9 + zero_v, fix_max);
       for (int i = 0;; ++i) {
         const int P = i & 1;
         const bool more = i + 1 < n;
@@ -3605,13 +3615,16 @@ __device__ __forceinline__ void wide_items(
       mval[static_cast<size_t>(slot) * kVHeads + h] = formed | (formed < n ? kMNegligible : 0);
       *seg_ready(slotm, slot - jseg, jseg, h) = 0;
     }
-    if (mrun && tid == 64 && fix_max > 0) {
+    if (mrun && tid == 64 && n > 0) {
+      const int fix_max = fin_count(n, formed);
+      const int fix_pos = atomicAdd(lv.hdr + fix_count(jseg) + zero_v, fix_max);
       const int4 seg = make_int4(static_cast<int>(c0r & 0xffffffffLL), static_cast<int>(c0r >> 32),
                                  ((nrun - 1) * kChunk + last_tok) | (jseg << 17), slot - 1);
       const int bsz = fin_block_chunks(n, formed);
       for (int b = 0; b < fix_max && fix_pos + b < fix_cap; ++b) {
-        fix[2 * (fix_pos + b)] = seg;
-        fix[2 * (fix_pos + b) + 1] = make_int4(h, b * bsz, min((b + 1) * bsz, formed), 0);
+        const int at = fix_at(jseg, fix_pos + b, fix_cap);
+        fix[2 * at] = seg;
+        fix[2 * at + 1] = make_int4(h, b * bsz, min((b + 1) * bsz, formed), 0);
       }
     }
     if (slot != kSlotNone && !(mrun && formed < n)) {
@@ -3957,7 +3970,7 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
   __shared__ int claimed;
   const ListView lv = list_view(lists, num_seqs, gcap);
   const int nmulti = lv.hdr[3];
-  const int ncorr = min(lv.hdr[9], fix_cap);   // correction blocks
+  const int nfront = min(lv.hdr[9], fix_cap), ncorr = min(nfront + lv.hdr[13], fix_cap);   // correction blocks
   // the blocks were written by the consumer launch: constant here (scalar loads)
   const auto* fix_c = (const __attribute__((address_space(4))) u32x4*)fix;
   const int tid = threadIdx.x;
@@ -3968,12 +3981,14 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
   // The next claim is requested while an item is worked on.  A group that waits
   // in a block holds at most another block: claims only grow.  Where no sequence
   // has a third segment nothing waits, and every group starts with its own item
-  // (256 first claims cost about 1.5 us).  It scans two parts at a time if the
-  // items would not be one round otherwise (the second part's loads follow the
-  // first part's stores: 1 x 1000 tokens in two segments 12.5 us, one part each
-  // 8.4).
+  // (256 first claims cost about 1.5 us).  It scans two parts at a time where
+  // everything fits into one round so and not with one part each (the second
+  // part's loads follow the first part's stores: 1 x 1000 tokens in two segments
+  // 12.5 us, one part each 8.4; but 8 x 2446, mixed gates, 91 us per call against
+  // 95 with one part each, and 5 x 1826, where neither fits, 80 against 77.5).
   const bool waits = lv.hdr[11] > 2;
-  const int parts = waits || nmulti * kVHeads * kFinParts + ncorr <= static_cast<int>(gridDim.x) ? 1 : 2;
+  const int scans = nmulti * kVHeads * kFinParts, grid = static_cast<int>(gridDim.x);
+  const int parts = !waits && scans + ncorr > grid && scans / 2 + ncorr <= grid ? 2 : 1;
   const int nscan = nmulti * kVHeads * (kFinParts / parts);
   const int nitem = ncorr + nscan;
   const int base = waits ? 0 : static_cast<int>(gridDim.x);
@@ -4000,7 +4015,8 @@ __global__ __launch_bounds__(kFinThreads) void finish_kernel(int* __restrict__ l
     }
     // block: (first token lo, hi, tokens | j << 17, slot of segment j - 1) and
     // (v-head, first chunk, end chunk): chunks [first, last) need OI S_j^T
-    const int item = it - nscan;
+    const int block = it - nscan;
+    const int item = block < nfront ? block : fix_cap - 1 - (block - nfront);
     const u32x4 fa = fix_c[2 * item], fb = fix_c[2 * item + 1];
     const int4 sg = make_int4(static_cast<int>(fa.x), static_cast<int>(fa.y), static_cast<int>(fa.z),
                               static_cast<int>(fa.w));
