@@ -22,6 +22,7 @@ struct PlanStats {
   float mfrac;       // share of a segment an M-run forms before its map is negligible (mean over the v-heads)
   int longest;       // chunks of the longest sequence
   int L;             // segment length in chunks
+  int nseg;          // segments of the longest sequence
   float warmup;      // warm-up chunks of a later segment's run (warm-up scheme)
   bool many;         // more than 32 sequences: the wide consumer is weighed too
 };
@@ -41,6 +42,10 @@ GDN_HD float plan_shorts_wide_us(float n) { return n <= 64.0f ? 9.8f + 0.137f * 
 // Single-chunk sequences beside runs on the split consumer, in batches of more
 // than 32 sequences: their groups start where a CU is free, so with few runs
 // (fewer than the 16 machines) the groups that found none start a round later.
+// Runs of two chunks or more take at least ceil(runs / 16) rounds of two: 16 runs
+// of two and three chunks among 32 to 47 sequences 37 to 40 us per call, 17 to 30
+// of them 44 to 45, which the balanced load alone puts at 39 (wide consumer 39).
+GDN_HD float plan_rounds(float runs) { return static_cast<float>((static_cast<int>(runs) + 15) / 16); }
 GDN_HD float plan_beside_runs_us(float shorts_us, float runs, float run_us, float balanced_us, float late) {
   const float again = plan_min(late * shorts_us, run_us);
   return shorts_us + (runs >= 16.0f ? balanced_us : plan_max(balanced_us, again));
@@ -70,15 +75,16 @@ GDN_HD float plan_split_mrun_us(const PlanStats& b) {
   const float mwork = (b.chunks - b.first) * b.mfrac;
   const float work = b.chunks + mwork;
   const float longest = static_cast<float>(b.L < b.longest ? b.L : b.longest);
-  const int nseg = b.longest > 0 ? (b.longest - 1) / b.L + 1 : 0;
-  const float tail = runs > kMachines ? kTail * (work / runs + kItem) : 0.0f;
+  const float run = work / runs + kItem;   // an average run
+  const float tail = runs > kMachines ? kTail * run : 0.0f;
   float balanced = ((work + kItem * runs) / kMachines + tail) * kStep;
+  if (b.many && runs > 16.0f) balanced = plan_max(balanced, plan_rounds(runs) * (2.0f + kItem) * kStep);
   if (!b.many)
     balanced += b.shorts * (kShort / 32.0f);
   else if (b.shorts > 0.0f)
-    balanced = 3.3f + plan_beside_runs_us(b.shorts * (7.7f / 32.0f), runs, (work / runs + kItem) * kStep, balanced, 0.6f);
+    balanced = 3.3f + plan_beside_runs_us(b.shorts * (7.7f / 32.0f), runs, run * kStep, balanced, 0.6f);
   const float body = plan_max(b.longs > 0.0f ? (longest + kItem) * kStep : 0.0f, balanced);
-  return body + (nseg > 1 ? kFinish + kScanStep * static_cast<float>(nseg - 2) + kCorr * mwork : 0.0f);
+  return body + (b.nseg > 1 ? kFinish + kScanStep * static_cast<float>(b.nseg - 2) + kCorr * mwork : 0.0f);
 }
 
 // Split consumer, warm-up scheme: one run per segment, each later segment's
@@ -91,11 +97,14 @@ GDN_HD float plan_split_warm_us(const PlanStats& b) {
   if (b.longs == 0.0f) return plan_shorts_split_us(b.shorts);
   const float work = b.chunks + b.warmup * (b.segments - b.longs);
   const float longest = static_cast<float>(b.longest > b.L ? b.L + b.warmup : b.longest);
-  const float tail = b.segments > kMachines ? kTail * (work / b.segments + kItem) : 0.0f;
+  const float run = work / b.segments + kItem;   // an average run
+  const float tail = b.segments > kMachines ? kTail * run : 0.0f;
   float balanced = ((work + kItem * b.segments) / kMachines + tail) * kStep;
+  if (b.many && b.segments > 16.0f) balanced = plan_max(balanced, plan_rounds(b.segments) * (2.0f + kItem) * kStep);
   if (b.many && b.shorts > 0.0f)
-    balanced = 8.2f + plan_beside_runs_us(b.shorts * (6.9f / 32.0f), b.segments, (work / b.segments + kItem) * kStep,
-                                          balanced, 0.48f);
+    balanced = 8.2f + plan_beside_runs_us(b.shorts * (6.9f / 32.0f), b.segments, run * kStep, balanced, 0.48f);
+  else if (b.many)
+    balanced += 4.0f;
   return plan_max((longest + kItem) * kStep, balanced) + (b.longest > b.L ? kSegmented * kStep : 0.0f);
 }
 
@@ -121,12 +130,11 @@ GDN_HD float plan_wide_mrun_us(const PlanStats& b) {
   const float mwork = (b.chunks - b.first) * b.mfrac;
   const float work = b.chunks + mwork;
   const float longest = static_cast<float>(b.L < b.longest ? b.L : b.longest);
-  const int nseg = (b.longest - 1) / b.L + 1;
   const float tail = runs > kMachines ? kTail * work / runs : 0.0f;
   const float balanced = ((work + kItem * runs) / kMachines + tail) * kStep + b.shorts * (kShort / 32.0f);
   const float lone = (longest + kItem) * kLone;
   return plan_max(lone, balanced) + kMix * plan_min(lone, balanced) +
-         (nseg > 1 ? kFinish + kScanStep * static_cast<float>(nseg - 2) + kCorr * mwork : 0.0f);
+         (b.nseg > 1 ? kFinish + kScanStep * static_cast<float>(b.nseg - 2) + kCorr * mwork : 0.0f);
 }
 
 GDN_HD float plan_wide_warm_us(const PlanStats& b) {

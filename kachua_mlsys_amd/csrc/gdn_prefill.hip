@@ -618,10 +618,10 @@ __device__ int plan_batch(const void* __restrict__ cu, int is64, int num_seqs, l
     float mfrac = 0.f;
     if (!warm) {
 #pragma unroll
-      for (int hh = 0; hh < kVHeads; ++hh)
-        mfrac += static_cast<float>(min(__builtin_amdgcn_readlane(wh, hh), Lc)) / (kVHeads * static_cast<float>(Lc));
+      for (int hh = 0; hh < kVHeads; ++hh) mfrac += static_cast<float>(min(__builtin_amdgcn_readlane(wh, hh), Lc));
+      mfrac /= kVHeads * static_cast<float>(Lc);   // one division: the plan may be what the launch waits for
     }
-    const PlanStats ps_c = {sl, a, 0.5f * (runs + nl), nl, ns, mfrac, ml, Lc, static_cast<float>(w_est), may_wide};
+    const PlanStats ps_c = {sl, a, 0.5f * (runs + nl), nl, ns, mfrac, ml, Lc, nseg_max, static_cast<float>(w_est), may_wide};
     float est;
     if (wv == 0)   // uniform
       est = warm ? plan_split_warm_us(ps_c) : plan_split_mrun_us(ps_c);

@@ -18,12 +18,13 @@ SHIM = """
 #include "gdn_plan_model.h"
 extern "C" float split_mrun_us(float chunks, float first, float segments, float longs, float shorts, float mfrac,
                                int longest, int L) {
-  return gdn::plan_split_mrun_us(gdn::PlanStats{chunks, first, segments, longs, shorts, mfrac, longest, L, 0.0f, false});
+  return gdn::plan_split_mrun_us(gdn::PlanStats{chunks, first, segments, longs, shorts, mfrac, longest, L, (longest - 1) / L + 1, 0.0f, false});
 }
 // more than 32 sequences: either consumer, M-runs (warmup < 0) or warm-up runs
 extern "C" float many_us(int wide, float chunks, float first, float segments, float longs, float shorts, int longest,
                          int L, float warmup) {
-  const gdn::PlanStats b = {chunks, first, segments, longs, shorts, 1.0f, longest, L, warmup, true};
+  const int nseg = longest > 0 ? (longest - 1) / L + 1 : 0;
+  const gdn::PlanStats b = {chunks, first, segments, longs, shorts, 1.0f, longest, L, nseg, warmup, true};
   if (wide) return warmup < 0.0f ? gdn::plan_wide_mrun_us(b) : gdn::plan_wide_warm_us(b);
   return warmup < 0.0f ? gdn::plan_split_mrun_us(b) : gdn::plan_split_warm_us(b);
 }
