@@ -108,8 +108,8 @@ GDN_HD float plan_split_warm_us(const PlanStats& b) {
   return plan_max((longest + kItem) * kStep, balanced) + (b.longest > b.L ? kSegmented * kStep : 0.0f);
 }
 
-// Wide consumer.  A run's 8 items take 8 of 256 CUs, two groups to a CU: a chunk
-// step takes kLone while the other group has no work or little (the longest
+// Wide consumer.  A run's 8 items take 8 of 256 CUs, two halves to a CU: a chunk
+// step takes kLone while the other half has no work or little (the longest
 // run's end) and kStep of a CU's time when both are busy, so the longest run and
 // the balanced load have steps of their own.
 //

@@ -20,6 +20,8 @@ SPLIT, WIDE = 0, 1
 CASES = {
     "33 x 70": ([70] * 33, "near-1", WIDE, False),
     "65 single chunks": ([30] * 65, "fast", WIDE, False),
+    "50 tokens over 100": ([1, 0] * 50, "fast", WIDE, False),
+    "one token among 90": ([0] * 40 + [1] + [0] * 49, "near-1", SPLIT, False),
     "90 single chunks": ([30] * 89 + [0], "fast", SPLIT, False),
     "one of 640 among 48": ([20] * 20 + [640] + [20] * 27, "near-1", SPLIT, False),
     "16 of 500 among 34": ([9] * 18 + [500] * 16, "near-1", SPLIT, False),
